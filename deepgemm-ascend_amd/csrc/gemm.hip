@@ -54,7 +54,27 @@ int check_m_indices(const int32_t* idx, int m, int alignment, int num_groups, hi
 // csrc/status.hip: the run table of an m_indices layout (for anchored tiles)
 int m_indices_runs(const int32_t* idx, int m, int alignment, int32_t* runs, const int32_t* blk_end, hipStream_t st);
 
+KernelFn lookup_quad_fp8(int bm, int bn, int epi);
+KernelFn lookup_quad_fp8_mn_a(int bm, int bn, int epi);
+KernelFn lookup_quad_fp8_mn_b(int bm, int bn, int epi);
+KernelFn lookup_quad_fp8_mn_ab(int bm, int bn, int epi);
+KernelFn lookup_quad_bf16(int bm, int bn, int epi);
+KernelFn lookup_quad_bf16_mn_a(int bm, int bn, int epi);
+KernelFn lookup_quad_bf16_mn_b(int bm, int bn, int epi);
+KernelFn lookup_quad_bf16_mn_ab(int bm, int bn, int epi);
+KernelFn lookup_quad_fp8fp4(int bm, int bn, int epi);
+
+KernelFn lookup_quad(int kind, int bm, int bn, int epi, bool a_mn, bool b_mn) {
+    if (kind == kFP8FP4) return a_mn || b_mn ? nullptr : lookup_quad_fp8fp4(bm, bn, epi);
+    if (kind == kFP8FP8) return a_mn ? (b_mn ? lookup_quad_fp8_mn_ab(bm, bn, epi) : lookup_quad_fp8_mn_a(bm, bn, epi))
+                                     : (b_mn ? lookup_quad_fp8_mn_b(bm, bn, epi) : lookup_quad_fp8(bm, bn, epi));
+    if (kind == kBF16) return a_mn ? (b_mn ? lookup_quad_bf16_mn_ab(bm, bn, epi) : lookup_quad_bf16_mn_a(bm, bn, epi))
+                                   : (b_mn ? lookup_quad_bf16_mn_b(bm, bn, epi) : lookup_quad_bf16(bm, bn, epi));
+    return nullptr;
+}
+
 KernelFn lookup_kernel(int kind, int bm, int bn, int epi, bool persistent) {
+    if (quad_tile(kind, bm, bn) && !persistent) return lookup_quad(kind, bm, bn, epi, false, false);
     switch (kind) {
         case kFP8FP8: return lookup_kernel_fp8fp8(bm, bn, epi, persistent);
         case kFP8FP4: return lookup_kernel_fp8fp4(bm, bn, epi, persistent);
@@ -723,6 +743,12 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
         if (a.split_k > 1) return dg_set_error("dg_gemm: workspace smaller than dg_gemm_workspace_size() reports");
         plan = choose(a, cus, false);
     }
+    if (a.d_dtype == DG_DTYPE_FP8_E4M3 && plan.skinny_nw == 0 && quad_tile(a.kind, plan.tile.bm, plan.tile.bn) &&
+        !quad_fp8_output(plan.tile.bn)) {
+        // FP8 output needs whole 32-column groups per wave: the 256-column tile, whose sums are the same
+        for (const TileCfg& t : kTiles)
+            if (t.bm == 256 && t.bn == 256) plan.tile = t;
+    }
     const TileCfg cfg = plan.tile;
     if (cfg.bm == 0) return dg_set_error("dg_gemm: no tile shape fits this problem");
     // (MN-major B also in the skinny kernel's 32-column plans)
@@ -873,23 +899,27 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
     p.split_k = plan.split;
     p.split_stages = plan.split_stages;
     p.num_tiles = (int)tiles;
+    // (K ranges of the four-wave tile kernel are always summed by a second launch)
+    const bool quad = !skinny && quad_tile(a.kind, cfg.bm, cfg.bn) && !persistent;
     if (plan.split > 1) {
         // DG_SPLIT_SPREAD=1 (test knob): the splits of a tile run on different XCDs
         const char* spread = std::getenv("DG_SPLIT_SPREAD");
         p.split_spread = spread != nullptr && spread[0] == '1';
         p.counters = reinterpret_cast<int*>(workspace);
         p.ws = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(workspace) + kCounterBytes);
-        p.split_reduce = plan.split_reduce;
+        p.split_reduce = plan.split_reduce || quad;
+        p.reduce_bm = cfg.bm;
+        p.reduce_bn = cfg.bn;
     }
     KernelFn reduce_fn = nullptr;
     if (p.split_reduce) {
-        reduce_fn = lookup_split_reduce(cfg.bm / 32, cfg.bn / 32, epi_kind);
+        reduce_fn = quad ? lookup_quad_reduce(epi_kind) : lookup_split_reduce(cfg.bm / 32, cfg.bn / 32, epi_kind);
         if (reduce_fn == nullptr) {
             dg_set_error("dg_gemm: no compiled split-K reduction kernel for this plan");
             return DG_ENOKERNEL;
         }
     }
-    int threads = skinny ? plan.skinny_nw * 64 : tile_threads(cfg.bm, cfg.bn);
+    int threads = skinny ? plan.skinny_nw * 64 : tile_threads(a.kind, cfg.bm, cfg.bn, persistent);
     unsigned lds_bytes = 0;
     if (gemv_mr > 0) {
         // workgroups of 8 waves / ks rows of B, dealt over the XCDs in contiguous runs
@@ -964,8 +994,11 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
             if (rc != DG_OK) return rc;
         }
     }
-    if (jit) return jit_run(a, cfg, epi_kind, plan.split, p, launched, st, compile_only);
-    for (int64_t base = 0; base < grid; base += launched) {
+    if (jit) {
+        const int rc = jit_run(a, cfg, epi_kind, plan.split, p, launched, st, compile_only);
+        if (rc != DG_OK || compile_only || reduce_fn == nullptr) return rc;
+    }
+    for (int64_t base = 0; !jit && base < grid; base += launched) {
         p.vbase = (int)base;
         const unsigned n = (unsigned)std::min<int64_t>(launched, grid - base);
         const hipError_t e = launch_module_kernel(reinterpret_cast<const void*>(fn), n, (unsigned)threads, p, st, lds_bytes);
@@ -977,9 +1010,11 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
     }
     if (reduce_fn != nullptr) {
         // second launch: one wave per 32x32 block of the tiles, DG_REDUCE_WAVES (tuning, default 1) per workgroup
+        // (quad plans: a thread per four outputs, four waves per workgroup)
         static const int rw_env = std::getenv("DG_REDUCE_WAVES") ? std::atoi(std::getenv("DG_REDUCE_WAVES")) : 1;
-        const int rw = rw_env == 2 || rw_env == 4 ? rw_env : 1;
-        const int64_t rgrid = ceil_div(tiles * (cfg.bm / 32) * (cfg.bn / 32), rw);
+        const int rw = quad ? 4 : rw_env == 2 || rw_env == 4 ? rw_env : 1;
+        const int64_t rgrid = quad ? ceil_div64(tiles * cfg.bm * cfg.bn, 1024)
+                                   : ceil_div(tiles * (cfg.bm / 32) * (cfg.bn / 32), rw);
         const int64_t rlaunched = cus_capped(cus) ? std::min<int64_t>(rgrid, cus >= 8 ? cus / 8 * 8 : cus) : rgrid;
         p.vgrid = (int)rgrid;
         for (int64_t base = 0; base < rgrid; base += rlaunched) {

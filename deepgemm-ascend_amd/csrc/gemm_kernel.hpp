@@ -74,6 +74,7 @@ struct KParams {
     // CU cap (set_num_sms) the plan's workgroups go out in launches of at most that many, and
     // workgroup b of a launch serves plan workgroup vbase + b.
     int vgrid, vbase;
+    int reduce_bm, reduce_bn;   // quad_reduce_kernel: the tile the partials belong to
 };
 
 // Epilogue variants.
@@ -539,6 +540,202 @@ __device__ __forceinline__ void epilogue_block(const KParams& p, const f32x16& a
     }   // !kFp8
 }
 
+// What a workgroup computes: its tile's place in D, the operands it reads and its share of K.
+struct TileLoc {
+    const uint8_t* a_base;     // first row of the operand (batch and K group applied; the tile's m0 / n0 not)
+    const uint8_t* b_base;     // (group applied)
+    const uint16_t* sfa;
+    const uint16_t* sfb;
+    uint8_t* d_base;
+    int m0, n0, batch, group;
+    int valid_end;             // rows >= valid_end are padding (M-grouped) / not written (masked)
+    int tile_end;              // rows >= tile_end belong to another tile (anchored tiles)
+    int k_len;                 // K extent of this tile's contraction
+    int split, tile_id;        // split-K: this workgroup's K range and the tile's index
+    bool anchored;
+};
+
+// The tile of plan workgroup `vb` of a BM x BN launch (NT threads).  False when there is nothing to
+// compute: no such tile, rows past masked_m, or a padding-only tile of an M-grouped layout, whose zeros
+// are written here.
+template <int BM, int BN, int NT, int KIND, int CT, int CS, int CM, int CN, int CK, bool AMN, bool BMN>
+__device__ __forceinline__ bool locate_tile(const KParams& p, const int vb, const int known_total, const int tid,
+                                            TileLoc& tl) {
+    constexpr bool kAFp4 = KIND == kFP4FP4;
+    constexpr bool kBFp4 = KIND == kFP8FP4 || KIND == kFP4FP4;
+    constexpr bool kBf16 = KIND == kBF16;
+    const int lane = tid & 63;
+    const int gemm_type = CT >= 0 ? CT : p.gemm_type;
+    const int split_k = CS > 0 ? CS : p.split_k;
+    const int nm = CM > 0 ? ceil_div(CM, BM) : p.num_m_blocks, nn = CN > 0 ? ceil_div(CN, BN) : p.num_n_blocks;
+    int t, split = 0;
+    if (split_k > 1) {
+        // Split-K launch: grid = 8 * ceil(tiles / 8) * split_k, and workgroup b serves tile
+        // (b / 8 / split_k) * 8 + b % 8, split (b / 8) % split_k, so all splits of a tile share
+        // b % 8 -- the XCD (and L2) the dispatcher places them on.
+        const int b = vb, r = b >> 3;
+        t = (r / split_k) * 8 + (b & 7);
+        split = r % split_k;
+        if (p.split_spread) {
+            // (test knob: consecutive workgroups -- different XCDs -- take the splits of a tile)
+            t = b / split_k;
+            split = b % split_k;
+        }
+        if (t >= p.num_tiles) return false;
+    } else if (gemm_type == kKGrouped) {
+        // K-grouped: each group's tiles are spread over the XCDs on their own, so at any time all
+        // XCDs work on one group and its A / B K-slices (Kg x (M + N) bytes) are streamed once,
+        // instead of every XCD pair streaming another group's and the groups together overflowing
+        // the last-level cache.  (groups in order; a group's tiles are consecutive workgroups)
+        const int per_group = nm * nn;
+        const int g = vb / per_group;
+        t = g * per_group + xcd_remap(vb - g * per_group, per_group);
+    } else {
+        t = xcd_remap(vb, p.vgrid);
+    }
+    const int tile_id = t;
+    int batch = 0;
+    if (gemm_type == kBatched || gemm_type == kMasked || gemm_type == kKGrouped) {
+        batch = t / (nm * nn);
+        t -= batch * nm * nn;
+    }
+    const int M = CM > 0 ? CM : p.m, N = CN > 0 ? CN : p.n;
+    int mb = 0, nb = 0, m0, anchor_group = -1, tile_end = M, anchor_valid = M;
+    const bool anchored = (gemm_type == kMGroupedPsum || gemm_type == kMGroupedIdx) && p.anchored && p.num_groups > 0;
+    if (anchored) {
+        const int* runs = gemm_type == kMGroupedIdx ? p.runs : nullptr;
+        // the launch's real tiles spread over the XCDs as xcd_remap spreads a full grid
+        const int total = known_total >= 0 ? known_total
+            : __builtin_amdgcn_readfirstlane(anchored_total(p.layout, p.num_groups, runs, p.alignment, BM, M, nn));
+        if (vb >= total) return false;
+        t = xcd_remap(vb, total);
+        anchored_tile(p.layout, p.num_groups, runs, p.alignment, t, BM, M, nn, anchor_group, m0, nb, tile_end,
+                      anchor_valid);
+        anchor_group = __builtin_amdgcn_readfirstlane(anchor_group);
+        if (anchor_group == -2) return false;   // past the last tile of this launch
+        m0 = __builtin_amdgcn_readfirstlane(m0);
+        nb = __builtin_amdgcn_readfirstlane(nb);
+        tile_end = __builtin_amdgcn_readfirstlane(tile_end);
+        anchor_valid = __builtin_amdgcn_readfirstlane(anchor_valid);
+    } else {
+        if (gemm_type == kMGroupedPsum && p.num_groups > 0)
+            expert_major_tile(p.layout, p.num_groups, p.alignment, t, BM, nm, nn, mb, nb);
+        else
+            swizzle_tile(t, nm, nn, p.group_m, mb, nb);
+        mb = __builtin_amdgcn_readfirstlane(mb);
+        nb = __builtin_amdgcn_readfirstlane(nb);
+        m0 = mb * BM;
+    }
+    const int n0 = nb * BN;
+
+    const uint8_t* a_base = p.a;
+    const uint8_t* b_base = p.b;
+    const uint16_t* sfa = p.sfa;
+    const uint16_t* sfb = p.sfb;
+    uint8_t* d_base = p.d;
+    const int out_esize = p.out_esize;
+    int group = 0;          // B operand group
+    int valid_end = M;      // rows >= valid_end are padding (psum) / not written (masked)
+    bool zero_tile = false;
+    int k_len = CK > 0 ? CK : p.k;   // K extent of this tile's contraction
+
+    if (gemm_type == kKGrouped) {
+        // K-grouped: group g contracts K rows [align(psum[g-1]), psum[g]) of A and B into D[g].
+        const int ks = batch == 0 ? 0 : align_up(p.layout[batch - 1], p.alignment);
+        k_len = __builtin_amdgcn_readfirstlane(max(0, p.layout[batch] - ks));
+        const int kso = __builtin_amdgcn_readfirstlane(ks);
+        a_base += AMN ? (int64_t)kso * p.lda : (int64_t)kso * (kAFp4 ? 1 : (kBf16 ? 4 : 2)) / 2;
+        b_base += BMN ? (int64_t)kso * p.ldb : (int64_t)kso * (kBFp4 ? 1 : (kBf16 ? 4 : 2)) / 2;
+        // (p.lda / p.ldb are in bytes: an MN-major K row is lda bytes)
+        if (!kBf16) {
+            sfa += (int64_t)(kso / 64) * p.sfa_ld;
+            sfb += (int64_t)(kso / 64) * p.sfb_ld;
+        }
+        d_base += (int64_t)batch * p.bsd * out_esize;
+    }
+
+    if (gemm_type == kBatched || gemm_type == kMasked) {
+        group = batch;
+        a_base += (int64_t)batch * p.bsa;
+        d_base += (int64_t)batch * p.bsd * out_esize;
+        if (!kBf16) sfa += (int64_t)batch * p.sfa_bs;
+        if (gemm_type == kMasked) {
+            valid_end = min(M, p.layout[batch]);
+            if (m0 >= valid_end) return false;   // whole tile beyond masked_m: nothing to write
+        }
+    } else if (anchored) {
+        group = anchor_group;
+        valid_end = anchor_valid;
+        if (group < 0) zero_tile = true;
+    } else if (gemm_type == kMGroupedPsum) {
+        int found = -1;
+        for (int base = 0; base < p.num_groups; base += 64) {
+            const int gi = base + lane;
+            bool pred = false;
+            if (gi < p.num_groups) pred = align_up(p.layout[gi], p.alignment) > m0;
+            const uint64_t mask = __ballot(pred);
+            if (mask) { found = base + __builtin_ctzll(mask); break; }
+        }
+        if (found < 0) {
+            zero_tile = true;
+        } else {
+            group = found;
+            valid_end = min(M, p.layout[found]);
+            if (valid_end <= m0) zero_tile = true;
+        }
+    } else if (gemm_type == kMGroupedIdx) {
+        group = __builtin_amdgcn_readfirstlane(p.layout[m0]);
+        // (padding rows, and ids past the last group -- which the m_indices check reports --
+        // read no B)
+        if (group < 0 || group >= p.num_groups) zero_tile = true;
+    }
+    group = __builtin_amdgcn_readfirstlane(group);
+    valid_end = __builtin_amdgcn_readfirstlane(valid_end);
+
+    if (zero_tile) {
+        // Padding-only tile of an M-grouped layout: its D rows are exact zeros (16-byte stores when
+        // the rows allow them).
+        const int rows = min(BM, tile_end - m0), cols = min(BN, N - n0);
+        const int row_bytes = cols * out_esize;
+        uint8_t* d0 = d_base + ((int64_t)m0 * p.ldd + n0) * out_esize;
+        const int64_t ld_bytes = p.ldd * out_esize;
+        if (row_bytes % 16 == 0 && ld_bytes % 16 == 0 && (reinterpret_cast<uint64_t>(d0) & 15) == 0) {
+            const int per_row = row_bytes / 16;
+            for (int e = tid; e < rows * per_row; e += NT)
+                *reinterpret_cast<i32x4*>(d0 + (int64_t)(e / per_row) * ld_bytes + (e % per_row) * 16) = i32x4{0, 0, 0, 0};
+        } else {
+            for (int e = tid; e < rows * cols; e += NT) {
+                const int rr = e / cols, cc = e % cols;
+                const int64_t off = (int64_t)(m0 + rr) * p.ldd + n0 + cc;
+                if (out_esize == 4) reinterpret_cast<float*>(d_base)[off] = 0.f;
+                else reinterpret_cast<uint16_t*>(d_base)[off] = 0;
+            }
+        }
+        return false;
+    }
+    if (gemm_type != kNormal && gemm_type != kKGrouped) {
+        b_base += (int64_t)group * p.bsb;
+        if (!kBf16) sfb += (int64_t)group * p.sfb_bs;
+    }
+
+    tl.a_base = a_base;
+    tl.b_base = b_base;
+    tl.sfa = sfa;
+    tl.sfb = sfb;
+    tl.d_base = d_base;
+    tl.m0 = m0;
+    tl.n0 = n0;
+    tl.batch = batch;
+    tl.group = group;
+    tl.valid_end = valid_end;
+    tl.tile_end = tile_end;
+    tl.k_len = k_len;
+    tl.split = split;
+    tl.tile_id = tile_id;
+    tl.anchored = anchored;
+    return true;
+}
+
 // The kernel body.  OCC = workgroups per CU the kernel is compiled for (its waves per SIMD bound
 // its registers).  CT / CS / CM / CN / CK fix the GEMM type, the K split and M / N / K at compile
 // time (-1 / 0 = read from the arguments): the ahead-of-time menu reads everything from the
@@ -641,159 +838,19 @@ __device__ __forceinline__ void gemm_body(const KParams& p, const int vb, const 
     const int wm = wave % WGM, wn = wave / WGM;
     const int r = lane & 31, q = lane >> 5;
 
-    // ------------------------------------------------------------------ tile selection
+    TileLoc tl;
+    if (!locate_tile<BM, BN, NT, KIND, CT, CS, CM, CN, CK, AMN, BMN>(p, vb, known_total, tid, tl)) return;
     const int gemm_type = CT >= 0 ? CT : p.gemm_type;
     const int split_k = CS > 0 ? CS : p.split_k;
-    const int nm = CM > 0 ? ceil_div(CM, BM) : p.num_m_blocks, nn = CN > 0 ? ceil_div(CN, BN) : p.num_n_blocks;
-    int t, split = 0;
-    if (split_k > 1) {
-        // Split-K launch: grid = 8 * ceil(tiles / 8) * split_k, and workgroup b serves tile
-        // (b / 8 / split_k) * 8 + b % 8, split (b / 8) % split_k, so all splits of a tile share
-        // b % 8 -- the XCD (and L2) the dispatcher places them on.
-        const int b = vb, r = b >> 3;
-        t = (r / split_k) * 8 + (b & 7);
-        split = r % split_k;
-        if (p.split_spread) {
-            // (test knob: consecutive workgroups -- different XCDs -- take the splits of a tile)
-            t = b / split_k;
-            split = b % split_k;
-        }
-        if (t >= p.num_tiles) return;
-    } else if (gemm_type == kKGrouped) {
-        // K-grouped: each group's tiles are spread over the XCDs on their own, so at any time all
-        // XCDs work on one group and its A / B K-slices (Kg x (M + N) bytes) are streamed once,
-        // instead of every XCD pair streaming another group's and the groups together overflowing
-        // the last-level cache.  (groups in order; a group's tiles are consecutive workgroups)
-        const int per_group = nm * nn;
-        const int g = vb / per_group;
-        t = g * per_group + xcd_remap(vb - g * per_group, per_group);
-    } else {
-        t = xcd_remap(vb, p.vgrid);
-    }
-    const int tile_id = t;
-    int batch = 0;
-    if (gemm_type == kBatched || gemm_type == kMasked || gemm_type == kKGrouped) {
-        batch = t / (nm * nn);
-        t -= batch * nm * nn;
-    }
     const int M = CM > 0 ? CM : p.m, N = CN > 0 ? CN : p.n;
-    int mb = 0, nb = 0, m0, anchor_group = -1, tile_end = M, anchor_valid = M;
-    const bool anchored = (gemm_type == kMGroupedPsum || gemm_type == kMGroupedIdx) && p.anchored && p.num_groups > 0;
-    if (anchored) {
-        const int* runs = gemm_type == kMGroupedIdx ? p.runs : nullptr;
-        // the launch's real tiles spread over the XCDs as xcd_remap spreads a full grid
-        const int total = known_total >= 0 ? known_total
-            : __builtin_amdgcn_readfirstlane(anchored_total(p.layout, p.num_groups, runs, p.alignment, BM, M, nn));
-        if (vb >= total) return;
-        t = xcd_remap(vb, total);
-        anchored_tile(p.layout, p.num_groups, runs, p.alignment, t, BM, M, nn, anchor_group, m0, nb, tile_end,
-                      anchor_valid);
-        anchor_group = __builtin_amdgcn_readfirstlane(anchor_group);
-        if (anchor_group == -2) return;   // past the last tile of this launch
-        m0 = __builtin_amdgcn_readfirstlane(m0);
-        nb = __builtin_amdgcn_readfirstlane(nb);
-        tile_end = __builtin_amdgcn_readfirstlane(tile_end);
-        anchor_valid = __builtin_amdgcn_readfirstlane(anchor_valid);
-    } else {
-        if (gemm_type == kMGroupedPsum && p.num_groups > 0)
-            expert_major_tile(p.layout, p.num_groups, p.alignment, t, BM, nm, nn, mb, nb);
-        else
-            swizzle_tile(t, nm, nn, p.group_m, mb, nb);
-        mb = __builtin_amdgcn_readfirstlane(mb);
-        nb = __builtin_amdgcn_readfirstlane(nb);
-        m0 = mb * BM;
-    }
-    const int n0 = nb * BN;
-
-    const uint8_t* a_base = p.a;
-    const uint8_t* b_base = p.b;
-    const uint16_t* sfa = p.sfa;
-    const uint16_t* sfb = p.sfb;
-    uint8_t* d_base = p.d;
-    const int out_esize = p.out_esize;
-    int group = 0;          // B operand group
-    int valid_end = M;      // rows >= valid_end are padding (psum) / not written (masked)
-    bool zero_tile = false;
-    int k_len = CK > 0 ? CK : p.k;   // K extent of this tile's contraction
-
-    if (gemm_type == kKGrouped) {
-        // K-grouped: group g contracts K rows [align(psum[g-1]), psum[g]) of A and B into D[g].
-        const int ks = batch == 0 ? 0 : align_up(p.layout[batch - 1], p.alignment);
-        k_len = __builtin_amdgcn_readfirstlane(max(0, p.layout[batch] - ks));
-        const int kso = __builtin_amdgcn_readfirstlane(ks);
-        a_base += AMN ? (int64_t)kso * p.lda : (int64_t)kso * (kAFp4 ? 1 : (kBf16 ? 4 : 2)) / 2;
-        b_base += BMN ? (int64_t)kso * p.ldb : (int64_t)kso * (kBFp4 ? 1 : (kBf16 ? 4 : 2)) / 2;
-        // (p.lda / p.ldb are in bytes: an MN-major K row is lda bytes)
-        if (!kBf16) {
-            sfa += (int64_t)(kso / 64) * p.sfa_ld;
-            sfb += (int64_t)(kso / 64) * p.sfb_ld;
-        }
-        d_base += (int64_t)batch * p.bsd * out_esize;
-    }
-
-    if (gemm_type == kBatched || gemm_type == kMasked) {
-        group = batch;
-        a_base += (int64_t)batch * p.bsa;
-        d_base += (int64_t)batch * p.bsd * out_esize;
-        if (!kBf16) sfa += (int64_t)batch * p.sfa_bs;
-        if (gemm_type == kMasked) {
-            valid_end = min(M, p.layout[batch]);
-            if (m0 >= valid_end) return;   // whole tile beyond masked_m: nothing to write
-        }
-    } else if (anchored) {
-        group = anchor_group;
-        valid_end = anchor_valid;
-        if (group < 0) zero_tile = true;
-    } else if (gemm_type == kMGroupedPsum) {
-        int found = -1;
-        for (int base = 0; base < p.num_groups; base += 64) {
-            const int gi = base + lane;
-            bool pred = false;
-            if (gi < p.num_groups) pred = align_up(p.layout[gi], p.alignment) > m0;
-            const uint64_t mask = __ballot(pred);
-            if (mask) { found = base + __builtin_ctzll(mask); break; }
-        }
-        if (found < 0) {
-            zero_tile = true;
-        } else {
-            group = found;
-            valid_end = min(M, p.layout[found]);
-            if (valid_end <= m0) zero_tile = true;
-        }
-    } else if (gemm_type == kMGroupedIdx) {
-        group = __builtin_amdgcn_readfirstlane(p.layout[m0]);
-        // (padding rows, and ids past the last group -- which the m_indices check reports --
-        // read no B)
-        if (group < 0 || group >= p.num_groups) zero_tile = true;
-    }
-    group = __builtin_amdgcn_readfirstlane(group);
-    valid_end = __builtin_amdgcn_readfirstlane(valid_end);
-
-    if (zero_tile) {
-        // Padding-only tile of an M-grouped layout: its D rows are exact zeros (16-byte stores when
-        // the rows allow them).
-        const int rows = min(BM, tile_end - m0), cols = min(BN, N - n0);
-        const int row_bytes = cols * out_esize;
-        uint8_t* d0 = d_base + ((int64_t)m0 * p.ldd + n0) * out_esize;
-        const int64_t ld_bytes = p.ldd * out_esize;
-        if (row_bytes % 16 == 0 && ld_bytes % 16 == 0 && (reinterpret_cast<uint64_t>(d0) & 15) == 0) {
-            const int per_row = row_bytes / 16;
-            for (int e = tid; e < rows * per_row; e += NT)
-                *reinterpret_cast<i32x4*>(d0 + (int64_t)(e / per_row) * ld_bytes + (e % per_row) * 16) = i32x4{0, 0, 0, 0};
-        } else {
-            for (int e = tid; e < rows * cols; e += NT) {
-                const int rr = e / cols, cc = e % cols;
-                const int64_t off = (int64_t)(m0 + rr) * p.ldd + n0 + cc;
-                if (out_esize == 4) reinterpret_cast<float*>(d_base)[off] = 0.f;
-                else reinterpret_cast<uint16_t*>(d_base)[off] = 0;
-            }
-        }
-        return;
-    }
-    if (gemm_type != kNormal && gemm_type != kKGrouped) {
-        b_base += (int64_t)group * p.bsb;
-        if (!kBf16) sfb += (int64_t)group * p.sfb_bs;
-    }
+    const int split = tl.split, tile_id = tl.tile_id, batch = tl.batch, group = tl.group, m0 = tl.m0, n0 = tl.n0;
+    const int valid_end = tl.valid_end, tile_end = tl.tile_end, k_len = tl.k_len;
+    const bool anchored = tl.anchored;
+    const uint8_t* const a_base = tl.a_base;
+    const uint8_t* const b_base = tl.b_base;
+    const uint16_t* const sfa = tl.sfa;
+    const uint16_t* const sfb = tl.sfb;
+    uint8_t* const d_base = tl.d_base;
 
     // (an anchored tile loads only its group's valid rows: the rest of the tile reads zeros)
     const int rows_a = anchored ? min(BM, valid_end - m0) : min(BM, M - m0);

@@ -1,5 +1,5 @@
-// Instantiates the tile kernel with MN-major operands (e4m3 x e4m3 and bf16 x bf16, the 128-byte-stage
-// tiles of at most 256 x 256): A, B or both read in place from [K][MN] storage (csrc/gemm_kernel.hpp,
+// Instantiates the eight-wave tile kernel with MN-major operands (bf16 x bf16, the 128-byte-stage tiles that
+// the four-wave kernel does not serve): A, B or both read in place from [K][MN] storage (csrc/gemm_kernel.hpp,
 // AMN / BMN).
 #include "gemm_tiles.hpp"
 
@@ -12,14 +12,13 @@ KernelFn mn_epi(int epi) {
     // (the anchored 384-row tiles leave no LDS for a 256-element MN-major B row)
     if constexpr (t.km != 2 || t.stages != 2 || t.bm > 256 || t.bn > 256) {
         return nullptr;
+    } else if constexpr (quad_tile(KIND, t.bm, t.bn)) {
+        return nullptr;   // (lookup_quad)
     } else {
         switch (epi) {
             case kEpiF32: return &gemm_kernel<t.bm, t.bn, t.wgm, t.nw, t.lw, t.stages, t.km, t.occ, KIND, kEpiF32, AMN, BMN>;
             case kEpiBf16: return &gemm_kernel<t.bm, t.bn, t.wgm, t.nw, t.lw, t.stages, t.km, t.occ, KIND, kEpiBf16, AMN, BMN>;
             case kEpiBf16SR: return &gemm_kernel<t.bm, t.bn, t.wgm, t.nw, t.lw, t.stages, t.km, t.occ, KIND, kEpiBf16SR, AMN, BMN>;
-            case kEpiFp8:
-                if constexpr (KIND == kFP8FP8) return &gemm_kernel<t.bm, t.bn, t.wgm, t.nw, t.lw, t.stages, t.km, t.occ, KIND, kEpiFp8, AMN, BMN>;
-                else return nullptr;
             default: return nullptr;
         }
     }
@@ -43,8 +42,8 @@ KernelFn mn_find(int bm, int bn, int epi, bool amn, bool bmn) {
 }  // namespace
 
 KernelFn lookup_kernel_mn(int kind, int bm, int bn, int epi, bool a_mn, bool b_mn) {
+    if (quad_tile(kind, bm, bn)) return lookup_quad(kind, bm, bn, epi, a_mn, b_mn);
     switch (kind) {
-        case kFP8FP8: return mn_find<kFP8FP8>(bm, bn, epi, a_mn, b_mn);
         case kBF16: return mn_find<kBF16>(bm, bn, epi, a_mn, b_mn);
         default: return nullptr;
     }

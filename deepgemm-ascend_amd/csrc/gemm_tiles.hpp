@@ -44,9 +44,26 @@ constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 // 256x224 over two wave columns: 128 + 96 -- keeps no split-K partial layout).
 constexpr bool tile_splittable(const TileCfg& t) { return t.nw == 0 || (t.bn / (t.nw / t.wgm)) % 32 == 0; }
 
+// Tiles that the four-wave kernel (quad_kernel.hpp) serves; the others run gemm_kernel.  Its 16-row blocks
+// split a side of 224 or 160 into two halves over two waves (4 + 3, 3 + 2 blocks); bf16's 32-row blocks do
+// not, and bf16 keeps the eight-wave kernel there.  FP4 x FP4 runs at twice the matrix rate and keeps it too.
+constexpr bool quad_tile(int kind, int bm, int bn) {
+    return bm == 256 && ((kind == kFP8FP8 || kind == kFP8FP4) ? bn == 256 || bn == 224 || bn == 160
+                                                              : kind == kBF16 && bn == 256);
+}
+// (FP8 output wants whole 32-column groups per wave)
+constexpr bool quad_fp8_output(int bn) { return bn == 256; }
+
+// The four-wave kernel of one tile (csrc/quad_*.hip, a translation unit per operand kind and layout; nullptr
+// where there is none).
+KernelFn lookup_quad(int kind, int bm, int bn, int epi, bool a_mn, bool b_mn);
+
 template <int I, int KIND>
 KernelFn pick_epi(int epi) {
     constexpr TileCfg t = kTiles[I];
+    if constexpr (quad_tile(KIND, t.bm, t.bn)) {
+        return nullptr;   // (lookup_quad)
+    } else {
     switch (epi) {
         case kEpiF32: return &gemm_kernel<t.bm, t.bn, t.wgm, t.nw, t.lw, t.stages, t.km, t.occ, KIND, kEpiF32, false, false, t.nsb>;
         case kEpiBf16: return &gemm_kernel<t.bm, t.bn, t.wgm, t.nw, t.lw, t.stages, t.km, t.occ, KIND, kEpiBf16, false, false, t.nsb>;
@@ -56,6 +73,7 @@ KernelFn pick_epi(int epi) {
             if constexpr (KIND == kFP8FP8) return &gemm_kernel<t.bm, t.bn, t.wgm, t.nw, t.lw, t.stages, t.km, t.occ, KIND, kEpiFp8, false, false, t.nsb>;
             else return nullptr;
         default: return nullptr;
+    }
     }
 }
 
@@ -116,7 +134,8 @@ KernelFn lookup_tile(int bm, int bn, int epi, bool persistent) {
 }
 
 // Threads per workgroup of the (bm, bn) kernel (0 if not in the menu).
-inline int tile_threads(int bm, int bn) {
+inline int tile_threads(int kind, int bm, int bn, bool persistent) {
+    if (quad_tile(kind, bm, bn) && !persistent) return 256;
     for (const TileCfg& t : kTiles)
         if (t.bm == bm && t.bn == bn) return t.nw * 64;
     return 0;
@@ -150,6 +169,8 @@ constexpr int kNumSkinnyRows = sizeof(kSkinnyRows) / sizeof(kSkinnyRows[0]);
 KernelFn lookup_skinny_rows(int kind, int mt, int nb, int d, int epi);
 // second launch of a split-K shared-ring plan: sums the partials of each 32x32 block, then its epilogue
 KernelFn lookup_split_reduce(int mt, int nb, int epi);
+// the same for split-K plans of the four-wave tile kernel
+KernelFn lookup_quad_reduce(int epi);
 
 // Decode GEMV kernels (csrc/gemv_kernel.hip): e4m3 x e4m3, M <= mr (1, 2, 4), fp32 / bf16 D;
 // whole rows of B per wave, A staged in LDS as f16 (gemv_lds(mr, k, rows per wave) bytes).

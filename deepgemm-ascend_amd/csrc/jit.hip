@@ -38,13 +38,14 @@ namespace {
 
 std::mutex g_mu;
 std::string g_include_dir;                      // directory holding gemm_kernel.hpp / dg_common.hpp
-std::string g_headers[2];                       // their text, read once
+std::string g_headers[3];                       // their text, read once
 bool g_headers_read = false;
 std::unordered_map<std::string, std::vector<char>> g_code;             // key -> code object
 std::unordered_map<std::string, hipFunction_t> g_fn;                    // key@device -> kernel
 int64_t g_stat_compiled = 0, g_stat_disk = 0, g_stat_mem = 0;
 
-const char* const kHeaderNames[2] = {"gemm_kernel.hpp", "dg_common.hpp"};
+constexpr int kNumHeaders = 3;
+const char* const kHeaderNames[kNumHeaders] = {"gemm_kernel.hpp", "dg_common.hpp", "quad_kernel.hpp"};
 const char* const kOptions[] = {"--offload-arch=gfx950", "-O3", "-std=c++20",
                                 // packed fp32 VALU ops stay off, as in the ahead-of-time build
                                 "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
@@ -77,7 +78,7 @@ std::string default_include_dir() {
 bool load_headers() {
     if (g_headers_read) return true;
     if (g_include_dir.empty()) g_include_dir = default_include_dir();
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < kNumHeaders; ++i) {
         if (!read_file(g_include_dir + "/" + kHeaderNames[i], g_headers[i])) {
             const std::string msg = "dg_jit: cannot read " + g_include_dir + "/" + kHeaderNames[i] +
                                     " (set the kernel header directory with dg_jit_set_include_dir)";
@@ -122,6 +123,15 @@ struct Spec {
 
 std::string source_of(const Spec& s) {
     char buf[768];
+    if (quad_tile(s.kind, s.t.bm, s.t.bn)) {
+        snprintf(buf, sizeof(buf),
+                 "#include \"quad_kernel.hpp\"\n"
+                 "extern \"C\" __global__ __launch_bounds__(256, 1) void dg_jit_kernel(const dg::KParams p) {\n"
+                 "    dg::quad_body<%d, %d, %d, %d, %d, %d, %d, %d, %d>(p, blockIdx.x + p.vbase);\n"
+                 "}\n",
+                 s.t.bm, s.t.bn, s.kind, s.epi, s.ct, s.cs, s.cm, s.cn, s.ck);
+        return buf;
+    }
     snprintf(buf, sizeof(buf),
              "#include \"gemm_kernel.hpp\"\n"
              "extern \"C\" __global__ __launch_bounds__(%d, %d) void dg_jit_kernel(const dg::KParams p) {\n"
@@ -136,8 +146,7 @@ std::string source_of(const Spec& s) {
 bool code_object(const std::string& src, std::string& key, const std::vector<char>*& code) {
     uint64_t h = 1469598103934665603ull;
     h = fnv1a(h, src);
-    h = fnv1a(h, g_headers[0]);
-    h = fnv1a(h, g_headers[1]);
+    for (const std::string& text : g_headers) h = fnv1a(h, text);
     for (int i = 0; i < kNumOptions; ++i) h = fnv1a(h, kOptions[i]);
     int major = 0, minor = 0;
     hiprtcVersion(&major, &minor);
@@ -161,8 +170,8 @@ bool code_object(const std::string& src, std::string& key, const std::vector<cha
         }
     }
     hiprtcProgram prog;
-    const char* hdr[2] = {g_headers[0].c_str(), g_headers[1].c_str()};
-    if (hiprtcCreateProgram(&prog, src.c_str(), "dg_jit_kernel.hip", 2, hdr, kHeaderNames) != HIPRTC_SUCCESS) {
+    const char* hdr[kNumHeaders] = {g_headers[0].c_str(), g_headers[1].c_str(), g_headers[2].c_str()};
+    if (hiprtcCreateProgram(&prog, src.c_str(), "dg_jit_kernel.hip", kNumHeaders, hdr, kHeaderNames) != HIPRTC_SUCCESS) {
         dg_set_error("dg_jit: hiprtcCreateProgram failed");
         return false;
     }
@@ -247,7 +256,7 @@ int jit_run(const dg_gemm_args& a, const TileCfg& cfg, int epi, int split, const
         size_t kp_size = sizeof(kp);
         void* config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, &kp, HIP_LAUNCH_PARAM_BUFFER_SIZE, &kp_size, HIP_LAUNCH_PARAM_END};
         const unsigned n = (unsigned)std::min<int64_t>(grid, (int64_t)p.vgrid - base);
-        const hipError_t e = hipModuleLaunchKernel(fn, n, 1, 1, (unsigned)(cfg.nw * 64), 1, 1, 0, st, nullptr, config);
+        const hipError_t e = hipModuleLaunchKernel(fn, n, 1, 1, (unsigned)tile_threads(a.kind, cfg.bm, cfg.bn, false), 1, 1, 0, st, nullptr, config);
         if (e != hipSuccess) {
             dg_set_error(hipGetErrorString(e));
             return DG_ELAUNCH;

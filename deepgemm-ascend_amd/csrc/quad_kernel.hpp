@@ -1,0 +1,885 @@
+// Four-wave GEMM tile kernel for gfx950: one wave per SIMD, each wave a quadrant of every half of the tile.
+//
+// The tile's A and B rows are cut into two halves each.  A stage is 128 bytes of K per row (128 e4m3 or
+// e2m1, 64 bf16 elements) and runs in four phases, one per pair of halves, in the order
+//   (A0, Bf) (A0, B1-f) (A1, B1-f) (A1, Bf),   f = stage parity,
+// so that consecutive phases share one operand half and every phase needs only one new half in registers:
+// phase 0 reads B1-f, phase 1 A1, phase 2 the next stage's A0 and phase 3 its first B half (B1-f, whose
+// registers the phase before has finished with).  A wave owns rows [64 w, +64) of a 128-row half and reads
+// each of its fragments from LDS exactly once per stage.
+//
+// LDS holds two stages.  Each half of a slot is refilled (buffer_load ... lds, stage c + 2) as soon as every
+// wave has read it: A0 and Bf during phases 0-1, A1 and B1-f during phases 2-3, so a load has 1 to 1.5 stages
+// to land and about 1.25 stages of bytes are in flight, against one stage for a ring that is refilled stage
+// by stage.  There are two barriers per stage (before phases 0 and 2), each behind a counted vmcnt that
+// leaves the loads of the last two half-stages in flight.
+//
+// What bounds it: matrix issue and, under sustained load, the board's power.  A 16x16x128 MFMA holds a
+// SIMD's matrix pipe for 32 cycles, in which a wave can issue about six other instructions, so LDS reads and
+// loads are dealt out one at a time between MFMAs (slots), the K offset of a stage rides in the loads' vector
+// offset and the row steps in constant scalar offsets (two instructions per load).  Measured on MI355X (e4m3,
+// 8192^3, sustained): MFMA busy 77 % of the cycles against 69 % for the eight-wave kernel it replaced, 2.9
+// against 2.5 PFLOP/s.
+//
+// e4m3 / e2m1: v_mfma_scale_f32_16x16x128_f8f6f4.  With random e4m3 operands in registers it sustains 4.26
+// PFLOP/s against 3.95 for the 32x32x64 form (less power per FLOP); errors against fp64 are the same.
+//   operand of lane l = r + 16 g (r = row 0..15, g = 0..3): e4m3 bytes [0,16) hold K [16 g, +16), bytes
+//   [16,32) K [64 + 16 g, +16); e2m1 16 bytes hold K [32 g, +32); scale = UE8M0 byte of K block g of row r;
+//   accumulator element i = column l % 16 of the second operand, row 4 g + i of the first.
+// bf16: v_mfma_f32_32x32x16_bf16 (1.78 PFLOP/s in registers, 1.44 for 16x16x32), laid out as in gemm_kernel.hpp.
+// B is the first MFMA operand, so a lane ends with runs of four consecutive columns of one row of D.
+#pragma once
+
+#include "gemm_kernel.hpp"
+
+namespace dg {
+
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
+typedef __attribute__((address_space(3))) i32x4 lds_i32x4;
+
+// s_waitcnt vmcnt(VM) lgkmcnt(0)
+template <int VM>
+__device__ __forceinline__ void wait_vmcnt_lds() {
+    constexpr int v = VM > 63 ? 63 : VM;
+    __builtin_amdgcn_s_waitcnt((v & 0xf) | ((v >> 4) << 14) | (0x7 << 4));
+}
+
+// D += first . second on v_mfma_scale_f32_16x16x128_f8f6f4, the accumulator in AGPRs (IN_V: in VGPRs).
+// Inline asm: given the builtin, the register allocator moves accumulators between the two register files
+// inside the main loop.  An MFMA needs two wait states after a VALU write of one of its operands, and a read
+// of its result must wait for the pipeline: the callers keep both distances.
+template <bool FP4_FIRST, bool IN_V>
+__device__ __forceinline__ void mfma_16x16x128(f32x4& d, const i32x4 (&x)[2], const i32x4 (&y)[2], int xs, int ys) {
+    const i32x8 yv = __builtin_shufflevector(y[0], y[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    const i32x8 x8 = __builtin_shufflevector(x[0], x[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    const i32x4 x4 = x[0];
+    if constexpr (FP4_FIRST && IN_V)
+        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0] cbsz:4"
+                     : "+v"(d) : "v"(x4), "v"(yv), "v"(xs), "v"(ys));
+    else if constexpr (FP4_FIRST)
+        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0] cbsz:4"
+                     : "+a"(d) : "v"(x4), "v"(yv), "v"(xs), "v"(ys));
+    else if constexpr (IN_V)
+        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0]"
+                     : "+v"(d) : "v"(x8), "v"(yv), "v"(xs), "v"(ys));
+    else
+        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0]"
+                     : "+a"(d) : "v"(x8), "v"(yv), "v"(xs), "v"(ys));
+}
+
+// The same for v_mfma_f32_32x32x16_bf16 (16 bytes of each operand per lane).
+template <bool IN_V>
+__device__ __forceinline__ void mfma_32x32x16_bf16(f32x16& d, const i32x4& x, const i32x4& y) {
+    if constexpr (IN_V) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(x), "v"(y));
+    else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(d) : "v"(x), "v"(y));
+}
+
+// Transposing LDS read of 8 bytes a lane at `addr` + OFF (ds_read_b64_tr_b8 / _b16).  Inline asm: before the
+// builtin the compiler waits for every buffer_load ... lds in flight (it cannot tell their destinations from
+// the read's), which drained the whole ring at each read (e4m3 4096^3 with both operands MN-major 195 us
+// against 55 us K-major).  The result arrives behind a counter the compiler does not see: arrived() before any
+// use.
+template <bool B16, int OFF>
+__device__ __forceinline__ void read_tr(i32x2& out, int addr) {
+    static_assert(OFF >= 0 && OFF < 65536, "LDS offset field");
+    if constexpr (B16) asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=&v"(out) : "v"(addr), "n"(OFF));
+    else asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=&v"(out) : "v"(addr), "n"(OFF));
+}
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// (after wait_lds: makes every later use of the values depend on the wait)
+__device__ __forceinline__ void arrived(i32x2 (&v)[4]) {
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+}
+
+// Four consecutive outputs of a row as two bf16 pairs (rounded to nearest even, or stochastically).
+template <int EPI>
+__device__ __forceinline__ i32x2 pack_quartet(f32x4 v, int n) {
+    if constexpr (EPI == kEpiBf16SR) {
+        const float x[4] = {v[0], v[1], v[2], v[3]};
+        uint16_t o[4];
+        sr_bf16_quartet(x, (uint32_t)n >> 2, o);
+        return i32x2{(int)((uint32_t)o[0] | ((uint32_t)o[1] << 16)), (int)((uint32_t)o[2] | ((uint32_t)o[3] << 16))};
+    } else {
+        return i32x2{(int)pack_bf16x2(v[0], v[1]), (int)pack_bf16x2(v[2], v[3])};
+    }
+}
+
+// Old D values (accumulate) at d: four consecutive columns, aligned for a vector load.
+template <int EPI>
+__device__ __forceinline__ f32x4 load_old4(const uint8_t* d) {
+    if constexpr (EPI == kEpiF32) {
+        return *reinterpret_cast<const f32x4*>(d);
+    } else {
+        const i32x2 w = *reinterpret_cast<const i32x2*>(d);
+        return f32x4{bf16_to_f32((uint16_t)(w[0] & 0xffff)), bf16_to_f32((uint16_t)((uint32_t)w[0] >> 16)),
+                     bf16_to_f32((uint16_t)(w[1] & 0xffff)), bf16_to_f32((uint16_t)((uint32_t)w[1] >> 16))};
+    }
+}
+
+// Four consecutive columns from n of row m, scaled by alpha already: bias, accumulate and the store, element by
+// element where the row ends or its alignment asks for it (columns past the row hash as zeros under
+// stochastic rounding).
+template <int EPI>
+__device__ __forceinline__ void store_quartet(const KParams& p, f32x4 v, uint8_t* d_base, int m, int n, int N, bool pad_row) {
+    constexpr bool kF32 = EPI == kEpiF32;
+    uint8_t* const d = d_base + ((int64_t)m * p.ldd + n) * (kF32 ? 4 : 2);
+    const bool vec = p.vec_store && n + 4 <= N;
+    f32x4 old = {0.f, 0.f, 0.f, 0.f};
+    if (p.accumulate && vec) old = load_old4<EPI == kEpiF32 ? kEpiF32 : kEpiBf16>(d);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        if (n + x >= N) {
+            v[x] = 0.f;
+            continue;
+        }
+        if (p.has_bias) v[x] += kF32 ? reinterpret_cast<const float*>(p.bias)[n + x]
+                                     : bf16_to_f32(reinterpret_cast<const uint16_t*>(p.bias)[n + x]);
+        if (p.accumulate) v[x] += vec ? old[x] : kF32 ? reinterpret_cast<const float*>(d)[x]
+                                                      : bf16_to_f32(reinterpret_cast<const uint16_t*>(d)[x]);
+    }
+    if (pad_row) v = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (kF32) {
+        if (vec) {
+            *reinterpret_cast<f32x4*>(d) = v;
+        } else {
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+                if (n + x < N) reinterpret_cast<float*>(d)[x] = v[x];
+        }
+    } else {
+        i32x2 w = pack_quartet<EPI>(v, n);
+        if (EPI == kEpiBf16SR && pad_row) w = i32x2{0, 0};
+        if (vec) {
+            *reinterpret_cast<i32x2*>(d) = w;
+        } else {
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+                if (n + x < N) reinterpret_cast<uint16_t*>(d)[x] = (uint16_t)((uint32_t)w[x >> 1] >> (16 * (x & 1)));
+        }
+    }
+}
+
+// FP8 output of a pair of 16-column blocks from column n: lane group q = lane / 16 holds columns
+// n + 4 q + {0..3} and n + 16 + 4 q + {0..3} of row m.  (n % 128 == 0 by the host's check and a wave's columns
+// start at a multiple of 32: a 32-column group lies inside the row or past it.)
+__device__ __forceinline__ void store_fp8_pair(const KParams& p, f32x4 v0, f32x4 v1, uint8_t* d_base, int m, bool row_ok,
+                                               int n, int N, int batch, int q) {
+    uint32_t amax = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint16_t b = f32_to_bf16_rne(i < 4 ? v0[i & 3] : v1[i & 3]);
+        if (i < 4) v0[i & 3] = bf16_to_f32(b); else v1[i & 3] = bf16_to_f32(b);
+        amax = max(amax, (uint32_t)(b & 0x7fffu));
+    }
+    amax = max(amax, (uint32_t)__shfl_xor((int)amax, 16));
+    amax = max(amax, (uint32_t)__shfl_xor((int)amax, 32));
+    const uint32_t sexp = ue8m0_of_bf16_amax(amax);
+    const float inv = __builtin_bit_cast(float, (254u - sexp) << 23);   // 2^(127 - s)
+    if (!row_ok || n >= N) return;
+    uint8_t* const d = d_base + (int64_t)m * p.ldd + n + 4 * q;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const f32x4 v = h ? v1 : v0;
+        int w = __builtin_amdgcn_cvt_pk_fp8_f32(v[0] * inv, v[1] * inv, 0, false);
+        w = __builtin_amdgcn_cvt_pk_fp8_f32(v[2] * inv, v[3] * inv, w, true);
+        *reinterpret_cast<int*>(d + 16 * h) = w;
+    }
+    if (q == 0) {
+        const int64_t col = (int64_t)batch * N + n;
+        p.sfd[((col >> 6) * p.sfd_ld + m) * 2 + ((col >> 5) & 1)] = (uint8_t)sexp;
+    }
+}
+
+// One operand's half-tile geometry in LDS and its loads.  MN: the operand is MN-major ([K][MN] storage).
+// MR = rows of an MFMA block, BLKS = 32 / 16-row blocks the tile has.
+template <int B, bool BF16, bool FP4, bool MN>
+struct QuadSide {
+    static constexpr int MR = BF16 ? 32 : 16;
+    static constexpr int UNITS = B / (2 * MR);               // pairs of blocks (one per wave row / column)
+    static_assert(UNITS * 2 * MR == B, "tile side");
+    static constexpr int NB0 = (UNITS + 1) / 2, NB1 = UNITS / 2;   // blocks of a wave in half 0 / 1
+    static constexpr int H0 = NB0 * 2 * MR, H1 = NB1 * 2 * MR;     // rows of half 0 / 1
+    static_assert(H0 <= 128 && NB1 >= 1, "halves of at most 128 rows");
+    static constexpr int RB = FP4 ? 64 : 128;                // bytes of one K-major LDS row
+    static constexpr int KROWS = BF16 ? 64 : 128;            // MN-major: K rows of a stage ...
+    static constexpr int PITCH = BF16 ? 256 : 128;           // ... of 128 elements each
+    // bytes of one half in LDS: K-major rows (e2m1 always 128 of them, so that every wave loads the same
+    // number of pieces), MN-major the whole K range of 128 elements
+    static constexpr int bytes(int h) { return MN ? KROWS * PITCH : FP4 ? 128 * RB : (h ? H1 : H0) * RB; }
+    static constexpr int SLOT = bytes(0) + bytes(1);
+    static constexpr int loads(int h) { return bytes(h) / 4096; }   // 1 KB wave loads per wave and half
+    static constexpr int nb(int h) { return h ? NB1 : NB0; }
+    static constexpr int rows(int h) { return h ? H1 : H0; }
+    static constexpr int RPW = 1024 / (MN ? PITCH : RB);     // LDS rows of one wave load
+    static constexpr int PPR = (MN ? PITCH : RB) / 16;       // 16-byte pieces of an LDS row
+    static constexpr int PIECES = MN ? 4 : FP4 ? 1 : 2;      // LDS reads of a fragment (MN: 8 bytes each)
+    // Piece swizzles that spread the rows of one LDS read over the banks (64 banks of 4 bytes; a read's
+    // 16-lane phases are those of gemm_kernel.hpp).  K-major: as there for 128-byte rows; 64-byte rows read
+    // by 16 rows x 4 pieces.  MN-major: the 8 (bf16: 4) K rows a 16-lane group of a transposing read touches,
+    // and the groups served together, land on distinct bank groups.
+    static __device__ __forceinline__ int swizzle(int row) {
+        if constexpr (MN) return BF16 ? ((row & 3) << 2) : (((row >> 1) & 3) | (((row >> 4) & 1) << 2));
+        else if constexpr (FP4) return (0 - (row >> 2)) & 3;
+        else return slot_swizzle<8>(row);
+    }
+};
+
+// CT / CS / CM / CN / CK: GEMM type, K split and sizes fixed at compile time (-1 / 0: from the arguments).
+template <int BM, int BN, int KIND, int EPI, int CT = -1, int CS = 0, int CM = 0, int CN = 0, int CK = 0,
+          bool AMN = false, bool BMN = false>
+__device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
+    constexpr bool kBf16 = KIND == kBF16;
+    constexpr bool kFp4B = KIND == kFP8FP4;
+    static_assert(KIND == kFP8FP8 || KIND == kFP8FP4 || KIND == kBF16, "operand kinds");
+    static_assert(!(kFp4B && BMN) && !(kFp4B && AMN), "e2m1 operands are K-major");
+    using SA = QuadSide<BM, kBf16, false, AMN>;
+    using SB = QuadSide<BN, kBf16, kFp4B, BMN>;
+    constexpr int U = kBf16 ? 2 : 1;                 // 32-byte fragments of a lane per block and stage
+    constexpr int KSTEPS = kBf16 ? 4 : 1;            // MFMAs per pair of blocks and stage
+    constexpr int KS = kBf16 ? 64 : 128;             // K elements per stage
+    constexpr int MR = SA::MR;
+    constexpr int NA0 = SA::NB0, NB0 = SB::NB0;
+    // LDS: scales of two slots ([half][A even / odd 64 K, B even / odd 64 K], 256 bytes each), A, B
+    constexpr int SF_AREA = 256, SF_SLOT = kBf16 ? 0 : 8 * SF_AREA;
+    constexpr int A_OFF = 2 * SF_SLOT, B_OFF = A_OFF + 2 * SA::SLOT, LDS_BYTES = B_OFF + 2 * SB::SLOT;
+    static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[LDS_BYTES];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    TileLoc tl;
+    if (!locate_tile<BM, BN, 256, KIND, CT, CS, CM, CN, CK, AMN, BMN>(p, vb, -1, tid, tl)) return;
+    const int gemm_type = CT >= 0 ? CT : p.gemm_type;
+    const int M = CM > 0 ? CM : p.m, N = CN > 0 ? CN : p.n;
+    const int m0 = tl.m0, n0 = tl.n0, k_len = tl.k_len;
+    const int rows_a = tl.anchored ? min(BM, tl.valid_end - m0) : min(BM, M - m0), rows_b = min(BN, N - n0);
+    // K stages of this workgroup: [c0, c0 + num_stages) of the whole K loop
+    const int split_k = CS > 0 ? CS : p.split_k;
+    const int all_stages = ceil_div(k_len, KS), nk64 = ceil_div(k_len, 64);
+    const int c0 = split_k > 1 ? tl.split * p.split_stages : 0;
+    const int num_stages = split_k > 1 ? min(p.split_stages, all_stages - c0) : all_stages;
+    constexpr int E = kBf16 ? 2 : 1;                 // bytes of an element (MN-major operands)
+
+    // ------------------------------------------------------------------ loads
+    // Wave load `it` of a half: LDS rows [RPW (4 it + wave), + RPW), 16 bytes a lane.  The lane's offset
+    // holds its row, its swizzled piece and the stage; the scalar offset the half and `it`.
+    const int64_t lda = p.lda, ldb = p.ldb;
+    const int kbytes_a = gemm_type == kKGrouped || CK > 0 ? k_len * E : p.kbytes_a;
+    const int kbytes_b = gemm_type == kKGrouped || CK > 0 ? (kFp4B ? k_len / 2 : k_len * E) : p.kbytes_b;
+    // (MN-major: the K rows of the contraction bound the range; K-major: the tile's rows)
+    const __amdgpu_buffer_rsrc_t rs_a = AMN ? make_rsrc(tl.a_base + m0 * E, (int64_t)k_len * lda - m0 * E)
+                                            : make_rsrc(tl.a_base + (int64_t)m0 * lda, (int64_t)rows_a * lda);
+    const __amdgpu_buffer_rsrc_t rs_b = BMN ? make_rsrc(tl.b_base + n0 * E, (int64_t)k_len * ldb - n0 * E)
+                                            : make_rsrc(tl.b_base + (int64_t)n0 * ldb, (int64_t)rows_b * ldb);
+    const int lrow_a = wave * SA::RPW + lane / SA::PPR, lrow_b = wave * SB::RPW + lane / SB::PPR;
+    const int piece_a = ((lane % SA::PPR) ^ SA::swizzle(lrow_a)) * 16, piece_b = ((lane % SB::PPR) ^ SB::swizzle(lrow_b)) * 16;
+    const uint32_t lane_a = (uint32_t)(lrow_a * lda + piece_a), lane_b = (uint32_t)(lrow_b * ldb + piece_b);
+    constexpr int kDeadOffset = 0x40000000;          // scalar offset that moves every lane out of range
+    int soff_a[2][4], soff_b[2][4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+            const int ra = 4 * SA::RPW * it, rb = 4 * SB::RPW * it;
+            soff_a[h][it] = (int)(AMN ? ra * lda + h * SA::H0 * E : (h * SA::H0 + ra) * lda);
+            soff_b[h][it] = (int)(BMN ? rb * ldb + h * SB::H0 * E : (h * SB::H0 + rb) * ldb);
+            // (e2m1 halves of fewer than 128 rows: the pieces past them are not loaded)
+            if (kFp4B && rb + wave * SB::RPW >= SB::rows(h)) soff_b[h][it] = kDeadOffset;
+            soff_a[h][it] = __builtin_amdgcn_readfirstlane(soff_a[h][it]);
+            soff_b[h][it] = __builtin_amdgcn_readfirstlane(soff_b[h][it]);
+        }
+    // Packed-SF loads: per half stage the four waves fetch A's and B's dwords (a row pair each) of the even
+    // and the odd 64 K.  LDS dword order [wave row / column][row pair][16-row block], so that one 16-byte
+    // read hands a lane the dwords of its row in all blocks.
+    __amdgpu_buffer_rsrc_t rs_sc;
+    uint32_t lane_sc[2] = {kOOBOffset, kOOBOffset};
+    int sc_stage = 0;
+    if constexpr (!kBf16) {
+        const bool is_a = wave < 2;
+        rs_sc = is_a ? make_rsrc(tl.sfa + m0, ((int64_t)nk64 * p.sfa_ld - m0) * 2)
+                     : make_rsrc(tl.sfb + n0, ((int64_t)nk64 * p.sfb_ld - n0) * 2);
+        const int ld2 = __builtin_amdgcn_readfirstlane((int)((is_a ? p.sfa_ld : p.sfb_ld) * 2));
+        sc_stage = 2 * ld2;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int per_wave = (is_a ? SA::rows(h) : SB::rows(h)) / 2;
+            const int row = (is_a ? h * SA::H0 : h * SB::H0) + (lane >> 5) * per_wave + (lane & 3) * 16 + ((lane >> 2) & 7) * 2;
+            if ((lane & 3) * 16 < per_wave && row < (is_a ? rows_a : rows_b)) lane_sc[h] = (uint32_t)((wave & 1) * ld2 + row * 2);
+        }
+    }
+    // Offsets of the stage whose loads go out next; past the last stage, past the K of a row and (MN-major)
+    // past the operand's columns they lie outside every range, and the lane writes zeros.
+    uint32_t va[2], vb_[2], vs[2];
+    auto set_stage = [&](int stage) {
+        const bool on = stage < num_stages;
+        const int c = c0 + stage;
+        if constexpr (AMN) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                va[h] = on && h * SA::H0 * E + piece_a < rows_a * E && piece_a < SA::rows(h) * E
+                            ? lane_a + (uint32_t)(c * KS) * (uint32_t)lda : kOOBOffset;
+        } else {
+            va[0] = va[1] = on && c * SA::RB + piece_a < kbytes_a ? lane_a + c * SA::RB : kOOBOffset;
+        }
+        if constexpr (BMN) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                vb_[h] = on && h * SB::H0 * E + piece_b < rows_b * E && piece_b < SB::rows(h) * E
+                             ? lane_b + (uint32_t)(c * KS) * (uint32_t)ldb : kOOBOffset;
+        } else {
+            vb_[0] = vb_[1] = on && c * SB::RB + piece_b < kbytes_b ? lane_b + c * SB::RB : kOOBOffset;
+        }
+        if constexpr (!kBf16) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) vs[h] = on ? lane_sc[h] + c * sc_stage : kOOBOffset;   // (a dead lane stays past the range)
+        }
+    };
+    constexpr int NSF = kBf16 ? 0 : 1;
+    // loads of a group: A half HA, B half HB (and their scales)
+    auto group_loads = [](int ha, int hb) constexpr { return SA::loads(ha) + SB::loads(hb) + NSF; };
+    auto issue = [&](auto idx_tag, auto s_tag, auto ha_tag, auto hb_tag) {
+        constexpr int IDX = decltype(idx_tag)::value, s = decltype(s_tag)::value;
+        constexpr int ha = decltype(ha_tag)::value, hb = decltype(hb_tag)::value;
+        constexpr int NLA = SA::loads(ha), NLB = SB::loads(hb);
+        if constexpr (IDX < NLA) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rs_a, (lds_void*)(smem + A_OFF + s * SA::SLOT + ha * SA::bytes(0) + IDX * 4096 + wave * 1024), 16, va[ha],
+                soff_a[ha][IDX], 0, 0);
+        } else if constexpr (IDX < NLA + NLB) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rs_b, (lds_void*)(smem + B_OFF + s * SB::SLOT + hb * SB::bytes(0) + (IDX - NLA) * 4096 + wave * 1024), 16,
+                vb_[hb], soff_b[hb][IDX - NLA], 0, 0);
+        } else if constexpr (!kBf16) {
+            const int h = wave < 2 ? ha : hb;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rs_sc, (lds_void*)(smem + s * SF_SLOT + h * 4 * SF_AREA + wave * SF_AREA), 4,
+                ha == hb ? vs[ha] : wave < 2 ? vs[ha] : vs[hb], 0, 0, 0);
+        }
+    };
+    auto issue_group = [&](int c, auto s_tag, auto ha_tag, auto hb_tag) {
+        set_stage(c);
+        static_for<group_loads(decltype(ha_tag)::value, decltype(hb_tag)::value)>([&](auto i) { issue(i, s_tag, ha_tag, hb_tag); });
+    };
+
+    // ------------------------------------------------------------------ fragments
+    const int r = lane % MR, q = lane / MR;
+    lds_u8* const lds = (lds_u8*)smem;
+    // Per-lane LDS address of piece x of K step u of a wave's first block; half, slot and (K-major) block
+    // are constant offsets from it.
+    constexpr int XA = AMN ? 1 : SA::PIECES, XB = BMN ? 1 : SB::PIECES;
+    int addr_a[U * XA * (AMN ? NA0 : 1)], addr_b[U * XB * (BMN ? NB0 : 1)];
+    const int s16 = lane & 15, g16 = lane >> 4;
+    auto mn_addr = [&](auto side, int half_row, int j, int u) -> int {
+        // transposing reads (gemm_kernel.hpp, load_frag_mn): in each 16-lane group lane s addresses 8 bytes of
+        // K row kb + s / 2 (bf16: kb + s / 4), and lane i receives consecutive K of MN row i
+        using S = decltype(side);
+        if constexpr (!kBf16) {
+            const int k = 16 * g16 + (s16 >> 1), pp = (half_row + 16 * j) >> 4;
+            return k * S::PITCH + ((pp ^ S::swizzle(k)) << 4) + (s16 & 1) * 8;
+        } else {
+            const int k = u * 32 + 8 * q + (s16 >> 2), col = half_row + 32 * j + 16 * (g16 & 1) + 4 * (s16 & 3);
+            return k * S::PITCH + (((col >> 3) ^ S::swizzle(k)) << 4) + ((col >> 2) & 1) * 8;
+        }
+    };
+    // a wave's first row of half h (rows(h) / 2 per wave); K-major addresses are taken for half 0, and half
+    // 1's rows lie at a multiple of 32 rows from them (same swizzle), MN-major ones per half
+    auto km_addr = [&](auto side, int w, int h, int u, int x) -> int {
+        using S = decltype(side);
+        const int row = w * (S::rows(h) / 2) + r;
+        int piece;
+        if constexpr (kBf16) piece = u * 4 + 2 * x + q;
+        else if constexpr (S::RB == 64) piece = q;
+        else piece = 4 * x + q;
+        return row * S::RB + ((piece ^ S::swizzle(row)) << 4);
+    };
+    // (waves 1 of an uneven side start half 1 at another row than half 0: the difference in bytes)
+    constexpr bool kEvenA = SA::H0 == SA::H1, kEvenB = SB::H0 == SB::H1;
+    int addr_a1[kEvenA ? 1 : U * XA * (AMN ? NA0 : 1)], addr_b1[kEvenB ? 1 : U * XB * (BMN ? NB0 : 1)];
+    auto fill = [&](auto side, auto mn_tag, int w, int h, int off, auto& out, auto x_tag, auto nb_tag) {
+        using S = decltype(side);
+        constexpr bool mn = decltype(mn_tag)::value != 0;
+        constexpr int X = decltype(x_tag)::value, NBX = decltype(nb_tag)::value;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if constexpr (mn) {
+#pragma unroll
+                for (int j = 0; j < NBX; ++j) out[u * NBX + j] = off + mn_addr(S{}, w * (S::rows(h) / 2), j, u);
+            } else {
+#pragma unroll
+                for (int x = 0; x < X; ++x) out[u * X + x] = off + km_addr(S{}, w, h, u, x);
+            }
+        }
+    };
+    fill(SA{}, Int<AMN>{}, wm, 0, A_OFF, addr_a, Int<XA>{}, Int<(AMN ? NA0 : 1)>{});
+    fill(SB{}, Int<BMN>{}, wn, 0, B_OFF, addr_b, Int<XB>{}, Int<(BMN ? NB0 : 1)>{});
+    if constexpr (!kEvenA) fill(SA{}, Int<AMN>{}, wm, 1, A_OFF, addr_a1, Int<XA>{}, Int<(AMN ? NA0 : 1)>{});
+    if constexpr (!kEvenB) fill(SB{}, Int<BMN>{}, wn, 1, B_OFF, addr_b1, Int<XB>{}, Int<(BMN ? NB0 : 1)>{});
+    // scales: 16 bytes = the dwords (row pair) of the wave's blocks; the lane's byte after a shift
+    const int addr_sa = (((g16 >> 1) * 2) * SF_AREA / 2) + wm * 128 + (s16 >> 1) * 16;
+    const int addr_sb = 2 * SF_AREA + (((g16 >> 1) * 2) * SF_AREA / 2) + wn * 128 + (s16 >> 1) * 16;
+    const int sc_shift = ((s16 & 1) * 2 + (g16 & 1)) * 8;
+
+    i32x4 fa[2][NA0][U][2], fb[2][NB0][U][2];        // [half][block][fragment][16 bytes]
+    i32x2 ta[NA0][U][4], tb[NB0][U][4];              // MN-major: the 8-byte pieces of the half being read
+    int sa[2][NA0], sb[2][NB0];                      // scales in the low byte
+    i32x4 sc_raw;
+    // 16-byte (MN-major: 8-byte) read X of block j, K step u
+    auto read_frag = [&](auto a_tag, auto s_tag, auto h_tag, auto j_tag, auto u_tag, auto x_tag) {
+        constexpr bool A = decltype(a_tag)::value != 0, mn = A ? AMN : BMN;
+        constexpr int s = decltype(s_tag)::value, h = decltype(h_tag)::value, j = decltype(j_tag)::value;
+        constexpr int u = decltype(u_tag)::value, x = decltype(x_tag)::value;
+        using S = typename Cond<A, SA, SB>::type;
+        constexpr int NBX = A ? NA0 : NB0, X = A ? XA : XB;
+        constexpr bool second = h == 1 && !(A ? kEvenA : kEvenB);
+        constexpr int idx = mn ? u * NBX + j : u * X + x;
+        int base;
+        if constexpr (A) base = second ? addr_a1[second ? idx : 0] : addr_a[idx];
+        else base = second ? addr_b1[second ? idx : 0] : addr_b[idx];
+        constexpr int at = s * S::SLOT + h * S::bytes(0);
+        if constexpr (mn) {
+            // e4m3: K kb .. kb + 7 with kb = 16 g + {0, 8, 64, 72}; bf16: K kb .. kb + 3 with kb = 8 q + {0, 4, 16, 20}:
+            // the K-major fragment's bytes in order
+            constexpr int kb = kBf16 ? (x & 1) * 4 + (x >> 1) * 16 : (x & 1) * 8 + (x >> 1) * 64;
+            if constexpr (A) read_tr<kBf16, at + kb * S::PITCH>(ta[j][u][x], base);
+            else read_tr<kBf16, at + kb * S::PITCH>(tb[j][u][x], base);
+        } else {
+            i32x4 (&f)[2] = A ? fa[h][A ? j : 0][u] : fb[h][A ? 0 : j][u];
+            f[x] = *(lds_i32x4*)(lds + base + at + j * MR * S::RB);
+        }
+    };
+    // MN-major: the pieces of the half just read have arrived; the fragments take them over
+    auto finish_read = [&](auto a_tag, auto h_tag) {
+        constexpr bool A = decltype(a_tag)::value != 0;
+        constexpr int h = decltype(h_tag)::value;
+        if constexpr (A ? AMN : BMN) {
+            wait_lds();
+            static_for<(A ? SA::nb(h) : SB::nb(h))>([&](auto j_c) {
+                static_for<U>([&](auto u_c) {
+                    constexpr int j = decltype(j_c)::value, u = decltype(u_c)::value;
+                    i32x2 (&t)[4] = A ? ta[A ? j : 0][u] : tb[A ? 0 : j][u];
+                    i32x4 (&f)[2] = A ? fa[h][A ? j : 0][u] : fb[h][A ? 0 : j][u];
+                    arrived(t);
+                    f[0] = __builtin_shufflevector(t[0], t[1], 0, 1, 2, 3);
+                    f[1] = __builtin_shufflevector(t[2], t[3], 0, 1, 2, 3);
+                });
+            });
+        }
+    };
+    auto read_scales = [&](auto a_tag, auto s_tag, auto h_tag) {
+        constexpr bool A = decltype(a_tag)::value != 0;
+        sc_raw = *(lds_i32x4*)(lds + (A ? addr_sa : addr_sb) + decltype(s_tag)::value * SF_SLOT + decltype(h_tag)::value * 4 * SF_AREA);
+    };
+    auto shift_scales = [&](auto a_tag, auto h_tag) {
+        constexpr bool A = decltype(a_tag)::value != 0;
+        constexpr int h = decltype(h_tag)::value;
+        static_for<(A ? SA::nb(h) : SB::nb(h))>([&](auto j_c) {
+            constexpr int j = decltype(j_c)::value;
+            const int v = (int)((uint32_t)sc_raw[j] >> sc_shift);
+            if constexpr (A) sa[h][j] = v; else sb[h][j] = v;
+        });
+    };
+
+    typedef typename Cond<kBf16, f32x16, f32x4>::type acc_t;
+    // (256 x 256 tiles would fill the AGPRs to the last one, and the allocator then moves a block in and out of
+    // them in the loop: the last 16-row blocks, or the last 32-row block, live in VGPRs, of which there are enough)
+    auto in_v = [](int ha, int hb, int i, int j) constexpr {
+        return BM * BN == 256 * 256 && ha == 1 && hb == 1 && i == NA0 - 1 && j >= (kBf16 ? 1 : 2);
+    };
+    acc_t acc[2][2][NA0][NB0];                        // [A half][B half]
+    static_for<4>([&](auto h_c) {
+        constexpr int ha = decltype(h_c)::value >> 1, hb = decltype(h_c)::value & 1;
+        static_for<SA::nb(ha)>([&](auto i) {
+            static_for<SB::nb(hb)>([&](auto j) {
+                acc_t& d = acc[ha][hb][decltype(i)::value][decltype(j)::value];
+                d = acc_t{};
+                // (zeros in place before the loop's first MFMA, two wait states and more ahead of it)
+                if constexpr (in_v(ha, hb, decltype(i)::value, decltype(j)::value)) asm volatile("" : "+v"(d));
+                else asm volatile("" : "+a"(d));
+            });
+        });
+    });
+    asm volatile("s_nop 3");
+    auto mfma = [&](auto ha_t, auto hb_t, auto i_t, auto j_t, auto u_t) {
+        constexpr int ha = decltype(ha_t)::value, hb = decltype(hb_t)::value, i = decltype(i_t)::value;
+        constexpr int j = decltype(j_t)::value, u = decltype(u_t)::value;
+        acc_t& d = acc[ha][hb][i][j];
+        if constexpr (kBf16) {
+            mfma_32x32x16_bf16<in_v(ha, hb, i, j)>(d, fb[hb][j][u >> 1][u & 1], fa[ha][i][u >> 1][u & 1]);
+        } else {
+            mfma_16x16x128<kFp4B, in_v(ha, hb, i, j)>(d, fb[hb][j][u], fa[ha][i][u], sb[hb][j], sa[ha][i]);
+        }
+    };
+
+    // ------------------------------------------------------------------ main loop
+    // Phase P of stage c in slot s (f = s).  Slot i of the phase: MFMA i, then at most one or two LDS reads
+    // and loads; scheduling barriers keep the compiler from regrouping them.
+    auto phase = [&](auto p_tag, auto s_tag, int c) {
+        constexpr int P = decltype(p_tag)::value, s = decltype(s_tag)::value, f = s;
+        constexpr int ha = P >= 2, hb = P == 0 || P == 3 ? f : 1 - f;
+        constexpr int NA = SA::nb(ha), NB = SB::nb(hb), NM = NA * NB * KSTEPS;
+        // the half read in this phase: B1-f, A1, the next stage's A0, its first B half (1 - f)
+        constexpr bool kReadA = P == 1 || P == 2;
+        constexpr int rslot = P >= 2 ? s ^ 1 : s, rh = P == 1 ? 1 : P == 2 ? 0 : 1 - f;
+        constexpr int RN = kReadA ? SA::nb(rh) : SB::nb(rh), RX = kReadA ? SA::PIECES : SB::PIECES;
+        constexpr int NR = RN * RX * U + NSF;
+        // the half stage refilled: {A0, Bf} in phases 0 and 1, {A1, B1-f} in phases 2 and 3
+        constexpr int lha = P >= 2, lhb = P >= 2 ? 1 - f : f;
+        constexpr int NL = SA::loads(lha) + SB::loads(lhb) + NSF;
+        constexpr int L0 = (P & 1) ? (NL + 1) / 2 : 0, L1 = (P & 1) ? NL : (NL + 1) / 2;
+        constexpr int first = (P & 1) == 0 ? 1 : 0;   // (slot 0 of phases 0 and 2 holds the barrier)
+        constexpr int kShift = NM >= 4 ? NM - 3 : 0;
+        // loads that may stay in flight at the barrier: the two half-stages issued last
+        constexpr int kFlight = P == 0 ? SA::loads(0) + SB::loads(1 - f) + SA::loads(1) + SB::loads(f) + 2 * NSF
+                                       : SA::loads(1) + SB::loads(f) + SA::loads(0) + SB::loads(f) + 2 * NSF;
+        static_for<NM>([&](auto i_c) {
+            constexpr int i = decltype(i_c)::value;
+            constexpr int u = i / (NA * NB), blk = i % (NA * NB);
+            // (the operand half read last is the outer loop: its first blocks arrived first)
+            if constexpr (P < 2) mfma(Int<ha>{}, Int<hb>{}, Int<blk % NA>{}, Int<blk / NA>{}, Int<u>{});
+            else mfma(Int<ha>{}, Int<hb>{}, Int<blk / NB>{}, Int<blk % NB>{}, Int<u>{});
+            if constexpr ((P & 1) == 0 && i == 0) {
+                // what the next two phases read has landed and what they refill has been read by every wave
+                // (this MFMA covers part of the wait)
+                __builtin_amdgcn_sched_barrier(0);
+                wait_vmcnt_lds<kFlight>();
+                stage_barrier();
+            }
+            static_for<NR>([&](auto b_c) {
+                constexpr int b = decltype(b_c)::value;
+                // (MN-major: the last quarter of the phase is left for the reads to arrive in)
+                constexpr int window = (kReadA ? AMN : BMN) ? (NM - first) * 3 / 4 : NM - first;
+                constexpr int at = NR <= window ? first + b : first + b * window / NR;
+                if constexpr (at == i) {
+                    if constexpr (b < NSF) {
+                        read_scales(Int<kReadA>{}, Int<rslot>{}, Int<rh>{});
+                    } else {
+                        constexpr int x = b - NSF, blkx = x / RX;
+                        read_frag(Int<kReadA>{}, Int<rslot>{}, Int<rh>{}, Int<blkx % RN>{}, Int<blkx / RN>{}, Int<x % RX>{});
+                    }
+                }
+            });
+            if constexpr (!kBf16 && i == kShift) shift_scales(Int<kReadA>{}, Int<rh>{});
+            static_for<L1 - L0>([&](auto l_c) {
+                constexpr int l = decltype(l_c)::value;
+                constexpr int at = first + l * (NM - first) / (L1 - L0);
+                if constexpr (at == i) issue(Int<L0 + l>{}, s_tag, Int<lha>{}, Int<lhb>{});
+            });
+            if constexpr (P == 3 && i == NM - 1) set_stage(c + 3);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        finish_read(Int<kReadA>{}, Int<rh>{});
+    };
+    auto stage = [&](int c, auto s_tag) {
+        phase(Int<0>{}, s_tag, c);
+        phase(Int<1>{}, s_tag, c);
+        phase(Int<2>{}, s_tag, c);
+        phase(Int<3>{}, s_tag, c);
+    };
+    issue_group(0, Int<0>{}, Int<0>{}, Int<0>{});
+    issue_group(0, Int<0>{}, Int<1>{}, Int<1>{});
+    issue_group(1, Int<1>{}, Int<0>{}, Int<1>{});
+    issue_group(1, Int<1>{}, Int<1>{}, Int<0>{});
+    wait_vmcnt_lds<SA::loads(1) + SB::loads(1) + SA::loads(0) + SB::loads(1) + SA::loads(1) + SB::loads(0) + 3 * NSF>();
+    stage_barrier();
+    static_for<2>([&](auto a_c) {
+        constexpr bool A = decltype(a_c)::value == 0;
+        if constexpr (!kBf16) {
+            read_scales(Int<A>{}, Int<0>{}, Int<0>{});
+            shift_scales(Int<A>{}, Int<0>{});
+        }
+        static_for<U>([&](auto u) {
+            static_for<(A ? NA0 : NB0)>([&](auto j) {
+                static_for<(A ? SA::PIECES : SB::PIECES)>([&](auto x) { read_frag(Int<A>{}, Int<0>{}, Int<0>{}, j, u, x); });
+            });
+        });
+        finish_read(Int<A>{}, Int<0>{});
+    });
+    set_stage(2);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 3");
+    int c = 0;
+    for (; c + 1 < num_stages; c += 2) {
+        stage(c, Int<0>{});
+        stage(c + 1, Int<1>{});
+    }
+    if (c < num_stages) stage(c, Int<0>{});
+    __builtin_amdgcn_s_waitcnt(0);
+    // (the last MFMAs' results: 19 wait states at most)
+    asm volatile("s_nop 15\n\ts_nop 7");
+    // A block's accumulator, read where it is used: the empty asm keeps the compiler from copying the whole
+    // tile out of the AGPRs ahead of the epilogue's branches.
+    auto take = [&](auto ha_c, auto hb_c, auto i_c, auto j_c) -> acc_t {
+        acc_t& t = acc[decltype(ha_c)::value][decltype(hb_c)::value][decltype(i_c)::value][decltype(j_c)::value];
+        if constexpr (in_v(decltype(ha_c)::value, decltype(hb_c)::value, decltype(i_c)::value, decltype(j_c)::value))
+            asm volatile("" : "+v"(t));
+        else
+            asm volatile("" : "+a"(t));
+        return t;
+    };
+
+    // ------------------------------------------------------------------ epilogue
+    auto row_of = [&](auto ha_c, auto i_c, int w, int rr) -> int {
+        constexpr int ha = decltype(ha_c)::value;
+        return m0 + ha * SA::H0 + w * (SA::rows(ha) / 2) + decltype(i_c)::value * MR + rr;
+    };
+    auto row_state = [&](int m, bool& row_ok, bool& pad_row) {
+        row_ok = m < tl.tile_end && !(gemm_type == kMasked && m >= tl.valid_end);
+        pad_row = false;
+        if (gemm_type == kMGroupedPsum) pad_row = m >= tl.valid_end;
+        else if (gemm_type == kMGroupedIdx) pad_row = tl.anchored ? m >= tl.valid_end : row_ok && p.layout[m] != tl.group;
+    };
+    // first column of the wave's blocks in half hb, within the tile
+    auto col_of = [&](auto hb_c) -> int {
+        constexpr int hb = decltype(hb_c)::value;
+        return hb * SB::H0 + wn * (SB::rows(hb) / 2);
+    };
+    if (split_k > 1) {
+        // This workgroup's partial tile, fp32 [BM][BN] (rows past M left out); quad_reduce_kernel sums the
+        // ranges in order and runs the epilogue.
+        float* const ws = p.ws + ((int64_t)tl.tile_id * split_k + tl.split) * (BM * BN);
+        static_for<2>([&](auto ha_c) {
+            static_for<SA::nb(decltype(ha_c)::value)>([&](auto i_c) {
+                const int m = row_of(ha_c, i_c, wm, r);
+                float* const row = ws + (m - m0) * BN;
+                static_for<2>([&](auto hb_c) {
+                    static_for<SB::nb(decltype(hb_c)::value)>([&](auto j_c) {
+                        const acc_t a = take(ha_c, hb_c, i_c, j_c);
+                        float* const d = row + col_of(hb_c) + decltype(j_c)::value * MR + 4 * q;
+                        if (m < M) {
+                            if constexpr (kBf16) {
+#pragma unroll
+                                for (int g = 0; g < 4; ++g)
+                                    *reinterpret_cast<f32x4*>(d + 8 * g) = f32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+                            } else {
+                                *reinterpret_cast<f32x4*>(d) = a;
+                            }
+                        }
+                    });
+                });
+            });
+        });
+        return;
+    }
+    constexpr bool kF32 = EPI == kEpiF32;
+    constexpr int DE = kF32 ? 4 : 2;                  // bytes of a D element (other than FP8 output)
+    if constexpr (EPI == kEpiFp8) {
+        static_assert(!kBf16 && SB::NB0 % 2 == 0 && SB::NB1 % 2 == 0, "FP8 output: whole 32-column groups per wave");
+        static_for<2>([&](auto ha_c) {
+            constexpr int ha = decltype(ha_c)::value;
+            static_for<SA::nb(ha)>([&](auto i_c) {
+                const int m = row_of(ha_c, i_c, wm, r);
+                bool row_ok, pad_row;
+                row_state(m, row_ok, pad_row);
+                static_for<2>([&](auto hb_c) {
+                    constexpr int hb = decltype(hb_c)::value;
+                    static_for<SB::nb(hb) / 2>([&](auto j_c) {
+                        constexpr int j = 2 * decltype(j_c)::value;
+                        store_fp8_pair(p, take(ha_c, hb_c, i_c, Int<j>{}) * p.alpha, take(ha_c, hb_c, i_c, Int<j + 1>{}) * p.alpha, tl.d_base, m, row_ok,
+                                       n0 + col_of(hb_c) + 16 * j, N, tl.batch, q);
+                    });
+                });
+            });
+        });
+        return;
+    } else {
+    // Vector path: D rows of whole, aligned quartets and no block of columns that the row's end cuts; else
+    // the rows go through LDS a block at a time and are stored element by element.
+    const bool vec = p.vec_store && !p.has_bias && (n0 + BN <= N || N % 32 == 0);
+    if (vec) {
+        static_for<2>([&](auto ha_c) {
+            constexpr int ha = decltype(ha_c)::value;
+            static_for<SA::nb(ha)>([&](auto i_c) {
+                const int m = row_of(ha_c, i_c, wm, r);
+                bool row_ok, pad_row;
+                row_state(m, row_ok, pad_row);
+                uint8_t* const drow = tl.d_base + ((int64_t)m * p.ldd + n0) * DE;
+                constexpr int NQ = (SB::NB0 + SB::NB1) * (kBf16 ? 4 : 1);   // quartets of a row a lane holds
+                f32x4 v[NQ];
+                int col[NQ];   // a quartet's first column within the tile
+                static_for<SB::NB0 + SB::NB1>([&](auto b_c) {
+                    constexpr int b = decltype(b_c)::value, hb = b >= SB::NB0, j = hb ? b - SB::NB0 : b;
+                    const acc_t a = take(ha_c, Int<hb>{}, i_c, Int<j>{});
+                    const int c0 = col_of(Int<hb>{}) + j * MR + 4 * q;
+                    if constexpr (kBf16) {
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            v[4 * b + g] = f32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]} * p.alpha;
+                            col[4 * b + g] = c0 + 8 * g;
+                        }
+                    } else {
+                        v[b] = a * p.alpha;
+                        col[b] = c0;
+                    }
+                });
+                if constexpr (EPI == kEpiF32 || EPI == kEpiBf16) {
+                    if (p.accumulate) {
+                        // (the row's old values in one burst, then the sums)
+                        f32x4 old[NQ];
+#pragma unroll
+                        for (int t = 0; t < NQ; ++t) {
+                            old[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                            if (row_ok && n0 + col[t] < N) old[t] = load_old4<EPI>(drow + col[t] * DE);
+                        }
+#pragma unroll
+                        for (int t = 0; t < NQ; ++t) v[t] = v[t] + old[t];
+                    }
+                }
+                if (pad_row) {
+#pragma unroll
+                    for (int t = 0; t < NQ; ++t) v[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+                if constexpr (kF32) {
+#pragma unroll
+                    for (int t = 0; t < NQ; ++t)
+                        if (row_ok && n0 + col[t] < N) *reinterpret_cast<f32x4*>(drow + col[t] * 4) = v[t];
+                } else {
+                    i32x2 pk[NQ];
+#pragma unroll
+                    for (int t = 0; t < NQ; ++t) {
+                        pk[t] = pack_quartet<EPI>(v[t], n0 + col[t]);
+                        if (EPI == kEpiBf16SR && pad_row) pk[t] = i32x2{0, 0};
+                    }
+                    if constexpr (kBf16) {
+                        // per 32-column block: after swapping the wave's halves a lane holds 16 columns in a row
+                        static_for<NQ / 4>([&](auto b_c) {
+                            constexpr int t = 4 * decltype(b_c)::value;
+                            i32x4 w[2];
+#pragma unroll
+                            for (int h = 0; h < 2; ++h) {
+                                const auto s02 = __builtin_amdgcn_permlane32_swap(pk[t + 2][h], pk[t][h], false, false);
+                                const auto s13 = __builtin_amdgcn_permlane32_swap(pk[t + 3][h], pk[t + 1][h], false, false);
+                                w[0][h] = (int)s02[0]; w[0][2 + h] = (int)s02[1];
+                                w[1][h] = (int)s13[0]; w[1][2 + h] = (int)s13[1];
+                            }
+                            const int cb = col[t] - 4 * q;
+                            if (row_ok && n0 + cb < N) {
+                                uint8_t* const d = drow + (cb + (q ? 0 : 16)) * 2;
+                                *reinterpret_cast<i32x4*>(d) = w[0];
+                                *reinterpret_cast<i32x4*>(d + 16) = w[1];
+                            }
+                        });
+                    } else {
+                        // per pair of 16-column blocks of a half: after swapping the odd and even lane groups a lane
+                        // holds eight columns in a row, 16 (q % 2) + 8 (q / 2) of the pair's 32
+                        static_for<2>([&](auto hb_c) {
+                            constexpr int hb = decltype(hb_c)::value, t0 = hb ? SB::NB0 : 0;
+                            const int cb = col_of(hb_c);
+                            static_for<SB::nb(hb) / 2>([&](auto j_c) {
+                                constexpr int j = 2 * decltype(j_c)::value, t = t0 + j;
+                                const auto s0 = __builtin_amdgcn_permlane16_swap(pk[t][0], pk[t + 1][0], false, false);
+                                const auto s1 = __builtin_amdgcn_permlane16_swap(pk[t][1], pk[t + 1][1], false, false);
+                                if (row_ok && n0 + cb + 16 * j + 16 * (q & 1) < N)
+                                    *reinterpret_cast<i32x4*>(drow + (cb + 16 * j + 16 * (q & 1) + 8 * (q >> 1)) * 2) =
+                                        i32x4{(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
+                            });
+                            if constexpr (SB::nb(hb) % 2 != 0) {
+                                constexpr int j = SB::nb(hb) - 1;
+                                if (row_ok && n0 + cb + 16 * j < N)
+                                    *reinterpret_cast<i32x2*>(drow + (cb + 16 * j + 4 * q) * 2) = pk[t0 + j];
+                            }
+                        });
+                    }
+                }
+            });
+        });
+        return;
+    }
+    static_for<2>([&](auto ha_c) {
+        constexpr int ha = decltype(ha_c)::value;
+        static_for<SA::nb(ha)>([&](auto i_c) {
+            // the block row of both wave rows, fp32: [2 MR][BN]
+            static_assert(2 * MR * BN * 4 <= LDS_BYTES, "staging area");
+            float* const st = reinterpret_cast<float*>(smem);
+            __syncthreads();
+            static_for<2>([&](auto hb_c) {
+                constexpr int hb = decltype(hb_c)::value;
+                static_for<SB::nb(hb)>([&](auto j_c) {
+                    constexpr int j = decltype(j_c)::value;
+                    float* const d = st + (wm * MR + r) * BN + col_of(hb_c) + j * MR + 4 * q;
+                    if constexpr (kBf16) {
+                        const acc_t a = take(ha_c, hb_c, i_c, j_c);
+#pragma unroll
+                        for (int g = 0; g < 4; ++g)
+                            *reinterpret_cast<f32x4*>(d + 8 * g) = f32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+                    } else {
+                        *reinterpret_cast<f32x4*>(d) = take(ha_c, hb_c, i_c, j_c);
+                    }
+                });
+            });
+            __syncthreads();
+            for (int e = tid; e < 2 * MR * (BN / 4); e += 256) {
+                const int rr = e / (BN / 4), n = n0 + e % (BN / 4) * 4;
+                const int m = row_of(ha_c, i_c, rr / MR, rr % MR);
+                bool row_ok, pad_row;
+                row_state(m, row_ok, pad_row);
+                if (!row_ok || n >= N) continue;
+                store_quartet<EPI>(p, *reinterpret_cast<const f32x4*>(st + rr * BN + (n - n0)) * p.alpha, tl.d_base, m, n, N, pad_row);
+            }
+        });
+    });
+    }
+}
+
+template <int BM, int BN, int KIND, int EPI, bool AMN = false, bool BMN = false>
+__global__ __launch_bounds__(256, 1) void quad_kernel(const KParams p) {
+    quad_body<BM, BN, KIND, EPI, -1, 0, 0, 0, 0, AMN, BMN>(p, blockIdx.x + p.vbase);
+}
+
+// Second launch of a split-K quad plan: a thread per four consecutive columns of D sums the partials of the
+// K ranges in order and stores the outputs.  Bound by the partials' bytes: one coalesced 16-byte read per
+// range, all in flight before the first add.
+template <int EPI>
+__global__ __launch_bounds__(256) void quad_reduce_kernel(const KParams p) {
+    const int bm = p.reduce_bm, bn = p.reduce_bn;
+    const int64_t e = ((int64_t)(blockIdx.x + p.vbase) * 256 + threadIdx.x) * 4;   // element of the tiles
+    const int64_t tile = e / (bm * bn);
+    if (tile >= p.num_tiles) return;
+    const int in = (int)(e - tile * (bm * bn)), rr = in / bn, cc = in % bn;
+    const int per = p.num_m_blocks * p.num_n_blocks, batch = (int)(tile / per);
+    int mb, nb;
+    swizzle_tile((int)(tile - (int64_t)batch * per), p.num_m_blocks, p.num_n_blocks, p.group_m, mb, nb);
+    const int m = mb * bm + rr, n = nb * bn + cc;
+    const bool live = m < p.m && n < p.n;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (live) {
+        const float* const src = p.ws + tile * p.split_k * (bm * bn) + in;
+        f32x4 part[8];
+        for (int s0 = 0; s0 < p.split_k; s0 += 8) {
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+                part[s] = s0 + s < p.split_k ? *reinterpret_cast<const f32x4*>(src + (int64_t)(s0 + s) * (bm * bn))
+                                             : f32x4{-0.f, -0.f, -0.f, -0.f};   // (the identity of IEEE addition)
+#pragma unroll
+            for (int s = 0; s < 8; ++s) v = s0 + s == 0 ? part[0] : v + part[s];
+        }
+    }
+    v = v * p.alpha;
+    uint8_t* const d_base = p.d + (int64_t)batch * p.bsd * p.out_esize;
+    if constexpr (EPI == kEpiFp8) {
+        // eight neighbouring threads hold 32 columns of a row
+        uint32_t amax = 0;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const uint16_t b = f32_to_bf16_rne(v[x]);
+            v[x] = bf16_to_f32(b);
+            amax = max(amax, (uint32_t)(b & 0x7fffu));
+        }
+#pragma unroll
+        for (int off = 1; off < 8; off <<= 1) amax = max(amax, (uint32_t)__shfl_xor((int)amax, off));
+        const uint32_t sexp = ue8m0_of_bf16_amax(amax);
+        const float inv = __builtin_bit_cast(float, (254u - sexp) << 23);
+        if (!live) return;
+        int w = __builtin_amdgcn_cvt_pk_fp8_f32(v[0] * inv, v[1] * inv, 0, false);
+        w = __builtin_amdgcn_cvt_pk_fp8_f32(v[2] * inv, v[3] * inv, w, true);
+        *reinterpret_cast<int*>(d_base + (int64_t)m * p.ldd + n) = w;
+        if (n % 32 == 0) {
+            const int64_t col = (int64_t)batch * p.n + n;
+            p.sfd[((col >> 6) * p.sfd_ld + m) * 2 + ((col >> 5) & 1)] = (uint8_t)sexp;
+        }
+    } else {
+        if (live) store_quartet<EPI>(p, v, d_base, m, n, p.n, false);
+    }
+}
+
+}  // namespace dg

@@ -1,0 +1,139 @@
+"""The four-wave tile kernel (csrc/quad_kernel.hpp) where it can go wrong: K of one stage, of an odd and an
+even number of stages and ending inside one; rows and columns one past and one short of a tile, a half tile and
+a block; every operand layout; D rows that take the vector path, that need element stores and that accumulate;
+K ranges summed by the second launch.  Against the CPU oracle (dequantise, fp32 matmul).  The bound on
+calc_diff is the repository's 1e-5; every element is also held to 1e-3 of itself or the root mean square (the
+alignment of e4m3 products inside one MFMA leaves up to 1.4e-4 of it), plus one unit of a bf16 result."""
+import pytest
+import torch
+
+import deep_gemm
+from oracle import gemm as og
+from helpers import gen, operand, calc_diff
+
+pytestmark = pytest.mark.gpu
+THRESH = 1e-5
+TILES = ['256x256', '256x224', '256x160', '128x128']
+
+
+@pytest.fixture
+def force(monkeypatch):
+    def _set(tile, split=None):
+        monkeypatch.setenv('DG_FORCE_BLOCK', tile)
+        if split:
+            monkeypatch.setenv('DG_SPLIT_K', str(split))
+    return _set
+
+
+def _check(d, ref):
+    """calc_diff, and every element within one bf16 unit (2^-7 of it at most, two roundings of nearly equal
+    sums) plus 1e-3 of the larger of it and the root mean square."""
+    unit = 2.0 ** -7 if d.dtype == torch.bfloat16 else 0.0
+    d, ref = d.double().cpu(), ref.double()
+    assert calc_diff(d, ref) < THRESH
+    rms = ref.pow(2).mean().sqrt()
+    off = (d - ref).abs() - unit * ref.abs()
+    worst = float((off / torch.maximum(ref.abs(), rms)).max())
+    print(f'  worst element: {worst:.2e}', flush=True)
+    assert worst <= 1e-3
+
+
+def _fp8(m, n, k, seed, b_kind='e4m3'):
+    g = gen(seed)
+    a, sfa, a_deq = operand(m, k, 'e4m3', (1, 32), g)
+    b, sfb, b_deq = operand(n, k, b_kind, (1, 32), g)
+    return (a.cuda(), sfa.cuda()), (b.cuda(), sfb.cuda()), a_deq, b_deq
+
+
+@pytest.mark.parametrize('tile', TILES)
+@pytest.mark.parametrize('m,n,k', [
+    (1, 1, 32), (255, 33, 128), (256, 160, 160), (257, 224, 256), (129, 225, 384), (191, 159, 640),
+    (300, 257, 416), (513, 480, 528), (64, 97, 1040), (400, 512, 2048)])
+def test_quad_k_major(force, tile, m, n, k):
+    print(f'quad {tile} fp8 m={m} n={n} k={k}', flush=True)
+    force(tile)
+    a, b, a_deq, b_deq = _fp8(m, n, k, 1)
+    for dt in (torch.bfloat16, torch.float32):
+        d = torch.full((m, n), float('nan'), dtype=dt, device='cuda')
+        deep_gemm.fp8_gemm_nt(a, b, d)
+        _check(d, og.gemm_nt(a_deq, b_deq, dt))
+
+
+@pytest.mark.parametrize('tile', TILES)
+@pytest.mark.parametrize('m,n,k', [(255, 225, 128), (257, 96, 352), (130, 500, 704)])
+def test_quad_fp4(force, tile, m, n, k):
+    print(f'quad {tile} fp8 x fp4 m={m} n={n} k={k}', flush=True)
+    force(tile)
+    a, b, a_deq, b_deq = _fp8(m, n, k, 2, 'e2m1')
+    d = torch.full((m, n), float('nan'), dtype=torch.bfloat16, device='cuda')
+    deep_gemm.fp8_fp4_gemm_nt(a, b, d)
+    _check(d, og.gemm_nt(a_deq, b_deq))
+
+
+@pytest.mark.parametrize('tile', ['256x256', '256x224', '128x128'])
+@pytest.mark.parametrize('form', ['nn', 'tn', 'tt'])
+@pytest.mark.parametrize('m,n,k', [(256, 224, 128), (272, 240, 416), (144, 496, 1152)])
+def test_quad_mn_major(force, tile, form, m, n, k):
+    print(f'quad {tile} {form} m={m} n={n} k={k}', flush=True)
+    force(tile)
+    (a, sfa), (b, sfb), a_deq, b_deq = _fp8(m, n, k, 3)
+    if form[0] == 't':
+        a, sfa = a.t().contiguous(), sfa.t().contiguous()
+    if form[1] == 'n':
+        b, sfb = b.t().contiguous(), sfb.t().contiguous()
+    d = torch.full((m, n), float('nan'), dtype=torch.float32, device='cuda')
+    getattr(deep_gemm, 'fp8_gemm_' + form)((a, sfa), (b, sfb), d)
+    _check(d, og.gemm_nt(a_deq, b_deq, torch.float32))
+
+
+@pytest.mark.parametrize('tile', ['256x256', '128x128'])
+@pytest.mark.parametrize('form', ['nt', 'nn', 'tn', 'tt'])
+@pytest.mark.parametrize('m,n,k', [(256, 256, 64), (264, 120, 200), (136, 392, 520)])
+def test_quad_bf16(force, tile, form, m, n, k):
+    print(f'quad {tile} bf16 {form} m={m} n={n} k={k}', flush=True)
+    force(tile)
+    g = gen(4)
+    a = (torch.randn(m, k, generator=g) * 0.1).bfloat16()
+    b = (torch.randn(n, k, generator=g) * 0.1).bfloat16()
+    x = (a if form[0] == 'n' else a.t().contiguous()).cuda()
+    y = (b if form[1] == 't' else b.t().contiguous()).cuda()
+    d = torch.full((m, n), float('nan'), dtype=torch.float32, device='cuda')
+    getattr(deep_gemm, 'bf16_gemm_' + form)(x, y, d)
+    _check(d, og.gemm_nt(a.float(), b.float(), torch.float32))
+
+
+@pytest.mark.parametrize('tile', TILES)
+@pytest.mark.parametrize('dt', [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize('n', [224, 231])
+def test_quad_accumulate_bias(force, tile, dt, n):
+    """D += A . B^T and a bias row, on rows of whole quartets and on rows that need element stores."""
+    m, k = 270, 384
+    print(f'quad {tile} accumulate / bias {dt} n={n}', flush=True)
+    force(tile)
+    a, b, a_deq, b_deq = _fp8(m, n, k, 5)
+    ref = og.gemm_nt(a_deq, b_deq, torch.float32)
+    scale = float(ref.abs().mean())
+    c = (torch.randn(m, n, generator=gen(6)) * scale).to(dt)
+    d = c.clone().cuda()
+    deep_gemm.fp8_gemm_nt(a, b, d, c=d)
+    _check(d, (ref + c.float()).to(dt))
+    bias = (torch.randn(1, n, generator=gen(7)) * scale).to(dt)
+    d = torch.full((m, n), float('nan'), dtype=dt, device='cuda')
+    deep_gemm.fp8_gemm_nt(a, b, d, c=bias.cuda())
+    _check(d, (ref + bias.float()).to(dt))
+
+
+@pytest.mark.parametrize('tile,split', [('256x256', 2), ('256x256', 5), ('128x128', 3), ('128x128', 11)])
+@pytest.mark.parametrize('m,n,k', [(300, 260, 1408), (130, 127, 2000)])
+def test_quad_split(force, tile, split, m, n, k):
+    """K ranges of one or several stages; the bf16 D is the rounding of the fp32 D."""
+    print(f'quad {tile} split {split} m={m} n={n} k={k}', flush=True)
+    force(tile, split)
+    a, b, a_deq, b_deq = _fp8(m, n, k, 8)
+    out = {}
+    for dt in (torch.float32, torch.bfloat16):
+        d = torch.full((m, n), float('nan'), dtype=dt, device='cuda')
+        deep_gemm.fp8_gemm_nt(a, b, d)
+        _check(d, og.gemm_nt(a_deq, b_deq, dt))
+        out[dt] = d
+    assert torch.equal(out[torch.bfloat16], out[torch.float32].bfloat16())
