@@ -8,6 +8,7 @@
 // (256 CUs, waves-of-tiles quantisation, measured cycles per K stage of each tile shape and a
 // fixed per-tile cost) and memoises the choice per problem signature.
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -132,7 +133,9 @@ struct Plan {
 };
 
 // K elements of one kernel stage of tile t
-int k_stage_elems(int kind, const TileCfg& t) { return (kind == kBF16 ? 32 : 64) * std::max(1, t.km); }
+int k_stage_elems(int kind, const TileCfg& t) {
+    return (kind == kBF16 ? 32 : 64) * (quad_tile(kind, t.bm, t.bn) ? 2 : std::max(1, t.km));
+}
 
 // Split-K is offered to dense / batched GEMMs whose tiles alone cannot fill the CUs.
 bool split_capable(const dg_gemm_args& a) { return a.gemm_type == kNormal || a.gemm_type == kBatched; }
@@ -420,6 +423,65 @@ bool tile_persistable(const TileCfg& t) {
 // CUs the launch may occupy are capped below the device's (set_num_sms).
 bool cus_capped(int cus) { return cus < device_cus(); }
 
+// Cost model of the four-wave kernel, fitted to measurements on MI355X (M 136..4096 at N x K 2112x7168,
+// 4096x7168, 7168x2048, 24576x1536, 7168x16384; every tile, K splits of 1 to 8; us).  A tile's 128-byte stage
+// takes `light` while few tiles run and, with many, the chip's share (L2 bandwidth and power): `share` times
+// the tiles running at once; the two meet as a fourth-power mean (bf16 256x256: 0.94 at 128 tiles, 1.13 at 168,
+// 1.35 at 224, 1.48 at 256).  `fixed` is its prologue and epilogue.
+struct QuadRate {
+    int bm, bn, occ;
+    double light, share, fixed;
+};
+constexpr QuadRate kQuadFp8[] = {{256, 256, 1, 0.94, 0.0045, 7.5}, {256, 224, 1, 0.815, 0.0040, 8.2}, {256, 160, 1, 0.64, 0.0030, 7.5},
+                                 {256, 128, 1, 0.54, 0.00245, 6.5}, {128, 128, 2, 0.353, 0.00172, 6.5}};
+constexpr QuadRate kQuadBf16[] = {{256, 256, 1, 0.87, 0.0058, 9.0}, {256, 128, 1, 0.49, 0.00334, 6.5}, {128, 128, 2, 0.32, 0.00217, 6.0}};
+// MN-major operands of a 128-row tile come in half lines and fill the LDS of a whole CU (bf16 tn 4096^3: 163 us
+// against 115 on 256x256 tiles)
+constexpr QuadRate kQuadMn128 = {128, 128, 1, 0.48, 0.0022, 7.0};
+
+double quad_time(const QuadRate& q, int64_t tiles, int stages, int cus) {
+    const int64_t slots = (int64_t)cus * q.occ, full = tiles / slots, rest = tiles % slots;
+    auto round = [&](int64_t running) {
+        // (two tiles on a CU share its path to the L2)
+        const double one = q.light * (running > cus ? 2 : 1), l = one * one, c = q.share * running * q.share * running;
+        return stages * std::sqrt(std::sqrt(l * l + c * c)) + q.fixed;
+    };
+    return full * round(slots) + (rest ? round(rest) : 0.0);
+}
+
+// Best four-wave plan by that model.  K is split while the ranges still run at once; their fp32 partials are
+// written and read back (7 TB/s, mostly from the caches) and summed by a second launch (3.5 us).
+bool quad_plan(const dg_gemm_args& a, int cus, bool allow_split, Plan& out) {
+    if (a.kind == kFP4FP4) return false;
+    const bool bf16 = a.kind == kBF16, mn = a.a_mn_major || a.b_mn_major;
+    const int groups = (a.gemm_type == kBatched || a.gemm_type == kMasked || a.gemm_type == kKGrouped) ? a.num_groups : 1;
+    const int k_tile = a.gemm_type == kKGrouped ? ceil_div(a.k, std::max(1, a.num_groups)) : a.k;
+    const int ns = std::max(1, ceil_div(k_tile, bf16 ? 64 : 128));
+    const QuadRate* const rates = bf16 ? kQuadBf16 : kQuadFp8;
+    const int num = bf16 ? (int)(sizeof(kQuadBf16) / sizeof(QuadRate)) : (int)(sizeof(kQuadFp8) / sizeof(QuadRate));
+    double best = 1e300;
+    for (int i = 0; i < num; ++i) {
+        const QuadRate q = mn && rates[i].bm == 128 ? kQuadMn128 : rates[i];
+        if (!tile_allowed(a, q.bm, q.bn)) continue;
+        TileCfg tc = {};
+        for (const TileCfg& c : kTiles)
+            if (c.bm == q.bm && c.bn == q.bn) tc = c;
+        const int64_t tiles = plan_tiles(a, tc), slots = (int64_t)cus * q.occ;
+        for (int sp = 1; sp <= 8 && sp <= ns; ++sp) {
+            if (sp > 1 && (!allow_split || tiles * sp > slots || tiles > kMaxSplitTiles || ns < 4 * sp)) break;
+            const int sps = ceil_div(ns, sp);
+            if (ceil_div(ns, sps) != sp) continue;
+            double t = quad_time(q, tiles * sp, sps, cus);
+            if (sp > 1) t += 3.5 + 8.0 * sp * a.m * (double)a.n * groups / 7e6;
+            if (t < best * (sp > 1 ? 0.97 : 1.0)) {
+                best = t;
+                out = {tc, sp, sps, 0, 0, 0};
+            }
+        }
+    }
+    return best < 1e300;
+}
+
 Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
     Plan skinny;
     if (skinny_kernel_plan(a, cus, allow_split, skinny_env(), skinny)) return skinny;
@@ -438,6 +500,8 @@ Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
         for (const TileCfg& tc : kTiles)
             if (tc.bm == 384 && tc.bn == (fp4_b ? 128 : 192)) return {tc, 1, ceil_div(a.k, k_stage_elems(a.kind, tc)), 0, 0, 0};
     }
+    Plan quad;
+    if (quad_plan(a, cus, allow_split, quad)) return quad;
     allow_split = false;   // wide problems fill the CUs with tiles
     const int groups = (a.gemm_type == kBatched || a.gemm_type == kMasked || a.gemm_type == kKGrouped) ? a.num_groups : 1;
     // (K-grouped: each tile contracts one group's share of K)
@@ -457,7 +521,7 @@ Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
         if (!tile_allowed(a, tc.bm, tc.bn) || tile_anchored(tc.bm)) continue;
         const int ns = ceil_div(k_tile, k_stage_elems(a.kind, tc));
         const int64_t tiles = plan_tiles(a, tc);
-        const int max_split = allow_split && tile_splittable(tc) && tiles <= kMaxSplitTiles ? std::min(16, std::max(1, ns / 4)) : 1;
+        const int max_split = allow_split && tile_splittable(a.kind, tc) && tiles <= kMaxSplitTiles ? std::min(16, std::max(1, ns / 4)) : 1;
         for (int sp = 1; sp <= max_split; ++sp) {
             const int sps = ceil_div(ns, sp);
             const int s_eff = ceil_div(ns, sps);
@@ -510,7 +574,7 @@ Plan choose(const dg_gemm_args& a, int cus, bool allow_split) {
         for (const TileCfg& c : kTiles)
             if (c.bm == a.block_m && c.bn == a.block_n) t = c;
         const int ns = ceil_div(a.k, k_stage_elems(a.kind, t));
-        int sp = allow_split && tile_splittable(t) && a.split_k > 1 && plan_tiles(a, t) <= kMaxSplitTiles ? std::min(a.split_k, std::max(1, ns)) : 1;
+        int sp = allow_split && tile_splittable(a.kind, t) && a.split_k > 1 && plan_tiles(a, t) <= kMaxSplitTiles ? std::min(a.split_k, std::max(1, ns)) : 1;
         const int sps = ceil_div(ns, sp);
         return {t, ceil_div(ns, sps), sps, 0, 0, 0};
     }
@@ -542,7 +606,7 @@ Plan choose(const dg_gemm_args& a, int cus, bool allow_split) {
         }
         return pl;
     }
-    if (allow_split && tile_splittable(pl.tile) && a.split_k > 1 && plan_tiles(a, pl.tile) <= kMaxSplitTiles) {
+    if (allow_split && tile_splittable(a.kind, pl.tile) && a.split_k > 1 && plan_tiles(a, pl.tile) <= kMaxSplitTiles) {
         // forced split count (tuning), on the heuristic's tile shape
         const int ns = ceil_div(a.k, k_stage_elems(a.kind, pl.tile));
         const int sps = ceil_div(ns, std::min(a.split_k, std::max(1, ns)));
@@ -737,7 +801,11 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
     if (plan.split > 1 && lib_ws) {
         if (!plan_only && !compile_only) {
             const int rc = stream_workspace(reinterpret_cast<hipStream_t>(stream), plan_workspace(a, plan), &workspace);
-            if (rc != DG_OK) return rc;
+            if (rc != DG_OK) {
+                // (a tile plan also runs unsplit: a call captured before its workspace exists does not need one)
+                if (plan.skinny_nw > 0 || a.split_k > 1) return rc;
+                plan = choose(a, cus, false);
+            }
         }
     } else if (plan.split > 1 && plan_workspace(a, plan) > a.workspace_bytes) {
         if (a.split_k > 1) return dg_set_error("dg_gemm: workspace smaller than dg_gemm_workspace_size() reports");
@@ -753,8 +821,8 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
     if (cfg.bm == 0) return dg_set_error("dg_gemm: no tile shape fits this problem");
     // (MN-major B also in the skinny kernel's 32-column plans)
     const bool skinny_mn = bmn && !amn && plan.skinny_nw > 0 && !plan.skinny_rows && cfg.bn == 32;
-    if ((amn || bmn) && !skinny_mn && (plan.skinny_nw > 0 || plan.split != 1 || cfg.km != 2 || cfg.stages != 2 ||
-                                       cfg.bm > 256 || cfg.bn > 256)) {
+    if ((amn || bmn) && !skinny_mn && (plan.skinny_nw > 0 || (!quad_tile(a.kind, cfg.bm, cfg.bn) &&
+                                       (plan.split != 1 || cfg.km != 2 || cfg.stages != 2 || cfg.bm > 256 || cfg.bn > 256)))) {
         dg_set_error("dg_gemm: MN-major operands need a 128-byte-stage tile plan (large M and N); this problem "
                      "plans another kernel");
         return DG_ENOKERNEL;
@@ -1092,7 +1160,10 @@ extern "C" int dg_gemm_noalloc(const dg_gemm_args* args, void* stream) {
     a.workspace = reinterpret_cast<void*>(1);   // (any non-null value: the plan may then split K)
     int rc = dg_gemm_workspace_size(&a, &need);
     if (rc != DG_OK) return rc;
-    if (need > kNoAllocScratchBytes) {
+    // (a tile plan whose partials do not fit runs unsplit instead)
+    const int cus = a.num_cus > 0 ? a.num_cus : dg::device_cus();
+    const bool falls_back = need > 0 && a.split_k <= 1 && dg::choose(a, cus, true).skinny_nw == 0;
+    if (need > kNoAllocScratchBytes && !falls_back) {
         char buf[200];
         snprintf(buf, sizeof(buf), "dg_gemm_noalloc: this problem's split-K plan needs %lld bytes of scratch, more than "
                  "the %lld-byte maximum (call dg_gemm with a workspace, or split_k = 1)", (long long)need,

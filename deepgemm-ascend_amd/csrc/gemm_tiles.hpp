@@ -40,19 +40,21 @@ constexpr TileCfg kTiles[] = {
 };
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
-// Split-K runs on tiles whose waves split N into equal 32-column multiples (a ragged tile --
-// 256x224 over two wave columns: 128 + 96 -- keeps no split-K partial layout).
-constexpr bool tile_splittable(const TileCfg& t) { return t.nw == 0 || (t.bn / (t.nw / t.wgm)) % 32 == 0; }
-
 // Tiles that the four-wave kernel (quad_kernel.hpp) serves; the others run gemm_kernel.  Its 16-row blocks
 // split a side of 224 or 160 into two halves over two waves (4 + 3, 3 + 2 blocks); bf16's 32-row blocks do
 // not, and bf16 keeps the eight-wave kernel there.  FP4 x FP4 runs at twice the matrix rate and keeps it too.
 constexpr bool quad_tile(int kind, int bm, int bn) {
-    return bm == 256 && ((kind == kFP8FP8 || kind == kFP8FP4) ? bn == 256 || bn == 224 || bn == 160
-                                                              : kind == kBF16 && bn == 256);
+    if (kind == kFP4FP4) return false;
+    return (bm == 256 && (bn == 256 || bn == 128 || (kind != kBF16 && (bn == 224 || bn == 160)))) || (bm == 128 && bn == 128);
 }
 // (FP8 output wants whole 32-column groups per wave)
-constexpr bool quad_fp8_output(int bn) { return bn == 256; }
+constexpr bool quad_fp8_output(int bn) { return bn == 256 || bn == 128; }
+
+// Split-K runs on tiles whose waves split N into equal 32-column multiples (a ragged tile --
+// 256x224 over two wave columns: 128 + 96 -- keeps no split-K partial layout).
+constexpr bool tile_splittable(int kind, const TileCfg& t) {
+    return quad_tile(kind, t.bm, t.bn) || t.nw == 0 || (t.bn / (t.nw / t.wgm)) % 32 == 0;
+}
 
 // The four-wave kernel of one tile (csrc/quad_*.hip, a translation unit per operand kind and layout; nullptr
 // where there is none).

@@ -38,7 +38,7 @@ namespace {
 
 std::mutex g_mu;
 std::string g_include_dir;                      // directory holding gemm_kernel.hpp / dg_common.hpp
-std::string g_headers[3];                       // their text, read once
+std::string g_headers[3];                       // the kernel headers' text, read once
 bool g_headers_read = false;
 std::unordered_map<std::string, std::vector<char>> g_code;             // key -> code object
 std::unordered_map<std::string, hipFunction_t> g_fn;                    // key@device -> kernel
@@ -79,7 +79,10 @@ bool load_headers() {
     if (g_headers_read) return true;
     if (g_include_dir.empty()) g_include_dir = default_include_dir();
     for (int i = 0; i < kNumHeaders; ++i) {
-        if (!read_file(g_include_dir + "/" + kHeaderNames[i], g_headers[i])) {
+        // (a directory set by dg_jit_set_include_dir may hold the first two headers only; the four-wave kernel's
+        // then comes from the library's own)
+        if (!read_file(g_include_dir + "/" + kHeaderNames[i], g_headers[i]) &&
+            !(i == 2 && read_file(default_include_dir() + "/" + kHeaderNames[i], g_headers[i]))) {
             const std::string msg = "dg_jit: cannot read " + g_include_dir + "/" + kHeaderNames[i] +
                                     " (set the kernel header directory with dg_jit_set_include_dir)";
             dg_set_error(msg.c_str());
@@ -126,10 +129,10 @@ std::string source_of(const Spec& s) {
     if (quad_tile(s.kind, s.t.bm, s.t.bn)) {
         snprintf(buf, sizeof(buf),
                  "#include \"quad_kernel.hpp\"\n"
-                 "extern \"C\" __global__ __launch_bounds__(256, 1) void dg_jit_kernel(const dg::KParams p) {\n"
+                 "extern \"C\" __global__ __launch_bounds__(256, dg::quad_occupancy(%d, %d)) void dg_jit_kernel(const dg::KParams p) {\n"
                  "    dg::quad_body<%d, %d, %d, %d, %d, %d, %d, %d, %d>(p, blockIdx.x + p.vbase);\n"
                  "}\n",
-                 s.t.bm, s.t.bn, s.kind, s.epi, s.ct, s.cs, s.cm, s.cn, s.ck);
+                 s.t.bm, s.t.bn, s.t.bm, s.t.bn, s.kind, s.epi, s.ct, s.cs, s.cm, s.cn, s.ck);
         return buf;
     }
     snprintf(buf, sizeof(buf),

@@ -821,8 +821,12 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
     }
 }
 
+// Workgroups per CU: two 128 x 128 tiles share a CU (68 KB of LDS each) and cover each other's prologue, epilogue
+// and LDS latency.
+constexpr int quad_occupancy(int bm, int bn) { return bm * bn <= 128 * 128 ? 2 : 1; }
+
 template <int BM, int BN, int KIND, int EPI, bool AMN = false, bool BMN = false>
-__global__ __launch_bounds__(256, 1) void quad_kernel(const KParams p) {
+__global__ __launch_bounds__(256, quad_occupancy(BM, BN)) void quad_kernel(const KParams p) {
     quad_body<BM, BN, KIND, EPI, -1, 0, 0, 0, 0, AMN, BMN>(p, blockIdx.x + p.vbase);
 }
 
