@@ -29,24 +29,51 @@ struct SfParams {
 // Is SF index `i` (operand rows / K columns [i*gran, (i+1)*gran)) inside the padding of a psum
 // layout, i.e. in [ceil(psum[g] / gran), align(psum[g], alignment) / gran) for the group g whose
 // aligned end is the first beyond i*gran?  The M-grouped layout pads MN rows, the K-grouped one K.
-__device__ __forceinline__ bool psum_is_padding(const SfParams& p, int i, int gran) {
+// Every lane of a wave asks together: up to 64 groups are read once, an entry a lane, and searched
+// with shuffles (a binary search in memory is a chain of dependent loads: 3 of the 8.3 us of 8064 x 7168
+// over 32 groups, and searched anew for each column 10 of the 15.6 us of a K-grouped 32768 x 7168).
+struct PsumLanes {
+    int value;          // psum[lane]
+    bool in_lanes;
+};
+
+__device__ __forceinline__ PsumLanes read_psum(const SfParams& p) {
+    const int lane = threadIdx.x & 63;
+    PsumLanes s = {0, p.psum != nullptr && p.num_groups >= 1 && p.num_groups <= 64};
+    if (s.in_lanes && lane < p.num_groups) s.value = p.psum[lane];
+    return s;
+}
+
+__device__ __forceinline__ bool psum_is_padding(const SfParams& p, const PsumLanes& s, int i, int gran) {
     const int row = i * gran;
-    int lo = 0, hi = p.num_groups;   // first g with align(psum[g]) > row
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (align_up(p.psum[mid], p.alignment) > row) hi = mid;
-        else lo = mid + 1;
+    int first = 0, value = 0;   // first g with align(psum[g]) > row
+    if (s.in_lanes) {
+#pragma unroll
+        for (int w = 64; w > 0; w >>= 1) {
+            if (w > p.num_groups) continue;
+            const int at = first + w - 1;
+            if (align_up(__shfl(s.value, at & 63, 64), p.alignment) <= row && at < p.num_groups) first += w;
+        }
+        value = __shfl(s.value, first & 63, 64);
+    } else {
+        int hi = p.num_groups;
+        while (first < hi) {
+            const int mid = (first + hi) >> 1;
+            if (align_up(p.psum[mid], p.alignment) > row) hi = mid;
+            else first = mid + 1;
+        }
+        if (first < p.num_groups) value = p.psum[first];
     }
-    if (lo == p.num_groups) return false;   // beyond the last group: untouched
-    return i >= ceil_div(p.psum[lo], gran);
+    if (first >= p.num_groups) return false;   // beyond the last group: untouched
+    return i >= ceil_div(value, gran);
 }
 
 // Is SF row i of an M-grouped operand padding?  num_groups >= 1: the psum layout above; -1: `psum`
 // holds the m_indices of the rows (gran_mn 1), a negative index marking a padding row.
-__device__ __forceinline__ bool mn_is_padding(const SfParams& p, int i) {
+__device__ __forceinline__ bool mn_is_padding(const SfParams& p, const PsumLanes& s, int i) {
     if (p.psum == nullptr) return false;
-    if (p.num_groups < 0) return p.psum[i] < 0;
-    return psum_is_padding(p, i, p.gran_mn);
+    if (p.num_groups < 0) return i < p.sf_mn && p.psum[i] < 0;
+    return psum_is_padding(p, s, i, p.gran_mn);
 }
 
 // kKGrouped: the psum layout splits K (csrc/apis/layout.hpp:94-111): SF of the K padding between
@@ -60,10 +87,10 @@ constexpr int kSfKPB = 2;   // 64-wide K columns per workgroup
 
 // Source bits of SF column j (fp32) for output column k64 half h, or 0 past the range / padding.
 template <bool kKGrouped>
-__device__ __forceinline__ bool sf_column_live(const SfParams& p, int k64, int h, int& j) {
+__device__ __forceinline__ bool sf_column_live(const SfParams& p, const PsumLanes& s, int k64, int h, int& j) {
     const int blk = 2 * k64 + h;   // 32-wide K block
     j = p.gran_k == 128 ? blk >> 2 : blk;
-    return __builtin_amdgcn_readfirstlane(blk < p.k32 && j < p.sf_k && !(kKGrouped && psum_is_padding(p, j, p.gran_k)));
+    return __builtin_amdgcn_readfirstlane(blk < p.k32 && j < p.sf_k && !(kKGrouped && psum_is_padding(p, s, j, p.gran_k)));
 }
 
 template <bool kFloat, bool kKGrouped, bool kVec>
@@ -71,7 +98,12 @@ __global__ __launch_bounds__(256) void transform_sf_kernel(const SfParams p) {
     constexpr int V = kVec ? 4 : 1;
     const int mn0 = (blockIdx.x * 256 + threadIdx.x) * V;
     const int b = blockIdx.z;
-    if (mn0 >= p.ld) return;
+    const PsumLanes groups = read_psum(p);
+    const int i = mn0 / p.gran_mn;
+    const bool mn_pad = !kKGrouped && !kVec && mn_is_padding(p, groups, i);
+    const bool row_ok = mn0 < p.mn && i < p.sf_mn && !mn_pad;
+    uint32_t bits[4] = {0, 0, 0, 0};   // (vector path) the source column read last ...
+    int held = -1;                     // ... and its index: four 32-wide blocks share one at gran_k = 128
 #pragma unroll
     for (int kk = 0; kk < kSfKPB; ++kk) {
         const int k64 = blockIdx.y * kSfKPB + kk;
@@ -79,52 +111,39 @@ __global__ __launch_bounds__(256) void transform_sf_kernel(const SfParams p) {
         uint16_t out[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) out[v] = 0;
-        if constexpr (kFloat && kVec) {
-            // (gran_mn == 1, stride_mn == 1, no psum on MN: row i = mn)
+        if constexpr (kFloat) {
             const uint32_t* s = reinterpret_cast<const uint32_t*>(p.src) + (int64_t)b * p.stride_b;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 int j;
-                if (!sf_column_live<kKGrouped>(p, k64, h, j)) continue;
+                if (!sf_column_live<kKGrouped>(p, groups, k64, h, j)) continue;
                 const uint32_t* col = s + (int64_t)j * p.stride_k;
-                uint32_t bits[4] = {0, 0, 0, 0};
-                if (mn0 + 4 <= p.mn) {
-                    const i32x4 w = *reinterpret_cast<const i32x4*>(col + mn0);
-                    bits[0] = w[0]; bits[1] = w[1]; bits[2] = w[2]; bits[3] = w[3];
+                if constexpr (kVec) {
+                    // (gran_mn == 1, stride_mn == 1, no psum on MN: row i = mn)
+                    if (held != j) {
+                        held = j;
+                        if (mn0 + 4 <= p.mn) {
+                            const i32x4 w = *reinterpret_cast<const i32x4*>(col + mn0);
+                            bits[0] = w[0]; bits[1] = w[1]; bits[2] = w[2]; bits[3] = w[3];
+                        } else {
+                            for (int v = 0; v < 4; ++v) bits[v] = mn0 + v < p.mn ? col[mn0 + v] : 0;
+                        }
+                    }
                 } else {
-                    for (int v = 0; v < 4; ++v)
-                        if (mn0 + v < p.mn) bits[v] = col[mn0 + v];
+                    bits[0] = row_ok ? col[(int64_t)i * p.stride_mn] : 0;
                 }
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    if ((bits[v] & 0x807fffffu) != 0 && mn0 + v < p.mn && p.err != nullptr) *p.err = 1;
+                for (int v = 0; v < V; ++v) {
+                    if ((bits[v] & 0x807fffffu) != 0 && p.err != nullptr) *p.err = 1;
                     out[v] |= (uint16_t)(((bits[v] >> 23) & 0xffu) << (8 * h));
                 }
             }
         } else {
-            const int mn = mn0;
-            const int i = mn / p.gran_mn;
-            const bool mn_pad = !kKGrouped && i < p.sf_mn && mn_is_padding(p, i);
-            if (mn < p.mn && i < p.sf_mn && !mn_pad) {
-                const int64_t row_off = (int64_t)b * p.stride_b + (int64_t)i * p.stride_mn;
-                if constexpr (kFloat) {
-                    const uint32_t* s = reinterpret_cast<const uint32_t*>(p.src);
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        int j;
-                        if (!sf_column_live<kKGrouped>(p, k64, h, j)) continue;
-                        const uint32_t bits = s[row_off + (int64_t)j * p.stride_k];
-                        if ((bits & 0x807fffffu) != 0 && p.err != nullptr) *p.err = 1;
-                        out[0] |= (uint16_t)(((bits >> 23) & 0xffu) << (8 * h));
-                    }
-                } else {
-                    const uint16_t* s = reinterpret_cast<const uint16_t*>(p.src);
-                    const bool live =
-                        __builtin_amdgcn_readfirstlane(k64 < p.sf_k && !(kKGrouped && psum_is_padding(p, k64, 64)));
-                    if (live) out[0] = s[row_off + (int64_t)k64 * p.stride_k];
-                }
-            }
+            const uint16_t* s = reinterpret_cast<const uint16_t*>(p.src) + (int64_t)b * p.stride_b;
+            const bool live = __builtin_amdgcn_readfirstlane(k64 < p.sf_k && !(kKGrouped && psum_is_padding(p, groups, k64, 64)));
+            if (live && row_ok) out[0] = s[(int64_t)i * p.stride_mn + (int64_t)k64 * p.stride_k];
         }
+        if (mn0 >= p.ld) continue;
         int16_t* d = p.dst + (int64_t)b * p.dst_stride_b + (int64_t)k64 * p.ld + mn0;
         if constexpr (kVec) {
             if (mn0 + 4 <= p.ld) {
@@ -139,59 +158,62 @@ __global__ __launch_bounds__(256) void transform_sf_kernel(const SfParams p) {
     }
 }
 
-// K-major fp32 sources (one contiguous row of SF per MN index, the reference's usual [MN, K / gran]
-// layout): a thread owns one MN index and kSfKPBK 64-wide K columns, reading the row's span of
-// them with 16-byte loads (the whole 128-byte line for gran_k = 32) instead of one scattered
-// float per output; the stores stay coalesced along MN.
-constexpr int kSfKPBK = 16;
+// K-major fp32 sources (one contiguous row of SF per MN index, the reference's usual [MN, K / gran] layout):
+// a workgroup turns 64 MN rows x 16 source floats through LDS.  One 16-byte load a thread (four threads read 64
+// consecutive bytes of a row), its four exponent bytes into LDS, then row pairs of a 64-wide K column per 4-byte
+// store, 128 consecutive bytes per column.  Latency-bound at the sizes of a GEMM's scales: many small
+// workgroups, one load deep.  (A thread per row that read a whole span and stored sixteen columns, launch and
+// GEMM included, 128 x 7168 x 2048: 14.6 us against 12.2; 1237 x 2112 x 7168: 32.0 against 29.3; eight batches of
+// 4096 x 1024 x 4096, both operands: 128 against 119.)
+constexpr int kSfRows = 64, kSfFloats = 16;
 
 template <bool kKGrouped>
 __global__ __launch_bounds__(256) void transform_sf_kmajor_kernel(const SfParams p) {
-    constexpr int F = 2 * kSfKPBK;             // floats of a block's K span at gran_k = 32
-    const int mn = blockIdx.x * 256 + threadIdx.x;
-    const int b = blockIdx.z, kbase = blockIdx.y * kSfKPBK;
-    if (mn >= p.ld) return;
-    const int i = mn / p.gran_mn;
-    const bool mn_pad = !kKGrouped && i < p.sf_mn && mn_is_padding(p, i);
-    const bool row_ok = mn < p.mn && i < p.sf_mn && !mn_pad;
-    const int per = p.gran_k == 128 ? 4 : 1;   // 32-wide K blocks per source float
-    const int j0 = 2 * kbase / per;            // first source float of the span
-    const int nf = F / per;                    // floats of the span (32 or 8)
-    uint32_t f[F];
+    constexpr int PITCH = kSfFloats / 4 + 1;   // dwords of an LDS row (odd: rows on distinct banks)
+    __shared__ uint32_t bytes[kSfRows * PITCH];
+    const int tid = threadIdx.x, b = blockIdx.z, mn0 = blockIdx.x * kSfRows;
+    const PsumLanes groups = read_psum(p);
+    {
+        const int row = tid >> 2, piece = tid & 3;
+        const int mn = mn0 + row, i = mn / p.gran_mn;
+        const bool mn_pad = !kKGrouped && mn_is_padding(p, groups, i);
+        const int j = (int)blockIdx.y * kSfFloats + 4 * piece;   // source columns [j, j + 4)
+        uint32_t f[4] = {0, 0, 0, 0};
+        if (mn < p.mn && i < p.sf_mn && !mn_pad) {
+            const uint32_t* src = reinterpret_cast<const uint32_t*>(p.src) + (int64_t)b * p.stride_b + (int64_t)i * p.stride_mn;
+            if (j + 4 <= p.sf_k) {
+                // (16-byte aligned: the host checks the row stride, j is a multiple of 4)
+                const i32x4 w = *reinterpret_cast<const i32x4*>(src + j);
+                f[0] = w[0]; f[1] = w[1]; f[2] = w[2]; f[3] = w[3];
+            } else {
 #pragma unroll
-    for (int t = 0; t < F; ++t) f[t] = 0;
-    if (row_ok) {
-        const uint32_t* row = reinterpret_cast<const uint32_t*>(p.src) + (int64_t)b * p.stride_b + (int64_t)i * p.stride_mn;
-        if (j0 + nf <= p.sf_k) {
-            // (16-byte aligned: the host checks the row stride, j0 is a multiple of 8)
-#pragma unroll
-            for (int t = 0; t < F / 4; ++t)
-                if (t * 4 < nf) {
-                    const i32x4 w = *reinterpret_cast<const i32x4*>(row + j0 + 4 * t);
-                    f[4 * t] = w[0]; f[4 * t + 1] = w[1]; f[4 * t + 2] = w[2]; f[4 * t + 3] = w[3];
-                }
-        } else {
-            for (int t = 0; t < nf; ++t)
-                if (j0 + t < p.sf_k) f[t] = row[j0 + t];
-        }
-    }
-#pragma unroll
-    for (int kk = 0; kk < kSfKPBK; ++kk) {
-        const int k64 = kbase + kk;
-        if (k64 >= p.k64) break;
-        uint16_t out = 0;
-        if (row_ok) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                int j;
-                if (!sf_column_live<kKGrouped>(p, k64, h, j)) continue;
-                // (constant register indices: j - j0 is 2 kk + h, or its quarter at gran_k = 128)
-                const uint32_t bits = per == 1 ? f[2 * kk + h] : f[(2 * kk + h) >> 2];
-                if ((bits & 0x807fffffu) != 0 && p.err != nullptr) *p.err = 1;
-                out |= (uint16_t)(((bits >> 23) & 0xffu) << (8 * h));
+                for (int t = 0; t < 4; ++t)
+                    if (j + t < p.sf_k) f[t] = src[j + t];
             }
         }
-        p.dst[(int64_t)b * p.dst_stride_b + (int64_t)k64 * p.ld + mn] = (int16_t)out;
+        uint32_t packed = 0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            if (kKGrouped && psum_is_padding(p, groups, j + t, p.gran_k)) f[t] = 0;
+            if ((f[t] & 0x807fffffu) != 0 && p.err != nullptr) *p.err = 1;
+            packed |= ((f[t] >> 23) & 0xffu) << (8 * t);
+        }
+        bytes[row * PITCH + piece] = packed;
+    }
+    __syncthreads();
+    const int per = p.gran_k == 128 ? 4 : 1;   // 32-wide K blocks per source float
+    const int cols = kSfFloats * per / 2;      // 64-wide K columns of the workgroup
+    const int pair = tid & 31, mn = mn0 + 2 * pair;
+    if (mn >= p.ld) return;
+    const uint8_t* const lo = reinterpret_cast<const uint8_t*>(bytes + 2 * pair * PITCH);
+    const uint8_t* const hi = lo + 4 * PITCH;
+    for (int c = tid >> 5; c < cols; c += 8) {
+        const int k64 = (int)blockIdx.y * cols + c;
+        if (k64 >= p.k64) break;
+        const int x0 = 2 * c / per, x1 = (2 * c + 1) / per;
+        const uint32_t odd = 2 * k64 + 1 < p.k32 ? 0xff00ff00u : 0;   // (K ends inside the column)
+        const uint32_t even = lo[x0] | ((uint32_t)hi[x0] << 16), next = lo[x1] | ((uint32_t)hi[x1] << 16);
+        *reinterpret_cast<uint32_t*>(p.dst + (int64_t)b * p.dst_stride_b + (int64_t)k64 * p.ld + mn) = even | (next << 8 & odd);
     }
 }
 
@@ -250,11 +272,12 @@ static int transform_sf_impl(bool k_grouped, const void* src, int32_t src_kind, 
                      (reinterpret_cast<uintptr_t>(src) % 16) == 0 && stride_k % 4 == 0 &&
                      (num_batches == 1 || stride_b % 4 == 0) && p.ld % 4 == 0 &&
                      (reinterpret_cast<uintptr_t>(dst) % 8) == 0 && (num_batches == 1 || dst_stride_b % 4 == 0);
-    // K-major path: fp32 rows contiguous along K, 16-byte aligned rows
+    // K-major path: fp32 rows contiguous along K, 16-byte aligned rows, 4-byte stores
     const bool kmajor = !vec && src_kind == DG_SF_F32 && stride_k == 1 && (reinterpret_cast<uintptr_t>(src) % 16) == 0 &&
-                        stride_mn % 4 == 0 && (num_batches == 1 || stride_b % 4 == 0);
-    const dim3 blocks((unsigned)ceil_div(p.ld, 256 * (vec ? 4 : 1)), (unsigned)ceil_div(p.k64, kmajor ? kSfKPBK : kSfKPB),
-                      (unsigned)num_batches);
+                        stride_mn % 4 == 0 && (num_batches == 1 || stride_b % 4 == 0) &&
+                        (reinterpret_cast<uintptr_t>(dst) % 4) == 0 && (num_batches == 1 || dst_stride_b % 2 == 0);
+    const dim3 blocks((unsigned)ceil_div(p.ld, kmajor ? kSfRows : 256 * (vec ? 4 : 1)),
+                      (unsigned)ceil_div(p.k64, kmajor ? kSfFloats * (gran_k == 128 ? 4 : 1) / 2 : kSfKPB), (unsigned)num_batches);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     if (kmajor) {
         if (k_grouped) hipLaunchKernelGGL((transform_sf_kmajor_kernel<true>), blocks, dim3(256), 0, st, p);

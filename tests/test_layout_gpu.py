@@ -139,3 +139,29 @@ def test_transpose_to_k_major(dtype, batch, k, mn):
     got = out.cpu().view(bits)
     assert torch.equal(got[..., :k], expect)
     assert int(got[..., k:].count_nonzero()) == 0
+
+
+@pytest.mark.parametrize('groups', [1, 33, 64, 65])
+@pytest.mark.parametrize('gran_k', [32, 128])
+def test_transform_sf_group_counts(groups, gran_k):
+    """The padding search, an entry a lane up to 64 groups and in memory beyond; K ends inside a 64-wide column
+    and inside a 128-wide scale; rows and K columns past a workgroup's 64 rows x 16 scales."""
+    alignment, k = 32, 4128 if gran_k == 128 else 1056
+    sizes = [(7 * i * i) % 75 for i in range(groups)]
+    sizes[0] = 33
+    total, ps = ol.psum_from_sizes(sizes, alignment)
+    sf = _make_sf((total, -(-k // gran_k)), torch.float32, gen(groups))
+    exp_src = sf.clone()
+    for span in ol.psum_pad_slices(ps, alignment, 1):
+        exp_src[span] = 0
+        sf[span] = -1
+    exp = ol.transform_sf(exp_src, total, k, 1, gran_k)
+    old = deep_gemm.get_mk_alignment_for_contiguous_layout()
+    deep_gemm.set_mk_alignment_for_contiguous_layout(alignment)
+    try:
+        out = deep_gemm.transform_sf_into_required_layout(sf.cuda(), total, k, (1, gran_k), is_sfa=True,
+                                                          psum_layout=torch.tensor(ps, dtype=torch.int32).cuda())
+    finally:
+        deep_gemm.set_mk_alignment_for_contiguous_layout(old)
+    torch.cuda.synchronize()
+    _check(out, exp)
