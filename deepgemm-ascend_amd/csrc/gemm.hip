@@ -812,7 +812,7 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
         plan = choose(a, cus, false);
     }
     if (a.d_dtype == DG_DTYPE_FP8_E4M3 && plan.skinny_nw == 0 && quad_tile(a.kind, plan.tile.bm, plan.tile.bn) &&
-        !quad_fp8_output(plan.tile.bn)) {
+        !quad_fp8_output(plan.tile.bm, plan.tile.bn)) {
         // FP8 output needs whole 32-column groups per wave: the 256-column tile, whose sums are the same
         for (const TileCfg& t : kTiles)
             if (t.bm == 256 && t.bn == 256) plan.tile = t;
@@ -987,7 +987,7 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
             return DG_ENOKERNEL;
         }
     }
-    int threads = skinny ? plan.skinny_nw * 64 : tile_threads(a.kind, cfg.bm, cfg.bn, persistent);
+    int threads = skinny ? plan.skinny_nw * 64 : tile_threads(a.kind, cfg.bm, cfg.bn, persistent || walk);
     unsigned lds_bytes = 0;
     if (gemv_mr > 0) {
         // workgroups of 8 waves / ks rows of B, dealt over the XCDs in contiguous runs

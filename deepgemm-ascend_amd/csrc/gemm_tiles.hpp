@@ -43,12 +43,16 @@ constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 // Tiles that the four-wave kernel (quad_kernel.hpp) serves; the others run gemm_kernel.  Its 16-row blocks
 // split a side of 224 or 160 into two halves over two waves (4 + 3, 3 + 2 blocks); bf16's 32-row blocks do
 // not, and bf16 keeps the eight-wave kernel there.  FP4 x FP4 runs at twice the matrix rate and keeps it too.
+// The anchored 384-row tiles: e4m3 at 384x192 (288 accumulators a lane; G=32 routed, 8192 rows, alignment 128,
+// N=4096 K=7168 with the scale transform 354 us on eight waves, 303 on four), e2m1 B at 384x128; bf16's 32-row
+// blocks would leave a wave column of 384x192 no whole number of them.
 constexpr bool quad_tile(int kind, int bm, int bn) {
     if (kind == kFP4FP4) return false;
+    if (bm == 384) return kind != kBF16 && (bn == 128 || (bn == 192 && kind == kFP8FP8));
     return (bm == 256 && (bn == 256 || bn == 128 || (kind != kBF16 && (bn == 224 || bn == 160)))) || (bm == 128 && bn == 128);
 }
 // (FP8 output wants whole 32-column groups per wave)
-constexpr bool quad_fp8_output(int bn) { return bn == 256 || bn == 128; }
+constexpr bool quad_fp8_output(int bm, int bn) { return bm <= 256 && (bn == 256 || bn == 128); }
 
 // Split-K runs on tiles whose waves split N into equal 32-column multiples (a ragged tile --
 // 256x224 over two wave columns: 128 + 96 -- keeps no split-K partial layout).

@@ -199,7 +199,7 @@ struct QuadSide {
     static_assert(UNITS * 2 * MR == B, "tile side");
     static constexpr int NB0 = (UNITS + 1) / 2, NB1 = UNITS / 2;   // blocks of a wave in half 0 / 1
     static constexpr int H0 = NB0 * 2 * MR, H1 = NB1 * 2 * MR;     // rows of half 0 / 1
-    static_assert(H0 <= 128 && NB1 >= 1, "halves of at most 128 rows");
+    static_assert(H0 <= 192 && NB1 >= 1 && (!MN || H0 <= 128), "halves of at most 192 rows (MN-major: 128)");
     static constexpr int RB = FP4 ? 64 : 128;                // bytes of one K-major LDS row
     static constexpr int KROWS = BF16 ? 64 : 128;            // MN-major: K rows of a stage ...
     static constexpr int PITCH = BF16 ? 256 : 128;           // ... of 128 elements each
@@ -224,32 +224,41 @@ struct QuadSide {
     }
 };
 
-// CT / CS / CM / CN / CK: GEMM type, K split and sizes fixed at compile time (-1 / 0: from the arguments).
-template <int BM, int BN, int KIND, int EPI, int CT = -1, int CS = 0, int CM = 0, int CN = 0, int CK = 0,
-          bool AMN = false, bool BMN = false>
-__device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
+// A tile's sides and LDS: scales of two slots ([half][A even / odd 64 K, B even / odd 64 K]; 256 bytes each, 512
+// where a wave owns more than four blocks of an A half), A, B.
+template <int BM, int BN, int KIND, bool AMN, bool BMN>
+struct QuadTile {
+    static_assert(KIND == kFP8FP8 || KIND == kFP8FP4 || KIND == kBF16, "operand kinds");
+    static_assert(KIND != kFP8FP4 || (!AMN && !BMN), "e2m1 operands are K-major");
+    using SA = QuadSide<BM, KIND == kBF16, false, AMN>;
+    using SB = QuadSide<BN, KIND == kBF16, KIND == kFP8FP4, BMN>;
+    static constexpr bool kWide = SA::NB0 > 4;
+    static_assert(SB::NB0 <= 4, "scale dwords of a B half: four blocks per wave");
+    static constexpr int SF_A = kWide ? 512 : 256, SF_B = 256, SF_HALF = 2 * (SF_A + SF_B), SF_SLOT = KIND == kBF16 ? 0 : 2 * SF_HALF;
+    static constexpr int A_OFF = 2 * SF_SLOT, B_OFF = A_OFF + 2 * SA::SLOT, LDS_BYTES = B_OFF + 2 * SB::SLOT;
+    static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
+};
+
+// One tile.  LIVE: blocks of A half 1 that hold valid rows; the others are not read and contribute no MFMA, and
+// their sums are zero.  (A tile that takes another LIVE runs a body of its own: loops that join before one epilogue
+// made the register allocator spill the accumulators.)
+template <int BM, int BN, int KIND, int EPI, int CT, int CS, int CM, int CN, int CK, bool AMN, bool BMN, int LIVE>
+__device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& tl, uint8_t* const smem) {
     constexpr bool kBf16 = KIND == kBF16;
     constexpr bool kFp4B = KIND == kFP8FP4;
-    static_assert(KIND == kFP8FP8 || KIND == kFP8FP4 || KIND == kBF16, "operand kinds");
-    static_assert(!(kFp4B && BMN) && !(kFp4B && AMN), "e2m1 operands are K-major");
-    using SA = QuadSide<BM, kBf16, false, AMN>;
-    using SB = QuadSide<BN, kBf16, kFp4B, BMN>;
+    using T = QuadTile<BM, BN, KIND, AMN, BMN>;
+    using SA = typename T::SA;
+    using SB = typename T::SB;
+    constexpr bool kWide = T::kWide;
+    constexpr int SF_A = T::SF_A, SF_B = T::SF_B, SF_HALF = T::SF_HALF, SF_SLOT = T::SF_SLOT, A_OFF = T::A_OFF, B_OFF = T::B_OFF;
     constexpr int U = kBf16 ? 2 : 1;                 // 32-byte fragments of a lane per block and stage
     constexpr int KSTEPS = kBf16 ? 4 : 1;            // MFMAs per pair of blocks and stage
     constexpr int KS = kBf16 ? 64 : 128;             // K elements per stage
     constexpr int MR = SA::MR;
     constexpr int NA0 = SA::NB0, NB0 = SB::NB0;
-    // LDS: scales of two slots ([half][A even / odd 64 K, B even / odd 64 K], 256 bytes each), A, B
-    constexpr int SF_AREA = 256, SF_SLOT = kBf16 ? 0 : 8 * SF_AREA;
-    constexpr int A_OFF = 2 * SF_SLOT, B_OFF = A_OFF + 2 * SA::SLOT, LDS_BYTES = B_OFF + 2 * SB::SLOT;
-    static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[LDS_BYTES];
-
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 1, wn = wave >> 1;
-    TileLoc tl;
-    if (!locate_tile<BM, BN, 256, KIND, CT, CS, CM, CN, CK, AMN, BMN>(p, vb, -1, tid, tl)) return;
     const int gemm_type = CT >= 0 ? CT : p.gemm_type;
     const int M = CM > 0 ? CM : p.m, N = CN > 0 ? CN : p.n;
     const int m0 = tl.m0, n0 = tl.n0, k_len = tl.k_len;
@@ -276,41 +285,61 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
     const int piece_a = ((lane % SA::PPR) ^ SA::swizzle(lrow_a)) * 16, piece_b = ((lane % SB::PPR) ^ SB::swizzle(lrow_b)) * 16;
     const uint32_t lane_a = (uint32_t)(lrow_a * lda + piece_a), lane_b = (uint32_t)(lrow_b * ldb + piece_b);
     constexpr int kDeadOffset = 0x40000000;          // scalar offset that moves every lane out of range
-    int soff_a[2][4], soff_b[2][4];
+    int soff_a[2][6], soff_b[2][4];
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int it = 0; it < 6; ++it) {
+            const int ra = 4 * SA::RPW * it;
+            soff_a[h][it] = __builtin_amdgcn_readfirstlane((int)(AMN ? ra * lda + h * SA::H0 * E : (h * SA::H0 + ra) * lda));
+        }
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
-            const int ra = 4 * SA::RPW * it, rb = 4 * SB::RPW * it;
-            soff_a[h][it] = (int)(AMN ? ra * lda + h * SA::H0 * E : (h * SA::H0 + ra) * lda);
+            const int rb = 4 * SB::RPW * it;
             soff_b[h][it] = (int)(BMN ? rb * ldb + h * SB::H0 * E : (h * SB::H0 + rb) * ldb);
             // (e2m1 halves of fewer than 128 rows: the pieces past them are not loaded)
             if (kFp4B && rb + wave * SB::RPW >= SB::rows(h)) soff_b[h][it] = kDeadOffset;
-            soff_a[h][it] = __builtin_amdgcn_readfirstlane(soff_a[h][it]);
             soff_b[h][it] = __builtin_amdgcn_readfirstlane(soff_b[h][it]);
         }
-    // Packed-SF loads: per half stage the four waves fetch A's and B's dwords (a row pair each) of the even
-    // and the odd 64 K.  LDS dword order [wave row / column][row pair][16-row block], so that one 16-byte
-    // read hands a lane the dwords of its row in all blocks.
-    __amdgpu_buffer_rsrc_t rs_sc;
-    uint32_t lane_sc[2] = {kOOBOffset, kOOBOffset};
-    int sc_stage = 0;
+    }
+    // Packed-SF loads, a dword = the bytes of a row pair and 64 K: per half stage the four waves fetch A's and
+    // B's dwords of the even and the odd 64 K (kWide: each A wave row's by a wave, then B's by two waves and,
+    // the same dwords again, by the other two).  LDS dword order [wave row / column][row pair][16-row block], so
+    // that one 16-byte read hands a lane the dwords of its row in four blocks.
+    constexpr int NSF = kBf16 ? 0 : kWide ? 2 : 1;    // SF loads per wave and half stage
+    __amdgpu_buffer_rsrc_t rs_sc, rs_sc2;
+    uint32_t lane_sc[2] = {kOOBOffset, kOOBOffset}, lane_sc2[2] = {kOOBOffset, kOOBOffset};
+    int sc_stage = 0, sc_stage2 = 0;
     if constexpr (!kBf16) {
-        const bool is_a = wave < 2;
-        rs_sc = is_a ? make_rsrc(tl.sfa + m0, ((int64_t)nk64 * p.sfa_ld - m0) * 2)
-                     : make_rsrc(tl.sfb + n0, ((int64_t)nk64 * p.sfb_ld - n0) * 2);
-        const int ld2 = __builtin_amdgcn_readfirstlane((int)((is_a ? p.sfa_ld : p.sfb_ld) * 2));
-        sc_stage = 2 * ld2;
+        const __amdgpu_buffer_rsrc_t rs_sfa = make_rsrc(tl.sfa + m0, ((int64_t)nk64 * p.sfa_ld - m0) * 2);
+        const __amdgpu_buffer_rsrc_t rs_sfb = make_rsrc(tl.sfb + n0, ((int64_t)nk64 * p.sfb_ld - n0) * 2);
+        const int lda2 = __builtin_amdgcn_readfirstlane((int)(p.sfa_ld * 2)), ldb2 = __builtin_amdgcn_readfirstlane((int)(p.sfb_ld * 2));
+        const int pair = ((lane >> 2) & 7) * 2, blk = lane & 3, w = lane >> 5;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int per_wave = (is_a ? SA::rows(h) : SB::rows(h)) / 2;
-            const int row = (is_a ? h * SA::H0 : h * SB::H0) + (lane >> 5) * per_wave + (lane & 3) * 16 + ((lane >> 2) & 7) * 2;
-            if ((lane & 3) * 16 < per_wave && row < (is_a ? rows_a : rows_b)) lane_sc[h] = (uint32_t)((wave & 1) * ld2 + row * 2);
+            // (A rows alternate between the wave rows block by block, a wave's B rows are contiguous)
+            const int row_b = h * SB::H0 + w * (SB::rows(h) / 2) + blk * 16 + pair;
+            const uint32_t off_b = blk < SB::nb(h) && row_b < rows_b ? (uint32_t)((wave & 1) * ldb2 + row_b * 2) : kOOBOffset;
+            if constexpr (kWide) {
+                const int wide_blk = lane & 7, row_a = h * SA::H0 + wide_blk * 32 + (wave & 1) * 16 + (lane >> 3) * 2;
+                if (wide_blk < SA::nb(h) && row_a < rows_a) lane_sc[h] = (uint32_t)((wave >> 1) * lda2 + row_a * 2);
+                lane_sc2[h] = off_b;
+            } else {
+                const int row_a = h * SA::H0 + blk * 32 + w * 16 + pair;
+                const uint32_t off_a = blk < SA::nb(h) && row_a < rows_a ? (uint32_t)((wave & 1) * lda2 + row_a * 2) : kOOBOffset;
+                lane_sc[h] = wave < 2 ? off_a : off_b;
+            }
+        }
+        rs_sc = kWide || wave < 2 ? rs_sfa : rs_sfb;
+        sc_stage = kWide || wave < 2 ? 2 * lda2 : 2 * ldb2;
+        if constexpr (kWide) {
+            rs_sc2 = rs_sfb;
+            sc_stage2 = 2 * ldb2;
         }
     }
     // Offsets of the stage whose loads go out next; past the last stage, past the K of a row and (MN-major)
     // past the operand's columns they lie outside every range, and the lane writes zeros.
-    uint32_t va[2], vb_[2], vs[2];
+    uint32_t va[2], vb_[2], vs[2], vs2[2];
     auto set_stage = [&](int stage) {
         const bool on = stage < num_stages;
         const int c = c0 + stage;
@@ -332,10 +361,12 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
         }
         if constexpr (!kBf16) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) vs[h] = on ? lane_sc[h] + c * sc_stage : kOOBOffset;   // (a dead lane stays past the range)
+            for (int h = 0; h < 2; ++h) {   // (a dead lane stays past the range)
+                vs[h] = on ? lane_sc[h] + c * sc_stage : kOOBOffset;
+                if constexpr (kWide) vs2[h] = on ? lane_sc2[h] + c * sc_stage2 : kOOBOffset;
+            }
         }
     };
-    constexpr int NSF = kBf16 ? 0 : 1;
     // loads of a group: A half HA, B half HB (and their scales)
     auto group_loads = [](int ha, int hb) constexpr { return SA::loads(ha) + SB::loads(hb) + NSF; };
     auto issue = [&](auto idx_tag, auto s_tag, auto ha_tag, auto hb_tag) {
@@ -350,11 +381,16 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 rs_b, (lds_void*)(smem + B_OFF + s * SB::SLOT + hb * SB::bytes(0) + (IDX - NLA) * 4096 + wave * 1024), 16,
                 vb_[hb], soff_b[hb][IDX - NLA], 0, 0);
+        } else if constexpr (kWide && IDX == NLA + NLB) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_sc, (lds_void*)(smem + s * SF_SLOT + ha * SF_HALF + wave * 256), 4,
+                                                     vs[ha], 0, 0, 0);
+        } else if constexpr (kWide) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rs_sc2, (lds_void*)(smem + s * SF_SLOT + hb * SF_HALF + 2 * SF_A + (wave & 1) * 256), 4, vs2[hb], 0, 0, 0);
         } else if constexpr (!kBf16) {
             const int h = wave < 2 ? ha : hb;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rs_sc, (lds_void*)(smem + s * SF_SLOT + h * 4 * SF_AREA + wave * SF_AREA), 4,
-                ha == hb ? vs[ha] : wave < 2 ? vs[ha] : vs[hb], 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_sc, (lds_void*)(smem + s * SF_SLOT + h * SF_HALF + wave * 256), 4,
+                                                     ha == hb ? vs[ha] : wave < 2 ? vs[ha] : vs[hb], 0, 0, 0);
         }
     };
     auto issue_group = [&](int c, auto s_tag, auto ha_tag, auto hb_tag) {
@@ -370,33 +406,34 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
     constexpr int XA = AMN ? 1 : SA::PIECES, XB = BMN ? 1 : SB::PIECES;
     int addr_a[U * XA * (AMN ? NA0 : 1)], addr_b[U * XB * (BMN ? NB0 : 1)];
     const int s16 = lane & 15, g16 = lane >> 4;
-    auto mn_addr = [&](auto side, int half_row, int j, int u) -> int {
+    auto mn_addr = [&](auto side, int row, int u) -> int {   // (row: first row of the block within the half)
         // transposing reads (gemm_kernel.hpp, load_frag_mn): in each 16-lane group lane s addresses 8 bytes of
         // K row kb + s / 2 (bf16: kb + s / 4), and lane i receives consecutive K of MN row i
         using S = decltype(side);
         if constexpr (!kBf16) {
-            const int k = 16 * g16 + (s16 >> 1), pp = (half_row + 16 * j) >> 4;
+            const int k = 16 * g16 + (s16 >> 1), pp = row >> 4;
             return k * S::PITCH + ((pp ^ S::swizzle(k)) << 4) + (s16 & 1) * 8;
         } else {
-            const int k = u * 32 + 8 * q + (s16 >> 2), col = half_row + 32 * j + 16 * (g16 & 1) + 4 * (s16 & 3);
+            const int k = u * 32 + 8 * q + (s16 >> 2), col = row + 16 * (g16 & 1) + 4 * (s16 & 3);
             return k * S::PITCH + (((col >> 3) ^ S::swizzle(k)) << 4) + ((col >> 2) & 1) * 8;
         }
     };
-    // a wave's first row of half h (rows(h) / 2 per wave); K-major addresses are taken for half 0, and half
-    // 1's rows lie at a multiple of 32 rows from them (same swizzle), MN-major ones per half
-    auto km_addr = [&](auto side, int w, int h, int u, int x) -> int {
+    // Rows of a wave's block j: A blocks alternate between the two wave rows (a tile of few valid rows then has
+    // its live blocks spread over all waves), a wave's B columns are contiguous, rows(h) / 2 of them.  Blocks lie
+    // a multiple of 16 (bf16: 32) rows apart, so that a lane's swizzle is the same for all of them.
+    auto km_addr = [&](auto side, int first, int u, int x) -> int {
         using S = decltype(side);
-        const int row = w * (S::rows(h) / 2) + r;
+        const int row = first + r;
         int piece;
         if constexpr (kBf16) piece = u * 4 + 2 * x + q;
         else if constexpr (S::RB == 64) piece = q;
         else piece = 4 * x + q;
         return row * S::RB + ((piece ^ S::swizzle(row)) << 4);
     };
-    // (waves 1 of an uneven side start half 1 at another row than half 0: the difference in bytes)
-    constexpr bool kEvenA = SA::H0 == SA::H1, kEvenB = SB::H0 == SB::H1;
-    int addr_a1[kEvenA ? 1 : U * XA * (AMN ? NA0 : 1)], addr_b1[kEvenB ? 1 : U * XB * (BMN ? NB0 : 1)];
-    auto fill = [&](auto side, auto mn_tag, int w, int h, int off, auto& out, auto x_tag, auto nb_tag) {
+    // (the wave columns of an uneven B side start half 1 at another column than half 0)
+    constexpr bool kEvenB = SB::H0 == SB::H1;
+    int addr_b1[kEvenB ? 1 : U * XB * (BMN ? NB0 : 1)];
+    auto fill = [&](auto side, auto mn_tag, int first, int step, int off, auto& out, auto x_tag, auto nb_tag) {
         using S = decltype(side);
         constexpr bool mn = decltype(mn_tag)::value != 0;
         constexpr int X = decltype(x_tag)::value, NBX = decltype(nb_tag)::value;
@@ -404,26 +441,25 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
         for (int u = 0; u < U; ++u) {
             if constexpr (mn) {
 #pragma unroll
-                for (int j = 0; j < NBX; ++j) out[u * NBX + j] = off + mn_addr(S{}, w * (S::rows(h) / 2), j, u);
+                for (int j = 0; j < NBX; ++j) out[u * NBX + j] = off + mn_addr(S{}, first + j * step, u);
             } else {
 #pragma unroll
-                for (int x = 0; x < X; ++x) out[u * X + x] = off + km_addr(S{}, w, h, u, x);
+                for (int x = 0; x < X; ++x) out[u * X + x] = off + km_addr(S{}, first, u, x);
             }
         }
     };
-    fill(SA{}, Int<AMN>{}, wm, 0, A_OFF, addr_a, Int<XA>{}, Int<(AMN ? NA0 : 1)>{});
-    fill(SB{}, Int<BMN>{}, wn, 0, B_OFF, addr_b, Int<XB>{}, Int<(BMN ? NB0 : 1)>{});
-    if constexpr (!kEvenA) fill(SA{}, Int<AMN>{}, wm, 1, A_OFF, addr_a1, Int<XA>{}, Int<(AMN ? NA0 : 1)>{});
-    if constexpr (!kEvenB) fill(SB{}, Int<BMN>{}, wn, 1, B_OFF, addr_b1, Int<XB>{}, Int<(BMN ? NB0 : 1)>{});
+    fill(SA{}, Int<AMN>{}, wm * MR, 2 * MR, A_OFF, addr_a, Int<XA>{}, Int<(AMN ? NA0 : 1)>{});
+    fill(SB{}, Int<BMN>{}, wn * (SB::H0 / 2), MR, B_OFF, addr_b, Int<XB>{}, Int<(BMN ? NB0 : 1)>{});
+    if constexpr (!kEvenB) fill(SB{}, Int<BMN>{}, wn * (SB::H1 / 2), MR, B_OFF, addr_b1, Int<XB>{}, Int<(BMN ? NB0 : 1)>{});
     // scales: 16 bytes = the dwords (row pair) of the wave's blocks; the lane's byte after a shift
-    const int addr_sa = (((g16 >> 1) * 2) * SF_AREA / 2) + wm * 128 + (s16 >> 1) * 16;
-    const int addr_sb = 2 * SF_AREA + (((g16 >> 1) * 2) * SF_AREA / 2) + wn * 128 + (s16 >> 1) * 16;
+    const int addr_sa = (g16 >> 1) * SF_A + wm * (SF_A / 2) + (s16 >> 1) * (kWide ? 32 : 16);
+    const int addr_sb = 2 * SF_A + (g16 >> 1) * SF_B + wn * (SF_B / 2) + (s16 >> 1) * 16;
     const int sc_shift = ((s16 & 1) * 2 + (g16 & 1)) * 8;
 
     i32x4 fa[2][NA0][U][2], fb[2][NB0][U][2];        // [half][block][fragment][16 bytes]
     i32x2 ta[NA0][U][4], tb[NB0][U][4];              // MN-major: the 8-byte pieces of the half being read
     int sa[2][NA0], sb[2][NB0];                      // scales in the low byte
-    i32x4 sc_raw;
+    i32x4 sc_raw[2];                                 // (dwords of four blocks each)
     // 16-byte (MN-major: 8-byte) read X of block j, K step u
     auto read_frag = [&](auto a_tag, auto s_tag, auto h_tag, auto j_tag, auto u_tag, auto x_tag) {
         constexpr bool A = decltype(a_tag)::value != 0, mn = A ? AMN : BMN;
@@ -431,10 +467,10 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
         constexpr int u = decltype(u_tag)::value, x = decltype(x_tag)::value;
         using S = typename Cond<A, SA, SB>::type;
         constexpr int NBX = A ? NA0 : NB0, X = A ? XA : XB;
-        constexpr bool second = h == 1 && !(A ? kEvenA : kEvenB);
+        constexpr bool second = !A && h == 1 && !kEvenB;
         constexpr int idx = mn ? u * NBX + j : u * X + x;
         int base;
-        if constexpr (A) base = second ? addr_a1[second ? idx : 0] : addr_a[idx];
+        if constexpr (A) base = addr_a[idx];
         else base = second ? addr_b1[second ? idx : 0] : addr_b[idx];
         constexpr int at = s * S::SLOT + h * S::bytes(0);
         if constexpr (mn) {
@@ -445,16 +481,16 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
             else read_tr<kBf16, at + kb * S::PITCH>(tb[j][u][x], base);
         } else {
             i32x4 (&f)[2] = A ? fa[h][A ? j : 0][u] : fb[h][A ? 0 : j][u];
-            f[x] = *(lds_i32x4*)(lds + base + at + j * MR * S::RB);
+            f[x] = *(lds_i32x4*)(lds + base + at + j * (A ? 2 : 1) * MR * S::RB);
         }
     };
     // MN-major: the pieces of the half just read have arrived; the fragments take them over
-    auto finish_read = [&](auto a_tag, auto h_tag) {
+    auto finish_read = [&](auto a_tag, auto h_tag, auto n_tag) {
         constexpr bool A = decltype(a_tag)::value != 0;
         constexpr int h = decltype(h_tag)::value;
         if constexpr (A ? AMN : BMN) {
             wait_lds();
-            static_for<(A ? SA::nb(h) : SB::nb(h))>([&](auto j_c) {
+            static_for<decltype(n_tag)::value>([&](auto j_c) {
                 static_for<U>([&](auto u_c) {
                     constexpr int j = decltype(j_c)::value, u = decltype(u_c)::value;
                     i32x2 (&t)[4] = A ? ta[A ? j : 0][u] : tb[A ? 0 : j][u];
@@ -466,30 +502,35 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
             });
         }
     };
-    auto read_scales = [&](auto a_tag, auto s_tag, auto h_tag) {
+    auto read_scales = [&](auto a_tag, auto s_tag, auto h_tag, auto x_tag) {
         constexpr bool A = decltype(a_tag)::value != 0;
-        sc_raw = *(lds_i32x4*)(lds + (A ? addr_sa : addr_sb) + decltype(s_tag)::value * SF_SLOT + decltype(h_tag)::value * 4 * SF_AREA);
+        constexpr int x = decltype(x_tag)::value;
+        sc_raw[x] = *(lds_i32x4*)(lds + (A ? addr_sa : addr_sb) + decltype(s_tag)::value * SF_SLOT + decltype(h_tag)::value * SF_HALF + 16 * x);
     };
-    auto shift_scales = [&](auto a_tag, auto h_tag) {
+    auto shift_scales = [&](auto a_tag, auto h_tag, auto n_tag) {
         constexpr bool A = decltype(a_tag)::value != 0;
         constexpr int h = decltype(h_tag)::value;
-        static_for<(A ? SA::nb(h) : SB::nb(h))>([&](auto j_c) {
+        static_for<decltype(n_tag)::value>([&](auto j_c) {
             constexpr int j = decltype(j_c)::value;
-            const int v = (int)((uint32_t)sc_raw[j] >> sc_shift);
+            const int v = (int)((uint32_t)sc_raw[j / 4][j % 4] >> sc_shift);
             if constexpr (A) sa[h][j] = v; else sb[h][j] = v;
         });
     };
 
     typedef typename Cond<kBf16, f32x16, f32x4>::type acc_t;
-    // (256 x 256 tiles would fill the AGPRs to the last one, and the allocator then moves a block in and out of
-    // them in the loop: the last 16-row blocks, or the last 32-row block, live in VGPRs, of which there are enough)
+    // (Tiles of 256 accumulators a lane or more would fill the 256 AGPRs to the last one, and the allocator then
+    // moves a block in and out of them in the loop: what passes 248 (384-row tiles: 252), the last blocks, lives in
+    // VGPRs.)
+    auto nb_a = [](int h) constexpr { return h ? LIVE : SA::NB0; };   // live blocks of A half h
+    constexpr int kAccRegs = kBf16 ? 16 : 4, kOver = (SA::NB0 + LIVE) * (SB::NB0 + SB::NB1) * kAccRegs - (kWide ? 252 : 248);
+    constexpr int kInV = kOver > 0 ? (kOver + kAccRegs - 1) / kAccRegs : 0;
     auto in_v = [](int ha, int hb, int i, int j) constexpr {
-        return BM * BN == 256 * 256 && ha == 1 && hb == 1 && i == NA0 - 1 && j >= (kBf16 ? 1 : 2);
+        return ha == 1 && hb == 1 && (LIVE - 1 - i) * SB::NB1 + SB::NB1 - 1 - j < kInV;
     };
     acc_t acc[2][2][NA0][NB0];                        // [A half][B half]
     static_for<4>([&](auto h_c) {
         constexpr int ha = decltype(h_c)::value >> 1, hb = decltype(h_c)::value & 1;
-        static_for<SA::nb(ha)>([&](auto i) {
+        static_for<nb_a(ha)>([&](auto i) {
             static_for<SB::nb(hb)>([&](auto j) {
                 acc_t& d = acc[ha][hb][decltype(i)::value][decltype(j)::value];
                 d = acc_t{};
@@ -517,27 +558,31 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
     auto phase = [&](auto p_tag, auto s_tag, int c) {
         constexpr int P = decltype(p_tag)::value, s = decltype(s_tag)::value, f = s;
         constexpr int ha = P >= 2, hb = P == 0 || P == 3 ? f : 1 - f;
-        constexpr int NA = SA::nb(ha), NB = SB::nb(hb), NM = NA * NB * KSTEPS;
+        constexpr int NA = nb_a(ha), NB = SB::nb(hb), NM = NA * NB * KSTEPS;
+        constexpr int NS = NM < 4 ? 6 : NM;           // slots: the first NM hold an MFMA
         // the half read in this phase: B1-f, A1, the next stage's A0, its first B half (1 - f)
         constexpr bool kReadA = P == 1 || P == 2;
         constexpr int rslot = P >= 2 ? s ^ 1 : s, rh = P == 1 ? 1 : P == 2 ? 0 : 1 - f;
-        constexpr int RN = kReadA ? SA::nb(rh) : SB::nb(rh), RX = kReadA ? SA::PIECES : SB::PIECES;
-        constexpr int NR = RN * RX * U + NSF;
+        constexpr int RN = kReadA ? nb_a(rh) : SB::nb(rh), RX = kReadA ? SA::PIECES : SB::PIECES;
+        constexpr int NSR = kBf16 || RN == 0 ? 0 : kReadA && RN > 4 ? 2 : 1;   // reads of scales
+        constexpr int NR = RN * RX * U + NSR;
         // the half stage refilled: {A0, Bf} in phases 0 and 1, {A1, B1-f} in phases 2 and 3
         constexpr int lha = P >= 2, lhb = P >= 2 ? 1 - f : f;
         constexpr int NL = SA::loads(lha) + SB::loads(lhb) + NSF;
         constexpr int L0 = (P & 1) ? (NL + 1) / 2 : 0, L1 = (P & 1) ? NL : (NL + 1) / 2;
         constexpr int first = (P & 1) == 0 ? 1 : 0;   // (slot 0 of phases 0 and 2 holds the barrier)
-        constexpr int kShift = NM >= 4 ? NM - 3 : 0;
+        constexpr int kShift = NS - 3;
         // loads that may stay in flight at the barrier: the two half-stages issued last
         constexpr int kFlight = P == 0 ? SA::loads(0) + SB::loads(1 - f) + SA::loads(1) + SB::loads(f) + 2 * NSF
                                        : SA::loads(1) + SB::loads(f) + SA::loads(0) + SB::loads(f) + 2 * NSF;
-        static_for<NM>([&](auto i_c) {
+        static_for<NS>([&](auto i_c) {
             constexpr int i = decltype(i_c)::value;
-            constexpr int u = i / (NA * NB), blk = i % (NA * NB);
-            // (the operand half read last is the outer loop: its first blocks arrived first)
-            if constexpr (P < 2) mfma(Int<ha>{}, Int<hb>{}, Int<blk % NA>{}, Int<blk / NA>{}, Int<u>{});
-            else mfma(Int<ha>{}, Int<hb>{}, Int<blk / NB>{}, Int<blk % NB>{}, Int<u>{});
+            if constexpr (i < NM) {
+                constexpr int u = i / (NA * NB), blk = i % (NA * NB);
+                // (the operand half read last is the outer loop: its first blocks arrived first)
+                if constexpr (P < 2) mfma(Int<ha>{}, Int<hb>{}, Int<blk % NA>{}, Int<blk / NA>{}, Int<u>{});
+                else mfma(Int<ha>{}, Int<hb>{}, Int<blk / NB>{}, Int<blk % NB>{}, Int<u>{});
+            }
             if constexpr ((P & 1) == 0 && i == 0) {
                 // what the next two phases read has landed and what they refill has been read by every wave
                 // (this MFMA covers part of the wait)
@@ -548,27 +593,27 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
             static_for<NR>([&](auto b_c) {
                 constexpr int b = decltype(b_c)::value;
                 // (MN-major: the last quarter of the phase is left for the reads to arrive in)
-                constexpr int window = (kReadA ? AMN : BMN) ? (NM - first) * 3 / 4 : NM - first;
+                constexpr int window = (kReadA ? AMN : BMN) ? (NS - first) * 3 / 4 : NS - first;
                 constexpr int at = NR <= window ? first + b : first + b * window / NR;
                 if constexpr (at == i) {
-                    if constexpr (b < NSF) {
-                        read_scales(Int<kReadA>{}, Int<rslot>{}, Int<rh>{});
+                    if constexpr (b < NSR) {
+                        read_scales(Int<kReadA>{}, Int<rslot>{}, Int<rh>{}, Int<b>{});
                     } else {
-                        constexpr int x = b - NSF, blkx = x / RX;
+                        constexpr int x = b - NSR, blkx = x / RX;
                         read_frag(Int<kReadA>{}, Int<rslot>{}, Int<rh>{}, Int<blkx % RN>{}, Int<blkx / RN>{}, Int<x % RX>{});
                     }
                 }
             });
-            if constexpr (!kBf16 && i == kShift) shift_scales(Int<kReadA>{}, Int<rh>{});
+            if constexpr (NSR > 0 && i == kShift) shift_scales(Int<kReadA>{}, Int<rh>{}, Int<RN>{});
             static_for<L1 - L0>([&](auto l_c) {
                 constexpr int l = decltype(l_c)::value;
-                constexpr int at = first + l * (NM - first) / (L1 - L0);
+                constexpr int at = first + l * (NS - first) / (L1 - L0);
                 if constexpr (at == i) issue(Int<L0 + l>{}, s_tag, Int<lha>{}, Int<lhb>{});
             });
-            if constexpr (P == 3 && i == NM - 1) set_stage(c + 3);
+            if constexpr (P == 3 && i == NS - 1) set_stage(c + 3);
             __builtin_amdgcn_sched_barrier(0);
         });
-        finish_read(Int<kReadA>{}, Int<rh>{});
+        finish_read(Int<kReadA>{}, Int<rh>{}, Int<RN>{});
     };
     auto stage = [&](int c, auto s_tag) {
         phase(Int<0>{}, s_tag, c);
@@ -585,15 +630,16 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
     static_for<2>([&](auto a_c) {
         constexpr bool A = decltype(a_c)::value == 0;
         if constexpr (!kBf16) {
-            read_scales(Int<A>{}, Int<0>{}, Int<0>{});
-            shift_scales(Int<A>{}, Int<0>{});
+            read_scales(Int<A>{}, Int<0>{}, Int<0>{}, Int<0>{});
+            if constexpr (A && kWide) read_scales(Int<A>{}, Int<0>{}, Int<0>{}, Int<1>{});
+            shift_scales(Int<A>{}, Int<0>{}, Int<(A ? NA0 : NB0)>{});
         }
         static_for<U>([&](auto u) {
             static_for<(A ? NA0 : NB0)>([&](auto j) {
                 static_for<(A ? SA::PIECES : SB::PIECES)>([&](auto x) { read_frag(Int<A>{}, Int<0>{}, Int<0>{}, j, u, x); });
             });
         });
-        finish_read(Int<A>{}, Int<0>{});
+        finish_read(Int<A>{}, Int<0>{}, Int<(A ? NA0 : NB0)>{});
     });
     set_stage(2);
     __builtin_amdgcn_sched_barrier(0);
@@ -611,7 +657,9 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
     // tile out of the AGPRs ahead of the epilogue's branches.
     auto take = [&](auto ha_c, auto hb_c, auto i_c, auto j_c) -> acc_t {
         acc_t& t = acc[decltype(ha_c)::value][decltype(hb_c)::value][decltype(i_c)::value][decltype(j_c)::value];
-        if constexpr (in_v(decltype(ha_c)::value, decltype(hb_c)::value, decltype(i_c)::value, decltype(j_c)::value))
+        if constexpr (decltype(i_c)::value >= nb_a(decltype(ha_c)::value))
+            t = acc_t{};
+        else if constexpr (in_v(decltype(ha_c)::value, decltype(hb_c)::value, decltype(i_c)::value, decltype(j_c)::value))
             asm volatile("" : "+v"(t));
         else
             asm volatile("" : "+a"(t));
@@ -621,7 +669,7 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
     // ------------------------------------------------------------------ epilogue
     auto row_of = [&](auto ha_c, auto i_c, int w, int rr) -> int {
         constexpr int ha = decltype(ha_c)::value;
-        return m0 + ha * SA::H0 + w * (SA::rows(ha) / 2) + decltype(i_c)::value * MR + rr;
+        return m0 + ha * SA::H0 + decltype(i_c)::value * 2 * MR + w * MR + rr;
     };
     auto row_state = [&](int m, bool& row_ok, bool& pad_row) {
         row_ok = m < tl.tile_end && !(gemm_type == kMasked && m >= tl.valid_end);
@@ -789,7 +837,7 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
         constexpr int ha = decltype(ha_c)::value;
         static_for<SA::nb(ha)>([&](auto i_c) {
             // the block row of both wave rows, fp32: [2 MR][BN]
-            static_assert(2 * MR * BN * 4 <= LDS_BYTES, "staging area");
+            static_assert(2 * MR * BN * 4 <= T::LDS_BYTES, "staging area");
             float* const st = reinterpret_cast<float*>(smem);
             __syncthreads();
             static_for<2>([&](auto hb_c) {
@@ -818,6 +866,30 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
             }
         });
     });
+    }
+}
+
+// CT / CS / CM / CN / CK: GEMM type, K split and sizes fixed at compile time (-1 / 0: from the arguments).
+template <int BM, int BN, int KIND, int EPI, int CT = -1, int CS = 0, int CM = 0, int CN = 0, int CK = 0,
+          bool AMN = false, bool BMN = false>
+__device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
+    using T = QuadTile<BM, BN, KIND, AMN, BMN>;
+    using SA = typename T::SA;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[T::LDS_BYTES];
+    TileLoc tl;
+    if (!locate_tile<BM, BN, 256, KIND, CT, CS, CM, CN, CK, AMN, BMN>(p, vb, -1, threadIdx.x, tl)) return;
+    auto run = [&](auto live) {
+        quad_tile_body<BM, BN, KIND, EPI, CT, CS, CM, CN, CK, AMN, BMN, decltype(live)::value>(p, tl, smem);
+    };
+    if constexpr (T::kWide) {
+        // anchored tiles end with their group: of 8192 rows routed to 32 groups, 180 to 333 each, a quarter of
+        // the tiles' blocks are dead (N=4096 K=7168: 309 us with every block, 303 without the dead ones)
+        const int live = ceil_div(tl.valid_end - tl.m0 - SA::H0, 2 * SA::MR);
+        if (!tl.anchored || live > 4) run(Int<SA::NB1>{});
+        else if (live > 2) run(Int<4>{});
+        else run(Int<2>{});
+    } else {
+        run(Int<SA::NB1>{});
     }
 }
 

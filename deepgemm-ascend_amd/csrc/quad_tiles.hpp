@@ -13,7 +13,7 @@ KernelFn pick_quad_epi(int epi) {
         case kEpiBf16: return &quad_kernel<BM, BN, KIND, kEpiBf16, AMN, BMN>;
         case kEpiBf16SR: return &quad_kernel<BM, BN, KIND, kEpiBf16SR, AMN, BMN>;
         case kEpiFp8:
-            if constexpr (KIND == kFP8FP8 && quad_fp8_output(BN)) return &quad_kernel<BM, BN, KIND, kEpiFp8, AMN, BMN>;
+            if constexpr (KIND == kFP8FP8 && quad_fp8_output(BM, BN)) return &quad_kernel<BM, BN, KIND, kEpiFp8, AMN, BMN>;
             else return nullptr;
         default: return nullptr;
     }
@@ -25,7 +25,7 @@ KernelFn find_quad(int bm, int bn, int epi) {
         return nullptr;
     } else {
         constexpr TileCfg t = kTiles[I];
-        if constexpr (quad_tile(KIND, t.bm, t.bn)) {
+        if constexpr (quad_tile(KIND, t.bm, t.bn) && (t.bm <= 256 || (!AMN && !BMN))) {
             if (bm == t.bm && bn == t.bn) return pick_quad_epi<t.bm, t.bn, KIND, AMN, BMN>(epi);
         }
         return find_quad<KIND, AMN, BMN, I + 1>(bm, bn, epi);

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import deep_gemm
-from oracle import gemm as og
+from oracle import gemm as og, layout as ol
 from helpers import gen, operand, calc_diff
 
 pytestmark = pytest.mark.gpu
@@ -137,3 +137,33 @@ def test_quad_split(force, tile, split, m, n, k):
         _check(d, og.gemm_nt(a_deq, b_deq, dt))
         out[dt] = d
     assert torch.equal(out[torch.bfloat16], out[torch.float32].bfloat16())
+
+
+@pytest.mark.parametrize('b_kind', ['e4m3', 'e2m1'])
+def test_quad_anchored_live_blocks(b_kind):
+    """384-row tiles of an M-grouped layout, whose loop leaves out the dead blocks of the second 192 rows: groups
+    that end one short of, at and one past each count of live blocks; the default plan of alignment 32."""
+    sizes = [1, 31, 192, 193, 223, 224, 225, 256, 257, 288, 289, 320, 321, 352, 353, 383, 384, 385, 0, 577]
+    alignment, n, k = 32, 200, 416
+    print(f'quad anchored {b_kind} sizes={sizes}', flush=True)
+    total, ps = ol.psum_from_sizes(sizes, alignment)
+    g = gen(9)
+    a, sfa, a_deq = operand(total, k, 'e4m3', (1, 32), g)
+    b, sfb, b_deq = operand(n, k, b_kind, (1, 32), g, batch=len(sizes))
+    layout = torch.tensor(ps, dtype=torch.int32)
+    old = deep_gemm.get_mk_alignment_for_contiguous_layout()
+    deep_gemm.set_mk_alignment_for_contiguous_layout(alignment)
+    try:
+        d = torch.full((total, n), float('nan'), dtype=torch.bfloat16, device='cuda')
+        fn = deep_gemm.m_grouped_fp8_gemm_nt_contiguous if b_kind == 'e4m3' else deep_gemm.m_grouped_fp8_fp4_gemm_nt_contiguous
+        fn((a.cuda(), sfa.cuda()), (b.cuda(), sfb.cuda()), d, layout.cuda())
+    finally:
+        deep_gemm.set_mk_alignment_for_contiguous_layout(old)
+    out, ref = d.cpu(), og.m_grouped_contiguous(a_deq, b_deq, layout, True, alignment)
+    end = 0
+    for size, stop in zip(sizes, ps):
+        start, end = end, -(-stop // alignment) * alignment
+        assert stop == start + size
+        if size:
+            _check(out[start:stop], ref[start:stop])
+        assert torch.equal(out[stop:end], torch.zeros_like(out[stop:end]))
