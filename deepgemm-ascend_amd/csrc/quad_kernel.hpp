@@ -262,7 +262,7 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
     const int gemm_type = CT >= 0 ? CT : p.gemm_type;
     const int M = CM > 0 ? CM : p.m, N = CN > 0 ? CN : p.n;
     const int m0 = tl.m0, n0 = tl.n0, k_len = tl.k_len;
-    const int rows_a = tl.anchored ? min(BM, tl.valid_end - m0) : min(BM, M - m0), rows_b = min(BN, N - n0);
+    const int rows_a = min(BM, tl.valid_end - m0), rows_b = min(BN, N - n0);
     // K stages of this workgroup: [c0, c0 + num_stages) of the whole K loop
     const int split_k = CS > 0 ? CS : p.split_k;
     const int all_stages = ceil_div(k_len, KS), nk64 = ceil_div(k_len, 64);

@@ -167,3 +167,26 @@ def test_quad_anchored_live_blocks(b_kind):
         if size:
             _check(out[start:stop], ref[start:stop])
         assert torch.equal(out[stop:end], torch.zeros_like(out[stop:end]))
+
+
+@pytest.mark.parametrize('tile', ['256x256', '256x128', '128x128'])
+def test_quad_masked_order(force, tile):
+    """Several tile rows per group: every live tile is served once and dead rows stay as they were, for more
+    groups than a wave has lanes, groups without rows and counts at the tiles' edges."""
+    g_num, max_m, n, k = 70, 520, 264, 160
+    print(f'quad masked {tile}', flush=True)
+    force(tile)
+    g = gen(10)
+    masked = torch.randint(0, 40, (g_num,), generator=g, dtype=torch.int32)
+    masked[:12] = torch.tensor([520, 0, 0, 1, 127, 128, 129, 256, 257, 384, 385, 512], dtype=torch.int32)
+    masked[64:67] = torch.tensor([0, 300, 520], dtype=torch.int32)
+    a, sfa, a_deq = operand(max_m, k, 'e4m3', (1, 32), g, batch=g_num)
+    b, sfb, b_deq = operand(n, k, 'e4m3', (1, 32), g, batch=g_num)
+    d = torch.full((g_num, max_m, n), float('nan'), dtype=torch.bfloat16, device='cuda')
+    deep_gemm.m_grouped_fp8_gemm_nt_masked((a.cuda(), sfa.cuda()), (b.cuda(), sfb.cuda()), d, masked.cuda(), 64)
+    out, ref = d.cpu(), og.m_grouped_masked(a_deq, b_deq, masked)
+    for i in range(g_num):
+        rows = int(masked[i])
+        assert torch.isnan(out[i, rows:].float()).all(), i
+        if rows:
+            assert calc_diff(out[i, :rows], ref[i, :rows]) < THRESH, i
