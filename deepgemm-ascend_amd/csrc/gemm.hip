@@ -940,6 +940,13 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
     static const int group_m_env = std::getenv("DG_GROUP_M") ? std::atoi(std::getenv("DG_GROUP_M")) : 0;   // tuning
     p.group_m = group_m_env > 0 ? group_m_env : 4;
     const int groups = (a.gemm_type == kBatched || a.gemm_type == kMasked || a.gemm_type == kKGrouped) ? a.num_groups : 1;
+    // A D that the last-level cache (256 MB) cannot hold beside the operands is stored past it, where the stores
+    // are a large part of the work (short K); e4m3 A, us, through the caches and past them: 32768x4096x2048 252 and
+    // 236, 24576x4096x2048 189 and 180, 20480x4096x2048 154 and 154, 12288x4096x2048 91 and 97, 32768x7168x1024
+    // 287 and 267, 8192x24576x1536 327 and 295; K = 7168 (32768x4096) 686 and 693.  bf16 operands lose: their two
+    // 16-byte stores a row fill 32 bytes of a line each (16384x4096x2048 219 and 248).
+    p.stream_d = a.kind != kBF16 && a.gemm_type != kMasked && a.k <= 4096 &&
+                 2 * (int64_t)a.m * a.n * groups >= 192LL << 20;
     int64_t tiles = plan.skinny_rows ? rows_tiles(a, cfg) : (int64_t)p.num_m_blocks * p.num_n_blocks * groups;
     if (tiles <= 0) return DG_OK;
     // split-K grids are padded to whole groups of 8 tiles (one per XCD); persistent grids hold

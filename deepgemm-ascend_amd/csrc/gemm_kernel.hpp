@@ -75,6 +75,7 @@ struct KParams {
     // workgroup b of a launch serves plan workgroup vbase + b.
     int vgrid, vbase;
     int reduce_bm, reduce_bn;   // quad_reduce_kernel: the tile the partials belong to
+    int stream_d;               // the four-wave kernel's bf16 D goes past the caches (16-byte stores)
 };
 
 // Epilogue variants.

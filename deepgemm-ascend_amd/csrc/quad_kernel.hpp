@@ -817,9 +817,12 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
                                 constexpr int j = 2 * decltype(j_c)::value, t = t0 + j;
                                 const auto s0 = __builtin_amdgcn_permlane16_swap(pk[t][0], pk[t + 1][0], false, false);
                                 const auto s1 = __builtin_amdgcn_permlane16_swap(pk[t][1], pk[t + 1][1], false, false);
-                                if (row_ok && n0 + cb + 16 * j + 16 * (q & 1) < N)
-                                    *reinterpret_cast<i32x4*>(drow + (cb + 16 * j + 16 * (q & 1) + 8 * (q >> 1)) * 2) =
-                                        i32x4{(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
+                                if (row_ok && n0 + cb + 16 * j + 16 * (q & 1) < N) {
+                                    i32x4* const d = reinterpret_cast<i32x4*>(drow + (cb + 16 * j + 16 * (q & 1) + 8 * (q >> 1)) * 2);
+                                    const i32x4 w = {(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
+                                    if (p.stream_d) __builtin_nontemporal_store(w, d);
+                                    else *d = w;
+                                }
                             });
                             if constexpr (SB::nb(hb) % 2 != 0) {
                                 constexpr int j = SB::nb(hb) - 1;
@@ -882,8 +885,8 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
         quad_tile_body<BM, BN, KIND, EPI, CT, CS, CM, CN, CK, AMN, BMN, decltype(live)::value>(p, tl, smem);
     };
     if constexpr (T::kWide) {
-        // anchored tiles end with their group: of 8192 rows routed to 32 groups, 180 to 333 each, a quarter of
-        // the tiles' blocks are dead (N=4096 K=7168: 309 us with every block, 303 without the dead ones)
+        // anchored tiles end with their group: of 8192 rows routed to 32 groups, 180 to 333 each, a third of
+        // the tiles' blocks is dead (N=4096 K=7168: 309 us with every block, 303 without the dead ones)
         const int live = ceil_div(tl.valid_end - tl.m0 - SA::H0, 2 * SA::MR);
         if (!tl.anchored || live > 4) run(Int<SA::NB1>{});
         else if (live > 2) run(Int<4>{});
