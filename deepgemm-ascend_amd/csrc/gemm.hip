@@ -5,8 +5,9 @@
 // bf16_gemm.hpp:16-78) and its select_gemm_config cost model
 // (csrc/jit_kernels/heuristics.hpp:592-755).  Kernels are compiled ahead of time for a
 // fixed menu of tile shapes; the heuristic scores each shape with a gfx950 model
-// (256 CUs, waves-of-tiles quantisation, measured cycles per K stage of each tile shape and a
-// fixed per-tile cost) and memoises the choice per problem signature.
+// (256 CUs, waves-of-tiles quantisation; the four-wave tiles by costs fitted to measurements,
+// quad_time, the others by cycles per K stage and a fixed per-tile cost) and memoises the choice
+// per problem signature.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -488,7 +489,8 @@ Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
     if (skinny_plan(a, cus, allow_split, skinny)) return skinny;
     // M-grouped layouts whose alignment rules out 256-row tiles take 384x192 tiles anchored at each
     // group's (m_indices: each run's) first row: a group of up to 384 rows streams its weights once instead of once
-    // per 128-row block.  Measured (G = 32 routed top-8 counts, ~257 rows a group, alignment 128,
+    // per 128-row block.  Measured on the eight-wave kernel (the four-wave one took N=4096 K=7168 on to 293
+    // beside its scale transform; G = 32 routed top-8 counts, ~257 rows a group, alignment 128,
     // cold us): N=4096 K=7168 345.6 vs 458.7 (128x256), N=7168 K=2048 200.3 vs 237.9; bf16
     // 635.6 vs 839.9 and 330.2 vs 408.5.  With alignment 256 the 256-row tiles are faster (443 vs
     // 526 at N=4096 K=7168).

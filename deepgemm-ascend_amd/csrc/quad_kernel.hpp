@@ -5,8 +5,8 @@
 //   (A0, Bf) (A0, B1-f) (A1, B1-f) (A1, Bf),   f = stage parity,
 // so that consecutive phases share one operand half and every phase needs only one new half in registers:
 // phase 0 reads B1-f, phase 1 A1, phase 2 the next stage's A0 and phase 3 its first B half (B1-f, whose
-// registers the phase before has finished with).  A wave owns rows [64 w, +64) of a 128-row half and reads
-// each of its fragments from LDS exactly once per stage.
+// registers the phase before has finished with).  A wave owns every other 16-row (bf16: 32-row) block of an A
+// half and half the columns of a B half, and reads each of its fragments from LDS exactly once per stage.
 //
 // LDS holds two stages.  Each half of a slot is refilled (buffer_load ... lds, stage c + 2) as soon as every
 // wave has read it: A0 and Bf during phases 0-1, A1 and B1-f during phases 2-3, so a load has 1 to 1.5 stages
