@@ -569,7 +569,7 @@ struct MemoHash {
 std::mutex g_memo_mu;
 std::unordered_map<MemoKey, Plan, MemoHash> g_memo;
 
-Plan choose(const dg_gemm_args& a, int cus, bool allow_split) {
+Plan choose_plan(const dg_gemm_args& a, int cus, bool allow_split) {
     allow_split = allow_split && split_capable(a);
     if (a.block_m > 0 && a.block_n > 0) {
         TileCfg t = {a.block_m, a.block_n, 0, 0, 0, 0, 0, 0, 0};
@@ -614,6 +614,19 @@ Plan choose(const dg_gemm_args& a, int cus, bool allow_split) {
         const int sps = ceil_div(ns, std::min(a.split_k, std::max(1, ns)));
         pl.split = ceil_div(ns, sps);
         pl.split_stages = sps;
+    }
+    return pl;
+}
+
+// The plan of a call, with the tile that it is launched on: the workspace is sized for that tile's partials.
+Plan choose(const dg_gemm_args& a, int cus, bool allow_split) {
+    Plan pl = choose_plan(a, cus, allow_split);
+    if (a.d_dtype == DG_DTYPE_FP8_E4M3 && pl.skinny_nw == 0 && quad_tile(a.kind, pl.tile.bm, pl.tile.bn) &&
+        !quad_fp8_output(pl.tile.bm, pl.tile.bn)) {
+        // FP8 output needs whole 32-column groups per wave: the 256-column tile over the same K ranges, whose sums
+        // are the same
+        for (const TileCfg& t : kTiles)
+            if (t.bm == 256 && t.bn == 256) pl.tile = t;
     }
     return pl;
 }
@@ -812,12 +825,6 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
     } else if (plan.split > 1 && plan_workspace(a, plan) > a.workspace_bytes) {
         if (a.split_k > 1) return dg_set_error("dg_gemm: workspace smaller than dg_gemm_workspace_size() reports");
         plan = choose(a, cus, false);
-    }
-    if (a.d_dtype == DG_DTYPE_FP8_E4M3 && plan.skinny_nw == 0 && quad_tile(a.kind, plan.tile.bm, plan.tile.bn) &&
-        !quad_fp8_output(plan.tile.bm, plan.tile.bn)) {
-        // FP8 output needs whole 32-column groups per wave: the 256-column tile, whose sums are the same
-        for (const TileCfg& t : kTiles)
-            if (t.bm == 256 && t.bn == 256) plan.tile = t;
     }
     const TileCfg cfg = plan.tile;
     if (cfg.bm == 0) return dg_set_error("dg_gemm: no tile shape fits this problem");

@@ -228,6 +228,23 @@ def test_workspace_size_of_decode_plans(lib):
     assert ws == 64 * 1024 + 64 * 4 * 128 * 64 * 4
 
 
+@pytest.mark.parametrize('m, n, k', [(300, 5760, 16384), (400, 4480, 16384), (400, 6528, 16384)])
+def test_workspace_size_of_fp8_output(lib, m, n, k):
+    """FP8 output runs the tile that dg_gemm_workspace_size reports for it: the partials of every K range fit,
+    also where bf16 output takes a 256x224 or 256x160 tile that covers fewer columns."""
+    args = _plan_args(m, n, k, 256)
+    args.d_dtype = _lib.DG_DTYPE_FP8_E4M3
+    args.sfd, args.sfd_ld, args.alpha = 16, m + m % 2, 1.0
+    nbytes = ctypes.c_int64(0)
+    assert lib.dg_gemm_workspace_size(ctypes.byref(args), ctypes.byref(nbytes)) == 0, lib.dg_last_error()
+    info = _lib.LaunchInfo()
+    args.library_workspace = 1
+    assert lib.dg_launch_plan(args, ctypes.byref(info)) == 0, lib.dg_last_error()
+    tiles = -(-m // info.block_m) * -(-n // info.block_n)
+    assert info.split_k > 1 and (info.block_m, info.block_n) == (256, 256)
+    assert nbytes.value >= 64 * 1024 + tiles * info.split_k * info.block_m * info.block_n * 4
+
+
 def test_error_words_and_stream_workspace_without_device(lib):
     # no kernel has run: nothing pending; the workspace query rejects null outputs
     assert lib.dg_take_errors() == 0
