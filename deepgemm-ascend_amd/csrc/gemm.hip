@@ -703,6 +703,12 @@ std::mutex g_stream_ws_mu;
 // Slot 0 holds the split-K workspace, slot 1 the run table of an anchored m_indices GEMM.
 std::map<std::tuple<int, hipStream_t, int>, StreamWorkspace> g_stream_ws;
 
+bool stream_capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
+    return cs != hipStreamCaptureStatusNone;
+}
+
 int stream_workspace(hipStream_t st, int64_t need, void** out, int slot = 0) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return dg_set_error("dg_gemm: no current HIP device");
@@ -712,9 +718,7 @@ int stream_workspace(hipStream_t st, int64_t need, void** out, int slot = 0) {
         *out = w.ptr;
         return DG_OK;
     }
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
-    if (cs != hipStreamCaptureStatusNone) {
+    if (stream_capturing(st)) {
         char buf[256];
         snprintf(buf, sizeof(buf), "dg_gemm: this call needs a %lld-byte workspace but the stream's is %lld "
                  "bytes, and it cannot grow while the stream is being captured: run the same call once before "
@@ -733,6 +737,13 @@ int stream_workspace(hipStream_t st, int64_t need, void** out, int slot = 0) {
     w.bytes = bytes;
     *out = p;
     return DG_OK;
+}
+
+// A call whose launches hand data on through a stream's buffer (partials to their reduction, the run table to its
+// tiles) keeps those launches together on the stream: another thread's call on it comes before or after.
+std::mutex g_stream_order_mu[16];
+std::unique_lock<std::mutex> stream_order(hipStream_t st) {
+    return std::unique_lock<std::mutex>(g_stream_order_mu[(reinterpret_cast<uintptr_t>(st) >> 6) % 16]);
 }
 
 // Checks, plans and launches one GEMM; with `info` it stops short of the launch and describes it.
@@ -813,13 +824,24 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
     const bool lib_ws = a.workspace == nullptr && a.library_workspace != 0;
     Plan plan = choose(a, cus, a.workspace != nullptr || lib_ws);
     void* workspace = a.workspace;
+    std::unique_lock<std::mutex> order;   // (held to the last launch)
     if (plan.split > 1 && lib_ws) {
         if (!plan_only && !compile_only) {
-            const int rc = stream_workspace(reinterpret_cast<hipStream_t>(stream), plan_workspace(a, plan), &workspace);
-            if (rc != DG_OK) {
-                // (a tile plan also runs unsplit: a call captured before its workspace exists does not need one)
-                if (plan.skinny_nw > 0 || a.split_k > 1) return rc;
+            const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+            // A tile plan also runs unsplit.  So it does in a graph, which may be replayed on any stream, beside
+            // others of its capture stream: none of them then writes the stream's partials.
+            const bool unsplit_too = plan.skinny_nw == 0 && a.split_k <= 1;
+            if (unsplit_too && stream_capturing(st)) {
                 plan = choose(a, cus, false);
+            } else {
+                order = stream_order(st);
+                const int rc = stream_workspace(st, plan_workspace(a, plan), &workspace);
+                if (rc != DG_OK) {
+                    if (!unsplit_too) return rc;
+                    (void)hipGetLastError();
+                    order.unlock();
+                    plan = choose(a, cus, false);
+                }
             }
         }
     } else if (plan.split > 1 && plan_workspace(a, plan) > a.workspace_bytes) {
@@ -1066,6 +1088,7 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
                     return dg_set_error("dg_gemm_noalloc: m_indices run table exceeds the scratch");
                 runs = reinterpret_cast<uint8_t*>(a.workspace) + kCounterBytes;
             } else {
+                order = stream_order(st);
                 rc = stream_workspace(st, need, &runs, 1);
                 if (rc != DG_OK) return rc;
             }

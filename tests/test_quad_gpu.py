@@ -4,6 +4,8 @@ a block; every operand layout; D rows that take the vector path, that need eleme
 K ranges summed by the second launch.  Against the CPU oracle (dequantise, fp32 matmul).  The bound on
 calc_diff is the repository's 1e-5; every element is also held to 1e-3 of itself or the root mean square (the
 alignment of e4m3 products inside one MFMA leaves up to 1.4e-4 of it), plus one unit of a bf16 result."""
+import threading
+
 import pytest
 import torch
 
@@ -190,3 +192,67 @@ def test_quad_masked_order(force, tile):
         assert torch.isnan(out[i, rows:].float()).all(), i
         if rows:
             assert calc_diff(out[i, :rows], ref[i, :rows]) < THRESH, i
+
+
+def _split_call(seed, m=300, n=2112, k=7168):
+    """A call whose default plan splits K on the four-wave tiles, and its eager result."""
+    plan = deep_gemm.launch_plan(m, n, k)
+    assert plan['split_k'] > 1 and plan['block_m'] >= 128, plan
+    a, b, a_deq, b_deq = _fp8(m, n, k, seed)
+    a = (a[0], deep_gemm.transform_sf_into_required_layout(a[1], m, k, (1, 32), is_sfa=True))
+    b = (b[0], deep_gemm.transform_sf_into_required_layout(b[1], n, k, (1, 32), is_sfa=False))
+    d = torch.empty(m, n, dtype=torch.float32, device='cuda')
+    deep_gemm.fp8_gemm_nt(a, b, d)
+    _check(d, og.gemm_nt(a_deq, b_deq, torch.float32))
+    return a, b, d.clone()
+
+
+def test_quad_split_captured_unsplit():
+    """A graph of a call that splits K when run eagerly, replayed beside eager calls of its capture stream: the
+    graph holds one unsplit launch, so neither side touches the other's partials."""
+    print('quad split captured', flush=True)
+    (a, b, ref), (a2, b2, ref2) = _split_call(21), _split_call(22)
+    s, t = torch.cuda.Stream(), torch.cuda.Stream()
+    d, d2 = torch.empty_like(ref), torch.empty_like(ref)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        deep_gemm.fp8_gemm_nt(a, b, d)       # the stream has its workspace before the capture
+    s.synchronize()
+    assert torch.equal(d, ref)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        deep_gemm.fp8_gemm_nt(a, b, d)
+    for i in range(4):
+        d.fill_(float(i + 1))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(t):
+            graph.replay()
+        with torch.cuda.stream(s):
+            deep_gemm.fp8_gemm_nt(a2, b2, d2)
+        torch.cuda.synchronize()
+        _check(d, ref.cpu())
+        assert torch.equal(d2, ref2), i
+
+
+def test_quad_split_two_threads_on_a_stream():
+    """Two host threads on one stream: each call's two launches stay together."""
+    print('quad split two threads', flush=True)
+    calls = [_split_call(23), _split_call(24)]
+    outs = [[torch.empty_like(calls[0][2]) for _ in range(20)] for _ in calls]
+    torch.cuda.synchronize()
+    start = threading.Barrier(2)
+
+    def work(i):
+        start.wait(timeout=30)
+        for d in outs[i]:
+            deep_gemm.fp8_gemm_nt(calls[i][0], calls[i][1], d)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join(timeout=60)
+    torch.cuda.synchronize()
+    for i in range(2):
+        for d in outs[i]:
+            assert torch.equal(d, calls[i][2])
