@@ -483,6 +483,15 @@ bool quad_plan(const dg_gemm_args& a, int cus, bool allow_split, Plan& out) {
     return best < 1e300;
 }
 
+// Rows of D that end inside a 32-column block send the four-wave kernel's last tile of each row through LDS, about
+// 7 us that a short contraction of one round does not hide (e4m3 291 x N x 544, packed scales: N = 3840 7.0 us,
+// N = 3796 14.0 and 6.7 on 64x128 tiles of gemm_kernel; 1000 x 3001 x 1024 18.4 there; bf16 291 x 3796 x 512 7.1).
+bool cut_rows_short(const dg_gemm_args& a, int cus) {
+    return (a.gemm_type == kNormal || a.gemm_type == kBatched) && !a.a_mn_major && !a.b_mn_major && a.n % 32 != 0 &&
+           a.k <= (a.kind == kBF16 ? 512 : 1024) &&
+           ceil_div64(a.m, 128) * ceil_div64(a.n, 128) * (a.gemm_type == kBatched ? a.num_groups : 1) <= cus;
+}
+
 Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
     Plan skinny;
     if (skinny_kernel_plan(a, cus, allow_split, skinny_env(), skinny)) return skinny;
@@ -503,7 +512,8 @@ Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
             if (tc.bm == 384 && tc.bn == (fp4_b ? 128 : 192)) return {tc, 1, ceil_div(a.k, k_stage_elems(a.kind, tc)), 0, 0, 0};
     }
     Plan quad;
-    if (quad_plan(a, cus, allow_split, quad)) return quad;
+    const bool cut_short = cut_rows_short(a, cus);
+    if (!cut_short && quad_plan(a, cus, allow_split, quad)) return quad;
     allow_split = false;   // wide problems fill the CUs with tiles
     const int groups = (a.gemm_type == kBatched || a.gemm_type == kMasked || a.gemm_type == kKGrouped) ? a.num_groups : 1;
     // (K-grouped: each tile contracts one group's share of K)
@@ -520,7 +530,7 @@ Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
         // (anchored tiles only where the alignment rules out 256-row tiles, above: at alignment 256 they
         // measured behind, 526 vs 443 us for 256x224 at G=32 N=4096 K=7168, and FP8 x FP4 G=8 x 4096
         // rows N=7168 K=3072 took 2546 us on 384x192)
-        if (!tile_allowed(a, tc.bm, tc.bn) || tile_anchored(tc.bm)) continue;
+        if (!tile_allowed(a, tc.bm, tc.bn) || tile_anchored(tc.bm) || (cut_short && quad_tile(a.kind, tc.bm, tc.bn))) continue;
         const int ns = ceil_div(k_tile, k_stage_elems(a.kind, tc));
         const int64_t tiles = plan_tiles(a, tc);
         const int max_split = allow_split && tile_splittable(a.kind, tc) && tiles <= kMaxSplitTiles ? std::min(16, std::max(1, ns / 4)) : 1;

@@ -245,6 +245,16 @@ def test_workspace_size_of_fp8_output(lib, m, n, k):
     assert nbytes.value >= 64 * 1024 + tiles * info.split_k * info.block_m * info.block_n * 4
 
 
+@pytest.mark.parametrize('n, k, tile', [(3796, 1024, (64, 128)), (3796, 1040, (128, 128)), (3808, 1024, (128, 128))])
+def test_cut_rows_plan(lib, n, k, tile):
+    """Short contractions whose D rows end inside a 32-column block leave the four-wave tiles."""
+    args = _plan_args(291, n, k, 256)
+    args.alpha = 1.0
+    info = _lib.LaunchInfo()
+    assert lib.dg_launch_plan(args, ctypes.byref(info)) == 0, lib.dg_last_error()
+    assert (info.block_m, info.block_n) == tile
+
+
 def test_error_words_and_stream_workspace_without_device(lib):
     # no kernel has run: nothing pending; the workspace query rejects null outputs
     assert lib.dg_take_errors() == 0
