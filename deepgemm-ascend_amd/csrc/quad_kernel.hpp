@@ -507,12 +507,16 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
         constexpr int x = decltype(x_tag)::value;
         sc_raw[x] = *(lds_i32x4*)(lds + (A ? addr_sa : addr_sb) + decltype(s_tag)::value * SF_SLOT + decltype(h_tag)::value * SF_HALF + 16 * x);
     };
-    auto shift_scales = [&](auto a_tag, auto h_tag, auto n_tag) {
+    auto shift_scales = [&](auto a_tag, auto h_tag, auto n_tag, auto prologue_tag) {
         constexpr bool A = decltype(a_tag)::value != 0;
         constexpr int h = decltype(h_tag)::value;
         static_for<decltype(n_tag)::value>([&](auto j_c) {
             constexpr int j = decltype(j_c)::value;
-            const int v = (int)((uint32_t)sc_raw[j / 4][j % 4] >> sc_shift);
+            int v = (int)((uint32_t)sc_raw[j / 4][j % 4] >> sc_shift);
+            // (the shift stays here: where K is a compile-time constant of few stages the loop is straight-line code,
+            // and the compiler moved it to one wait state ahead of the MFMA that reads it; the ahead-of-time loops of
+            // the 384-row tiles hold it in place without, and have no register left for it)
+            if constexpr (!kWide || CK > 0 || decltype(prologue_tag)::value != 0) asm volatile("" : "+v"(v));
             if constexpr (A) sa[h][j] = v; else sb[h][j] = v;
         });
     };
@@ -604,7 +608,7 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
                     }
                 }
             });
-            if constexpr (NSR > 0 && i == kShift) shift_scales(Int<kReadA>{}, Int<rh>{}, Int<RN>{});
+            if constexpr (NSR > 0 && i == kShift) shift_scales(Int<kReadA>{}, Int<rh>{}, Int<RN>{}, Int<0>{});
             static_for<L1 - L0>([&](auto l_c) {
                 constexpr int l = decltype(l_c)::value;
                 constexpr int at = first + l * (NS - first) / (L1 - L0);
@@ -632,7 +636,7 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
         if constexpr (!kBf16) {
             read_scales(Int<A>{}, Int<0>{}, Int<0>{}, Int<0>{});
             if constexpr (A && kWide) read_scales(Int<A>{}, Int<0>{}, Int<0>{}, Int<1>{});
-            shift_scales(Int<A>{}, Int<0>{}, Int<(A ? NA0 : NB0)>{});
+            shift_scales(Int<A>{}, Int<0>{}, Int<(A ? NA0 : NB0)>{}, Int<1>{});
         }
         static_for<U>([&](auto u) {
             static_for<(A ? NA0 : NB0)>([&](auto j) {

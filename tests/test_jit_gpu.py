@@ -81,6 +81,27 @@ def test_jit_fp8_fp4_and_bf16():
     assert torch.equal(aot, jit)
 
 
+@pytest.mark.parametrize('b_kind', ['e4m3', 'e2m1'])
+@pytest.mark.parametrize('m,n,k', [(512, 512, 128), (512, 1056, 256), (1024, 2112, 384), (256, 512, 640)])
+def test_jit_few_stages(b_kind, m, n, k):
+    """Four-wave bodies whose K is a compile-time constant of one to five stages: straight-line loops."""
+    print(f'jit few stages {b_kind} m={m} n={n} k={k}', flush=True)
+    assert deep_gemm.launch_plan(m, n, k)['block_m'] >= 128
+    g = gen(36)
+    a, sfa, a_deq = operand(m, k, 'e4m3', (1, 32), g)
+    b, sfb, b_deq = operand(n, k, b_kind, (1, 32), g)
+    a, sfa, b, sfb = a.cuda(), sfa.cuda(), b.cuda(), sfb.cuda()
+    fn = deep_gemm.fp8_gemm_nt if b_kind == 'e4m3' else deep_gemm.fp8_fp4_gemm_nt
+
+    def run():
+        d = torch.empty(m, n, dtype=torch.float32, device='cuda')
+        fn((a, sfa), (b, sfb), d)
+        return d
+    aot, jit = _both(run)
+    assert torch.equal(aot, jit)
+    assert calc_diff(jit.cpu(), og.gemm_nt(a_deq, b_deq, torch.float32)) < THRESH
+
+
 def test_jit_m_grouped_and_masked():
     print('jit m-grouped / masked', flush=True)
     g = gen(33)
