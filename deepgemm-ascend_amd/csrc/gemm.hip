@@ -819,10 +819,14 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
     }
     if ((amn ? lda_b < a.m * esz_a : lda_b < kbytes_a) || (bmn ? ldb_b < a.n * esz_b : ldb_b < kbytes_b) || a.ldd < a.n)
         return dg_set_error("dg_gemm: leading dimension smaller than the row");
-    // (an MN-major operand's whole K extent must fit a buffer range below the dead-load offset)
-    if ((amn ? (int64_t)a.k * lda_b >= 0x40000000LL : (int64_t)256 * lda_b > 0x7fffffffLL) ||
-        (bmn ? (int64_t)a.k * ldb_b >= 0x40000000LL : (int64_t)256 * ldb_b > 0x7fffffffLL))
+    if ((!amn && (int64_t)256 * lda_b > 0x7fffffffLL) || (!bmn && (int64_t)256 * ldb_b > 0x7fffffffLL))
         return dg_set_error("dg_gemm: row stride too large for 32-bit tile offsets");
+    // (an MN-major operand's whole K extent must fit a buffer range below the dead-load offset; its K-major copy may
+    // be any size)
+    if ((amn && (int64_t)a.k * lda_b >= 0x40000000LL) || (bmn && (int64_t)a.k * ldb_b >= 0x40000000LL)) {
+        dg_set_error("dg_gemm: MN-major operands of 1 GiB or more are not read in place");
+        return DG_ENOKERNEL;
+    }
     if (!bf16 && ((a.sfa_ld | a.sfb_ld | a.sfa_batch_stride | a.sfb_batch_stride) & 1))
         return dg_set_error("dg_gemm: SF leading dimensions and batch strides must be even (int16 elements)");
     if (a.gemm_type == kMGroupedPsum || a.gemm_type == kMGroupedIdx) {

@@ -118,7 +118,9 @@ typedef struct dg_gemm_args {
     int32_t a_mn_major;           /* 1: A is stored [K][M] (M contiguous; lda = stride between its K
                                      rows, in elements), read in place.  e4m3 x e4m3 and bf16 x bf16
                                      dense, batched and K-grouped GEMMs on the tiles of 128 x 128 to
-                                     256 x 256 with 128-byte stages only; any other plan fails with DG_ENOKERNEL (callers then copy to K-major).
+                                     256 x 256 with 128-byte stages only; any other plan, and an
+                                     operand whose K rows span 1 GiB or more, fails with
+                                     DG_ENOKERNEL (callers then copy to K-major).
                                      The reference's operand majors: deep_gemm/include/deep_gemm/
                                      fp8_gemm.hpp:18-35.                                            */
     int32_t b_mn_major;           /* 1: B is stored [K][N], likewise                                 */

@@ -5,6 +5,7 @@ import re
 from pathlib import Path
 
 import pytest
+import torch
 
 from deep_gemm import _lib
 
@@ -253,6 +254,39 @@ def test_cut_rows_plan(lib, n, k, tile):
     info = _lib.LaunchInfo()
     assert lib.dg_launch_plan(args, ctypes.byref(info)) == 0, lib.dg_last_error()
     assert (info.block_m, info.block_n) == tile
+
+
+@pytest.mark.parametrize('kind, m, n, k, form', [
+    (_lib.DG_KIND_BF16, 4096, 151936, 5120, 'nn'), (_lib.DG_KIND_BF16, 256, 128256, 8192, 'nn'),
+    (_lib.DG_KIND_BF16, 4096, 129280, 7168, 'nn'), (_lib.DG_KIND_FP8_FP8, 512, 151936, 8192, 'nn'),
+    (_lib.DG_KIND_BF16, 8192, 4096, 65536, 'tn'), (_lib.DG_KIND_BF16, 192, 65536, 8192, 'nn')])
+def test_large_mn_major_operands_are_copied(lib, monkeypatch, kind, m, n, k, form):
+    """An MN-major operand of 1 GiB or more has no kernel that reads it in place (DG_ENOKERNEL, not an error of
+    the call): the wrapper then launches on a K-major copy, which plans at any size."""
+    from deep_gemm import gemm
+    elem = 2 if kind == _lib.DG_KIND_BF16 else 1
+    dtype = torch.bfloat16 if elem == 2 else torch.float8_e4m3fn
+    a_mn, b_mn = form[0] == 't', form[1] == 'n'
+    args = _plan_args(m, n, k, 256)
+    args.kind, args.alpha, args.library_workspace = kind, 1.0, 1
+    launches = []
+
+    def launch(args, d, allow_no_kernel=False):
+        rc = lib.dg_launch_plan(ctypes.byref(args), ctypes.byref(_lib.LaunchInfo()))
+        launches.append((args.a_mn_major, args.b_mn_major, rc))
+        if rc == _lib.DG_ENOKERNEL and allow_no_kernel:
+            return False
+        assert rc == 0, lib.dg_last_error()
+        return True
+
+    monkeypatch.setattr(gemm, '_launch', launch)
+    monkeypatch.setattr(gemm, '_transpose_to_k_major', lambda t, k: torch.empty(t.size(-2), k, dtype=t.dtype, device='meta'))
+    a = torch.empty(k, m, dtype=dtype, device='meta').t() if a_mn else torch.empty(m, k, dtype=dtype, device='meta')
+    b = torch.empty(k, n, dtype=dtype, device='meta').t() if b_mn else torch.empty(n, k, dtype=dtype, device='meta')
+    gemm._launch_operands(args, torch.empty(m, n, device='meta'), a, b, k, False, False)
+    big = (a_mn and k * m * elem >= 1 << 30, b_mn and k * n * elem >= 1 << 30)
+    assert any(big) and launches[0] == (int(a_mn), int(b_mn), _lib.DG_ENOKERNEL), launches
+    assert launches[-1] == (int(a_mn and not big[0]), int(b_mn and not big[1]), 0), launches
 
 
 def test_error_words_and_stream_workspace_without_device(lib):
