@@ -1177,7 +1177,7 @@ namespace {
 constexpr int64_t kNoAllocScratchBytes = (16 << 20) + dg::kCounterBytes;
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 
-std::mutex g_scratch_mu;
+std::mutex g_scratch_mu, g_scratch_order_mu;
 void* g_scratch_ptr[64] = {nullptr};
 
 // Device address of `scratch` on the current device (host code never passes the array's name:
@@ -1213,23 +1213,33 @@ extern "C" int dg_gemm_noalloc(const dg_gemm_args* args, void* stream) {
     a.workspace = reinterpret_cast<void*>(1);   // (any non-null value: the plan may then split K)
     int rc = dg_gemm_workspace_size(&a, &need);
     if (rc != DG_OK) return rc;
-    // (a tile plan whose partials do not fit runs unsplit instead)
-    const int cus = a.num_cus > 0 ? a.num_cus : dg::device_cus();
-    const bool falls_back = need > 0 && a.split_k <= 1 && dg::choose(a, cus, true).skinny_nw == 0;
-    if (need > kNoAllocScratchBytes && !falls_back) {
+    // Every stream and every captured graph of the device shares the scratch.  A four-wave tile plan runs unsplit and
+    // leaves it alone: calls of more than 128 rows on two streams, or in a replay beside an eager call, share nothing.
+    if (need > 0 && a.split_k == 0) {
+        const dg::Plan plan = dg::choose(a, a.num_cus > 0 ? a.num_cus : dg::device_cus(), true);
+        if (plan.skinny_nw == 0 && dg::quad_tile(a.kind, plan.tile.bm, plan.tile.bn)) {
+            a.split_k = 1;
+            need = 0;
+        }
+    }
+    if (need > kNoAllocScratchBytes) {
         char buf[200];
         snprintf(buf, sizeof(buf), "dg_gemm_noalloc: this problem's split-K plan needs %lld bytes of scratch, more than "
                  "the %lld-byte maximum (call dg_gemm with a workspace, or split_k = 1)", (long long)need,
                  (long long)kNoAllocScratchBytes);
         return dg_set_error(buf);
     }
-    // (the scratch stands in for a workspace whether or not this plan splits K, so the plan is
-    // always the one dg_gemm makes when given a workspace)
+    // (the scratch stands in for a workspace whether or not this plan splits K, so other plans are the ones that
+    // dg_gemm makes when given a workspace)
     void* ptr = nullptr;
     rc = scratch_address(&ptr);
     if (rc != DG_OK) return rc;
     a.workspace = ptr;
     a.workspace_bytes = kNoAllocScratchBytes;
+    // a call that hands data on through the scratch (partials to their reduction, the run table to its tiles) keeps
+    // its launches together: another thread's call on the stream comes before or after
+    std::unique_lock<std::mutex> order(g_scratch_order_mu, std::defer_lock);
+    if (need > 0 || a.gemm_type == dg::kMGroupedIdx) order.lock();
     return gemm_impl(&a, stream, false, nullptr, true);
 }
 

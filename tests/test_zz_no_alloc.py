@@ -1,6 +1,6 @@
 """dg_gemm_noalloc (the allocation-free dg_gemm: split-K scratch in a fixed device array) against
-dg_gemm with a caller workspace, through the C ABI: the same plan, bit-identical D, on two calls in
-a row (the second smaller), plus the oracle and the over-size rejection."""
+dg_gemm with a caller workspace, through the C ABI: decode plans (the same plan, bit-identical D, on two calls in
+a row, the second smaller), tile plans (unsplit), the oracle and the over-size rejection."""
 import ctypes
 
 import pytest
@@ -85,6 +85,79 @@ def test_noalloc_gemv_plan():
         d_ws = _run(lib, args, False)
         assert torch.equal(d_noalloc.view(torch.int16), d_ws.view(torch.int16))
         assert calc_diff(d_noalloc, ref) < 1e-5
+
+
+@pytest.mark.parametrize('m,n,k', [(129, 2112, 7168), (200, 2112, 7168), (300, 2112, 7168), (400, 4480, 8192)])
+def test_noalloc_tile_plans_run_unsplit(m, n, k):
+    """Tile plans whose default splits K (within and past the scratch's 16 MiB) run unsplit and never write the
+    scratch that other streams and graphs of the device use: bit-identical to dg_gemm without a K split, and so is
+    a captured call, replayed while calls of the same shape run on another stream."""
+    lib = _lib.load()
+    args, keep, ref = _args(m, n, k, 10)
+    info = _lib.LaunchInfo()
+    args.workspace, args.workspace_bytes = 1, 1 << 40
+    _lib.check(lib.dg_launch_plan(ctypes.byref(args), ctypes.byref(info)), lib)
+    print(f'noalloc tile plan m={m} n={n} k={k} split_k={info.split_k} block={info.block_m}x{info.block_n}', flush=True)
+    assert info.split_k > 1 and info.skinny == 0
+    args.d_dtype = _lib.DG_DTYPE_F32
+    args.workspace, args.workspace_bytes, args.split_k = None, 0, 1
+    out = [torch.empty(m, n, device='cuda') for _ in range(4)]
+
+    def call(fn, d, stream):
+        args.d = d.data_ptr()
+        _lib.check(fn(ctypes.byref(args), ctypes.c_void_p(stream.cuda_stream)), lib)
+    s, t = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    call(lib.dg_gemm, out[0], s)
+    args.split_k = 0
+    call(lib.dg_gemm_noalloc, out[1], s)
+    torch.cuda.synchronize()
+    assert calc_diff(out[0].bfloat16().cpu(), ref) < 1e-5
+    assert torch.equal(out[0], out[1])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        call(lib.dg_gemm_noalloc, out[2], s)
+    for i in range(4):
+        for d in out[1:]:
+            d.fill_(float(i + 1))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            graph.replay()
+        call(lib.dg_gemm_noalloc, out[1], t)
+        call(lib.dg_gemm_noalloc, out[3], t)
+        torch.cuda.synchronize()
+        assert all(torch.equal(d, out[0]) for d in out[1:]), i
+
+
+def test_noalloc_two_threads_on_a_stream():
+    """Two host threads on one stream, decode plans summed by a second launch: each call's launches stay together."""
+    import threading
+    lib = _lib.load()
+    print('noalloc two threads', flush=True)
+    stream = torch.cuda.Stream()
+    calls = []
+    for seed in (11, 12):
+        args, keep, _ = _args(128, 4096, 7168, seed)
+        ref = _run(lib, args, False)
+        args.workspace, args.workspace_bytes = None, 0
+        calls.append((args, keep, ref, [torch.empty(128, 4096, dtype=torch.bfloat16, device='cuda') for _ in range(20)]))
+    torch.cuda.synchronize()
+    start, errors = threading.Barrier(2), []
+
+    def work(args, outs):
+        start.wait(timeout=30)
+        for d in outs:
+            args.d = d.data_ptr()
+            errors.append(lib.dg_gemm_noalloc(ctypes.byref(args), ctypes.c_void_p(stream.cuda_stream)))
+    threads = [threading.Thread(target=work, args=(c[0], c[3])) for c in calls]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join(timeout=60)
+    torch.cuda.synchronize()
+    assert errors == [0] * 40
+    for _, _, ref, outs in calls:
+        assert all(torch.equal(d.cpu(), ref) for d in outs)
 
 
 def test_noalloc_rejects_oversize_and_a_workspace():
