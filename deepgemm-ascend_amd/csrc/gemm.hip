@@ -941,8 +941,8 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
     const bool persistent = want_persistent && !jit && !skinny && !amn && !bmn && plan.split == 1 && tile_persistable(cfg) &&
                             a.k > 0 && a.gemm_type != kKGrouped && a_span <= 0x7fffffffLL &&
                             b_span <= 0x7fffffffLL && sfa_span <= 0x7fffffffLL && sfb_span <= 0x7fffffffLL;
-    KernelFn fn = jit ? nullptr
-                : skinny ? (plan.skinny_rows ? lookup_skinny_rows(a.kind, cfg.bm / 32, cfg.bn / 32, plan.skinny_d, epi_kind)
+    // (a JIT call has it too: a capture runs it where the run-time compiled kernel is not loaded yet)
+    KernelFn fn = skinny ? (plan.skinny_rows ? lookup_skinny_rows(a.kind, cfg.bm / 32, cfg.bn / 32, plan.skinny_d, epi_kind)
                           : skinny_mn ? lookup_skinny_mn(a.kind, cfg.bm / 32, cfg.bn / 32, plan.skinny_nw, plan.skinny_d, plan.skinny_ar, epi_kind)
                                       : lookup_skinny(a.kind, cfg.bm / 32, cfg.bn / 32, plan.skinny_nw, plan.skinny_d, plan.skinny_ar, epi_kind))
                 : (amn || bmn) ? lookup_kernel_mn(a.kind, cfg.bm, cfg.bn, epi_kind, amn, bmn)
@@ -1115,11 +1115,13 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
             if (rc != DG_OK) return rc;
         }
     }
+    bool tiles_done = false;
     if (jit) {
-        const int rc = jit_run(a, cfg, epi_kind, plan.split, p, launched, st, compile_only);
-        if (rc != DG_OK || compile_only || reduce_fn == nullptr) return rc;
+        const int rc = jit_run(a, cfg, epi_kind, plan.split, p, launched, st, compile_only, fn != nullptr);
+        if (rc != kJitNotLoaded && (rc != DG_OK || compile_only || reduce_fn == nullptr)) return rc;
+        tiles_done = rc == DG_OK;
     }
-    for (int64_t base = 0; !jit && base < grid; base += launched) {
+    for (int64_t base = 0; !tiles_done && base < grid; base += launched) {
         p.vbase = (int)base;
         const unsigned n = (unsigned)std::min<int64_t>(launched, grid - base);
         const hipError_t e = launch_module_kernel(reinterpret_cast<const void*>(fn), n, (unsigned)threads, p, st, lds_bytes);

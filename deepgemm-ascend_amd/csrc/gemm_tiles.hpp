@@ -148,9 +148,12 @@ inline int tile_threads(int kind, int bm, int bn, bool persistent) {
 }
 
 // Run-time compiled kernel of one launch plan (csrc/jit.hip): compile or fetch it and, unless
-// compile_only, launch it on `st`.
+// compile_only, launch it on `st`.  With an ahead-of-time kernel of the plan at hand nothing is compiled or
+// loaded inside a stream capture (a captured plan may differ from the eager one): kJitNotLoaded, and the caller
+// launches that kernel, whose results are the same bits.
+constexpr int kJitNotLoaded = 1;
 int jit_run(const dg_gemm_args& a, const TileCfg& cfg, int epi, int split, const KParams& p, int64_t grid,
-            hipStream_t st, bool compile_only);
+            hipStream_t st, bool compile_only, bool ahead_of_time);
 
 // Skinny-M kernels (csrc/skinny_kernel.hpp): strips of 32 nb columns, M <= ar (<= 32 mt) rows of
 // A, nw waves splitting K, each with a ring of d group slots.

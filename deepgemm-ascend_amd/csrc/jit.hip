@@ -145,8 +145,8 @@ std::string source_of(const Spec& s) {
     return buf;
 }
 
-// Code object of `src` (memory, then disk, then hipRTC); `key` receives its cache key.
-bool code_object(const std::string& src, std::string& key, const std::vector<char>*& code) {
+// Cache key of `src` with the headers, options and compiler in use.
+std::string cache_key(const std::string& src) {
     uint64_t h = 1469598103934665603ull;
     h = fnv1a(h, src);
     for (const std::string& text : g_headers) h = fnv1a(h, text);
@@ -156,8 +156,17 @@ bool code_object(const std::string& src, std::string& key, const std::vector<cha
     h = fnv1a(h, std::to_string(major) + "." + std::to_string(minor));
     char hex[32];
     snprintf(hex, sizeof(hex), "%016llx", (unsigned long long)h);
-    key = std::string("dg_gemm_") + hex;
+    return std::string("dg_gemm_") + hex;
+}
 
+bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
+    return cs != hipStreamCaptureStatusNone;
+}
+
+// Code object of `src` (memory, then disk, then hipRTC) under its cache key.
+bool code_object(const std::string& src, const std::string& key, const std::vector<char>*& code) {
     auto it = g_code.find(key);
     if (it != g_code.end()) {
         code = &it->second;
@@ -213,10 +222,8 @@ bool code_object(const std::string& src, std::string& key, const std::vector<cha
 
 }  // namespace
 
-// Compile (or fetch from the caches) the kernel for one launch plan and, unless compile_only,
-// launch it on `st`.
 int jit_run(const dg_gemm_args& a, const TileCfg& cfg, int epi, int split, const KParams& p, int64_t grid,
-            hipStream_t st, bool compile_only) {
+            hipStream_t st, bool compile_only, bool ahead_of_time) {
     Spec s;
     s.t = cfg;
     s.kind = a.kind;
@@ -233,14 +240,17 @@ int jit_run(const dg_gemm_args& a, const TileCfg& cfg, int epi, int split, const
     {
         std::lock_guard<std::mutex> lk(g_mu);
         if (!load_headers()) return DG_EINVAL;
-        std::string key;
-        const std::vector<char>* code = nullptr;
-        if (!code_object(src, key, code)) return DG_ENOKERNEL;
-        if (compile_only) return DG_OK;
+        const std::string key = cache_key(src);
         int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return dg_set_error("dg_jit: hipGetDevice failed");
+        if (!compile_only && hipGetDevice(&dev) != hipSuccess) return dg_set_error("dg_jit: hipGetDevice failed");
         const std::string fkey = key + "@" + std::to_string(dev);
-        auto it = g_fn.find(fkey);
+        auto it = compile_only ? g_fn.end() : g_fn.find(fkey);
+        const std::vector<char>* code = nullptr;
+        if (it == g_fn.end()) {
+            if (!compile_only && ahead_of_time && capturing(st)) return kJitNotLoaded;
+            if (!code_object(src, key, code)) return DG_ENOKERNEL;
+            if (compile_only) return DG_OK;
+        }
         if (it != g_fn.end()) {
             ++g_stat_mem;
             fn = it->second;

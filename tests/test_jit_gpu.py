@@ -165,6 +165,74 @@ def test_jit_batched_and_split(monkeypatch):
     assert calc_diff(jit.cpu(), og.gemm_nt(a_deq, b_deq)) < THRESH
 
 
+def test_jit_capture_compiles_nothing():
+    """A captured call runs another plan than the eager one (no K split): the graph takes the ahead-of-time kernel
+    where the run-time compiled one was not built before, and the built one where it was; every replay matches."""
+    m, n, k = 300, 2112, 7168
+    print('jit capture', flush=True)
+    assert deep_gemm.launch_plan(m, n, k)['split_k'] > 1
+    g = gen(37)
+    a, sfa, _ = operand(m, k, 'e4m3', (1, 32), g)
+    b, sfb, _ = operand(n, k, 'e4m3', (1, 32), g)
+    a = (a.cuda(), deep_gemm.transform_sf_into_required_layout(sfa.cuda(), m, k, (1, 32), is_sfa=True))
+    b = (b.cuda(), deep_gemm.transform_sf_into_required_layout(sfb.cuda(), n, k, (1, 32), is_sfa=False))
+    d, e = (torch.empty(m, n, dtype=torch.float32, device='cuda') for _ in range(2))
+    s = torch.cuda.Stream()
+
+    def eager(split):
+        if split == 1:
+            os.environ['DG_SPLIT_K'] = '1'
+        try:
+            deep_gemm.fp8_gemm_nt(a, b, e)
+        finally:
+            os.environ.pop('DG_SPLIT_K', None)
+        torch.cuda.synchronize()
+        return e.clone()
+    unsplit = eager(1)
+    deep_gemm.set_jit(True)
+    with torch.cuda.stream(s):
+        split = eager(0)
+    assert not torch.equal(split, unsplit)
+    for built in (False, True):
+        if built:
+            assert torch.equal(eager(1), unsplit)   # builds the unsplit body
+        before = _lib.jit_stats()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            deep_gemm.fp8_gemm_nt(a, b, d)
+        after = _lib.jit_stats()
+        assert after[:2] == before[:2] and after[2] == before[2] + built, (before, after)
+        for i in range(3):
+            d.fill_(float(i + 1))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(d, unsplit), i
+            with torch.cuda.stream(s):
+                assert torch.equal(eager(0), split)
+
+
+def test_jit_split_tiles_match_ahead_of_time(monkeypatch):
+    """Forced K splits on the four-wave tiles: the run-time compiled tiles, then the second launch that sums them."""
+    g = gen(38)
+    m, n, k = 300, 260, 1408
+    a, sfa, a_deq = operand(m, k, 'e4m3', (1, 32), g)
+    b, sfb, b_deq = operand(n, k, 'e4m3', (1, 32), g)
+    a, sfa, b, sfb = a.cuda(), sfa.cuda(), b.cuda(), sfb.cuda()
+    for tile, split in (('256x256', 3), ('256x224', 2), ('256x128', 5), ('128x128', 4)):
+        print(f'jit split {tile} x {split}', flush=True)
+        monkeypatch.setenv('DG_FORCE_BLOCK', tile)
+        monkeypatch.setenv('DG_SPLIT_K', str(split))
+
+        def run():
+            d = torch.empty(m, n, dtype=torch.float32, device='cuda')
+            deep_gemm.fp8_gemm_nt((a, sfa), (b, sfb), d)
+            return d
+        aot, jit = _both(run)
+        assert torch.equal(aot, jit)
+        assert calc_diff(jit.cpu(), og.gemm_nt(a_deq, b_deq, torch.float32)) < THRESH
+
+
 def test_jit_dry_run_compiles_without_launch():
     print('jit dry run', flush=True)
     g = gen(35)
