@@ -843,9 +843,10 @@ int gemm_impl(const dg_gemm_args* args, void* stream, bool compile_only, dg_laun
         if (!plan_only && !compile_only) {
             const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
             // A tile plan also runs unsplit.  So it does in a graph, which may be replayed on any stream, beside
-            // others of its capture stream: none of them then writes the stream's partials.
+            // others of its capture stream, and on hipStreamPerThread, one handle for a stream of each thread: none
+            // of them then writes the partials of a call beside it.
             const bool unsplit_too = plan.skinny_nw == 0 && a.split_k <= 1;
-            if (unsplit_too && stream_capturing(st)) {
+            if (unsplit_too && (st == hipStreamPerThread || stream_capturing(st))) {
                 plan = choose(a, cus, false);
             } else {
                 order = stream_order(st);

@@ -113,8 +113,9 @@ typedef struct dg_gemm_args {
                                      need, zero-filled, only ever grown and never freed (a captured
                                      graph may hold it).  Growing it while the stream is being
                                      captured is an error: run the call once before the capture.
-                                     Tile plans (block_m >= 128, other than decode's) captured with
-                                     split_k = 0 run unsplit and need none.                      */
+                                     Tile plans (block_m >= 128, other than decode's) captured, or
+                                     on hipStreamPerThread, with split_k = 0 run unsplit and need
+                                     none.                                                       */
     int32_t a_mn_major;           /* 1: A is stored [K][M] (M contiguous; lda = stride between its K
                                      rows, in elements), read in place.  e4m3 x e4m3 and bf16 x bf16
                                      dense, batched and K-grouped GEMMs on the tiles of 128 x 128 to

@@ -4,12 +4,14 @@ a block; every operand layout; D rows that take the vector path, that need eleme
 K ranges summed by the second launch.  Against the CPU oracle (dequantise, fp32 matmul).  The bound on
 calc_diff is the repository's 1e-5; every element is also held to 1e-3 of itself or the root mean square (the
 alignment of e4m3 products inside one MFMA leaves up to 1.4e-4 of it), plus one unit of a bf16 result."""
+import ctypes
 import threading
 
 import pytest
 import torch
 
 import deep_gemm
+from deep_gemm import _lib
 from oracle import gemm as og, layout as ol
 from helpers import gen, operand, calc_diff
 
@@ -256,3 +258,42 @@ def test_quad_split_two_threads_on_a_stream():
     for i in range(2):
         for d in outs[i]:
             assert torch.equal(d, calls[i][2])
+
+
+def test_quad_split_per_thread_streams():
+    """hipStreamPerThread names another stream in every thread: calls of two threads share no partials (they run
+    unsplit)."""
+    print('quad split per-thread streams', flush=True)
+    lib = _lib.load()
+    m, n, k = 300, 2112, 7168
+    calls = []
+    for seed in (25, 26):
+        a, b, _ = _split_call(seed)
+        args = _lib.GemmArgs()
+        args.kind, args.gemm_type, args.m, args.n, args.k, args.num_groups = _lib.DG_KIND_FP8_FP8, _lib.DG_GEMM_NORMAL, m, n, k, 1
+        args.a, args.b, args.sfa, args.sfb = a[0].data_ptr(), b[0].data_ptr(), a[1].data_ptr(), b[1].data_ptr()
+        args.lda, args.ldb, args.ldd = k, k, n
+        args.sfa_ld, args.sfb_ld = a[1].stride(-1), b[1].stride(-1)
+        args.d_dtype, args.alpha, args.alignment, args.library_workspace, args.split_k = _lib.DG_DTYPE_F32, 1.0, 256, 1, 1
+        ref = torch.empty(m, n, device='cuda')
+        args.d = ref.data_ptr()
+        _lib.check(lib.dg_gemm(ctypes.byref(args), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), lib)
+        args.split_k = 0
+        calls.append((args, (a, b), ref, [torch.empty_like(ref) for _ in range(20)]))
+    torch.cuda.synchronize()
+    start, codes = threading.Barrier(2), []
+
+    def work(args, outs):
+        start.wait(timeout=30)
+        for d in outs:
+            args.d = d.data_ptr()
+            codes.append(lib.dg_gemm(ctypes.byref(args), ctypes.c_void_p(2)))
+    threads = [threading.Thread(target=work, args=(c[0], c[3])) for c in calls]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join(timeout=60)
+    torch.cuda.synchronize()
+    assert codes == [0] * 40
+    for _, _, ref, outs in calls:
+        assert all(torch.equal(d, ref) for d in outs)
