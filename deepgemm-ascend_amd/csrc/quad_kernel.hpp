@@ -507,16 +507,17 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
         constexpr int x = decltype(x_tag)::value;
         sc_raw[x] = *(lds_i32x4*)(lds + (A ? addr_sa : addr_sb) + decltype(s_tag)::value * SF_SLOT + decltype(h_tag)::value * SF_HALF + 16 * x);
     };
+    constexpr bool kPinShift = !kWide || CK > 0;
     auto shift_scales = [&](auto a_tag, auto h_tag, auto n_tag, auto prologue_tag) {
         constexpr bool A = decltype(a_tag)::value != 0;
         constexpr int h = decltype(h_tag)::value;
         static_for<decltype(n_tag)::value>([&](auto j_c) {
             constexpr int j = decltype(j_c)::value;
             int v = (int)((uint32_t)sc_raw[j / 4][j % 4] >> sc_shift);
-            // (the shift stays here: where K is a compile-time constant of few stages the loop is straight-line code,
-            // and the compiler moved it to one wait state ahead of the MFMA that reads it; the ahead-of-time loops of
-            // the 384-row tiles hold it in place without, and have no register left for it)
-            if constexpr (!kWide || CK > 0 || decltype(prologue_tag)::value != 0) asm volatile("" : "+v"(v));
+            // (the shift stays ahead of the s_nop that follows: where K is a compile-time constant of few stages the
+            // loop is straight-line code, and the compiler moved it to one wait state ahead of the MFMA that reads it;
+            // the ahead-of-time loops of the 384-row tiles hold it in place without, and have no register left for it)
+            if constexpr (kPinShift || decltype(prologue_tag)::value != 0) asm volatile("" : "+v"(v));
             if constexpr (A) sa[h][j] = v; else sb[h][j] = v;
         });
     };
@@ -575,7 +576,9 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
         constexpr int NL = SA::loads(lha) + SB::loads(lhb) + NSF;
         constexpr int L0 = (P & 1) ? (NL + 1) / 2 : 0, L1 = (P & 1) ? NL : (NL + 1) / 2;
         constexpr int first = (P & 1) == 0 ? 1 : 0;   // (slot 0 of phases 0 and 2 holds the barrier)
-        constexpr int kShift = NS - 3;
+        // (after the phase's last MFMA and two wait states ahead of the next phase's: two slots earlier the wait for the
+        // scales cost 128x128 tiles, of four slots a phase, 3-5 %)
+        constexpr int kShift = kPinShift ? NS - 1 : NS - 3;
         // loads that may stay in flight at the barrier: the two half-stages issued last
         constexpr int kFlight = P == 0 ? SA::loads(0) + SB::loads(1 - f) + SA::loads(1) + SB::loads(f) + 2 * NSF
                                        : SA::loads(1) + SB::loads(f) + SA::loads(0) + SB::loads(f) + 2 * NSF;
@@ -608,12 +611,15 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
                     }
                 }
             });
-            if constexpr (NSR > 0 && i == kShift) shift_scales(Int<kReadA>{}, Int<rh>{}, Int<RN>{}, Int<0>{});
             static_for<L1 - L0>([&](auto l_c) {
                 constexpr int l = decltype(l_c)::value;
                 constexpr int at = first + l * (NS - first) / (L1 - L0);
                 if constexpr (at == i) issue(Int<L0 + l>{}, s_tag, Int<lha>{}, Int<lhb>{});
             });
+            if constexpr (NSR > 0 && i == kShift) {
+                shift_scales(Int<kReadA>{}, Int<rh>{}, Int<RN>{}, Int<0>{});
+                if constexpr (kPinShift) asm volatile("s_nop 1");
+            }
             if constexpr (P == 3 && i == NS - 1) set_stage(c + 3);
             __builtin_amdgcn_sched_barrier(0);
         });
