@@ -741,109 +741,171 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
         });
         return;
     } else {
-    // Vector path: D rows of whole, aligned quartets and no block of columns that the row's end cuts; else
-    // the rows go through LDS a block at a time and are stored element by element.
-    const bool vec = p.vec_store && !p.has_bias && (n0 + BN <= N || N % 32 == 0);
-    if (vec) {
-        static_for<2>([&](auto ha_c) {
-            constexpr int ha = decltype(ha_c)::value;
-            static_for<SA::nb(ha)>([&](auto i_c) {
-                const int m = row_of(ha_c, i_c, wm, r);
-                bool row_ok, pad_row;
-                row_state(m, row_ok, pad_row);
-                uint8_t* const drow = tl.d_base + ((int64_t)m * p.ldd + n0) * DE;
-                constexpr int NQ = (SB::NB0 + SB::NB1) * (kBf16 ? 4 : 1);   // quartets of a row a lane holds
-                f32x4 v[NQ];
-                int col[NQ];   // a quartet's first column within the tile
-                static_for<SB::NB0 + SB::NB1>([&](auto b_c) {
-                    constexpr int b = decltype(b_c)::value, hb = b >= SB::NB0, j = hb ? b - SB::NB0 : b;
-                    const acc_t a = take(ha_c, Int<hb>{}, i_c, Int<j>{});
-                    const int c0 = col_of(Int<hb>{}) + j * MR + 4 * q;
-                    if constexpr (kBf16) {
+    // Vector path: D rows of aligned quartets.  Whole blocks of columns are stored from registers; the one that
+    // the row's end cuts goes through LDS as a strip of the tile's rows and is stored element by element.  Rows of
+    // unaligned quartets all go through LDS, a block row at a time.
+    if (p.vec_store) {
+        const int row_cols = N - n0;                  // columns of D from the tile's first
+        const int cut = row_cols < BN && row_cols % MR != 0 ? row_cols / MR * MR : BN;   // the cut block's first
+        const int stored = min(row_cols, cut);        // columns stored from registers
+        auto whole = [&](int first) -> bool { return first < stored; };                   // (a block's first column)
+        float* const lds_bias = reinterpret_cast<float*>(smem);                           // [BN], zeros past the row
+        float* const strip = lds_bias + 256;                                              // [BM][MR]
+        static_assert(BN <= 256 && 1024 + BM * MR * 4 <= T::LDS_BYTES, "staging areas");
+        if (p.has_bias || cut < BN) __syncthreads();   // (every wave has read its last fragments)
+        if (p.has_bias) {
+            if (tid < BN) {
+                lds_bias[tid] = tid >= row_cols ? 0.f
+                              : kF32 ? reinterpret_cast<const float*>(p.bias)[n0 + tid]
+                                     : bf16_to_f32(reinterpret_cast<const uint16_t*>(p.bias)[n0 + tid]);
+            }
+            __syncthreads();
+        }
+        constexpr int NQ = (SB::NB0 + SB::NB1) * (kBf16 ? 4 : 1);   // quartets of a row a lane holds
+        auto first_of = [&](int t) -> int {   // first column of a quartet's block within the tile
+            const int b = kBf16 ? t / 4 : t;
+            return b >= SB::NB0 ? col_of(Int<1>{}) + (b - SB::NB0) * MR : col_of(Int<0>{}) + b * MR;
+        };
+        constexpr bool kMayAccumulate = EPI == kEpiF32 || EPI == kEpiBf16;
+        // PLAIN: no bias, no old values and no cut block.  The straight-line code of a tile's rows runs once per tile, so
+        // that its size is time.
+        auto store_rows = [&](auto plain_tag) {
+            constexpr bool PLAIN = decltype(plain_tag)::value != 0;
+            static_for<2>([&](auto ha_c) {
+                constexpr int ha = decltype(ha_c)::value;
+                static_for<SA::nb(ha)>([&](auto i_c) {
+                    const int m = row_of(ha_c, i_c, wm, r);
+                    bool row_ok, pad_row;
+                    row_state(m, row_ok, pad_row);
+                    uint8_t* const drow = tl.d_base + ((int64_t)m * p.ldd + n0) * DE;
+                    f32x4 v[NQ];
+                    int col[NQ];   // a quartet's first column within the tile
+                    static_for<SB::NB0 + SB::NB1>([&](auto b_c) {
+                        constexpr int b = decltype(b_c)::value, hb = b >= SB::NB0, j = hb ? b - SB::NB0 : b;
+                        const acc_t a = take(ha_c, Int<hb>{}, i_c, Int<j>{});
+                        const int c0 = col_of(Int<hb>{}) + j * MR + 4 * q;
+                        if constexpr (kBf16) {
 #pragma unroll
-                        for (int g = 0; g < 4; ++g) {
-                            v[4 * b + g] = f32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]} * p.alpha;
-                            col[4 * b + g] = c0 + 8 * g;
+                            for (int g = 0; g < 4; ++g) {
+                                v[4 * b + g] = f32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]} * p.alpha;
+                                col[4 * b + g] = c0 + 8 * g;
+                            }
+                        } else {
+                            v[b] = a * p.alpha;
+                            col[b] = c0;
+                        }
+                        if (!PLAIN && first_of(kBf16 ? 4 * b : b) == cut) {
+                            float* const row = strip + (m - m0) * MR + 4 * q;
+#pragma unroll
+                            for (int g = 0; g < (kBf16 ? 4 : 1); ++g) *reinterpret_cast<f32x4*>(row + 8 * g) = v[kBf16 ? 4 * b + g : b];
+                        }
+                    });
+                    if constexpr (!PLAIN && kMayAccumulate) {
+                        if (p.has_bias) {
+#pragma unroll
+                            for (int t = 0; t < NQ; ++t) v[t] = v[t] + *reinterpret_cast<const f32x4*>(lds_bias + col[t]);
+                        }
+                        if (p.accumulate) {
+                            // (the row's old values in one burst, then the sums)
+                            f32x4 old[NQ];
+#pragma unroll
+                            for (int t = 0; t < NQ; ++t) {
+                                old[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                                if (row_ok && whole(first_of(t))) old[t] = load_old4<EPI>(drow + col[t] * DE);
+                            }
+#pragma unroll
+                            for (int t = 0; t < NQ; ++t) v[t] = v[t] + old[t];
+                        }
+                    }
+                    if (pad_row) {
+#pragma unroll
+                        for (int t = 0; t < NQ; ++t) v[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+                    if constexpr (kF32) {
+                        if (row_ok) {
+#pragma unroll
+                            for (int t = 0; t < NQ; ++t)
+                                if (whole(first_of(t))) *reinterpret_cast<f32x4*>(drow + col[t] * 4) = v[t];
                         }
                     } else {
-                        v[b] = a * p.alpha;
-                        col[b] = c0;
-                    }
-                });
-                if constexpr (EPI == kEpiF32 || EPI == kEpiBf16) {
-                    if (p.accumulate) {
-                        // (the row's old values in one burst, then the sums)
-                        f32x4 old[NQ];
+                        i32x2 pk[NQ];
 #pragma unroll
                         for (int t = 0; t < NQ; ++t) {
-                            old[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                            if (row_ok && n0 + col[t] < N) old[t] = load_old4<EPI>(drow + col[t] * DE);
+                            pk[t] = pack_quartet<EPI>(v[t], n0 + col[t]);
+                            if (EPI == kEpiBf16SR && pad_row) pk[t] = i32x2{0, 0};
                         }
+                        if constexpr (kBf16) {
+                            // per 32-column block: after swapping the wave's halves a lane holds 16 columns in a row
+                            i32x4 w[NQ / 4][2];
 #pragma unroll
-                        for (int t = 0; t < NQ; ++t) v[t] = v[t] + old[t];
-                    }
-                }
-                if (pad_row) {
+                            for (int b = 0; b < NQ / 4; ++b) {
 #pragma unroll
-                    for (int t = 0; t < NQ; ++t) v[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                }
-                if constexpr (kF32) {
-#pragma unroll
-                    for (int t = 0; t < NQ; ++t)
-                        if (row_ok && n0 + col[t] < N) *reinterpret_cast<f32x4*>(drow + col[t] * 4) = v[t];
-                } else {
-                    i32x2 pk[NQ];
-#pragma unroll
-                    for (int t = 0; t < NQ; ++t) {
-                        pk[t] = pack_quartet<EPI>(v[t], n0 + col[t]);
-                        if (EPI == kEpiBf16SR && pad_row) pk[t] = i32x2{0, 0};
-                    }
-                    if constexpr (kBf16) {
-                        // per 32-column block: after swapping the wave's halves a lane holds 16 columns in a row
-                        static_for<NQ / 4>([&](auto b_c) {
-                            constexpr int t = 4 * decltype(b_c)::value;
-                            i32x4 w[2];
-#pragma unroll
-                            for (int h = 0; h < 2; ++h) {
-                                const auto s02 = __builtin_amdgcn_permlane32_swap(pk[t + 2][h], pk[t][h], false, false);
-                                const auto s13 = __builtin_amdgcn_permlane32_swap(pk[t + 3][h], pk[t + 1][h], false, false);
-                                w[0][h] = (int)s02[0]; w[0][2 + h] = (int)s02[1];
-                                w[1][h] = (int)s13[0]; w[1][2 + h] = (int)s13[1];
-                            }
-                            const int cb = col[t] - 4 * q;
-                            if (row_ok && n0 + cb < N) {
-                                uint8_t* const d = drow + (cb + (q ? 0 : 16)) * 2;
-                                *reinterpret_cast<i32x4*>(d) = w[0];
-                                *reinterpret_cast<i32x4*>(d + 16) = w[1];
-                            }
-                        });
-                    } else {
-                        // per pair of 16-column blocks of a half: after swapping the odd and even lane groups a lane
-                        // holds eight columns in a row, 16 (q % 2) + 8 (q / 2) of the pair's 32
-                        static_for<2>([&](auto hb_c) {
-                            constexpr int hb = decltype(hb_c)::value, t0 = hb ? SB::NB0 : 0;
-                            const int cb = col_of(hb_c);
-                            static_for<SB::nb(hb) / 2>([&](auto j_c) {
-                                constexpr int j = 2 * decltype(j_c)::value, t = t0 + j;
-                                const auto s0 = __builtin_amdgcn_permlane16_swap(pk[t][0], pk[t + 1][0], false, false);
-                                const auto s1 = __builtin_amdgcn_permlane16_swap(pk[t][1], pk[t + 1][1], false, false);
-                                if (row_ok && n0 + cb + 16 * j + 16 * (q & 1) < N) {
-                                    i32x4* const d = reinterpret_cast<i32x4*>(drow + (cb + 16 * j + 16 * (q & 1) + 8 * (q >> 1)) * 2);
-                                    const i32x4 w = {(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
-                                    if (p.stream_d) __builtin_nontemporal_store(w, d);
-                                    else *d = w;
+                                for (int h = 0; h < 2; ++h) {
+                                    const auto s02 = __builtin_amdgcn_permlane32_swap(pk[4 * b + 2][h], pk[4 * b][h], false, false);
+                                    const auto s13 = __builtin_amdgcn_permlane32_swap(pk[4 * b + 3][h], pk[4 * b + 1][h], false, false);
+                                    w[b][0][h] = (int)s02[0]; w[b][0][2 + h] = (int)s02[1];
+                                    w[b][1][h] = (int)s13[0]; w[b][1][2 + h] = (int)s13[1];
                                 }
-                            });
-                            if constexpr (SB::nb(hb) % 2 != 0) {
-                                constexpr int j = SB::nb(hb) - 1;
-                                if (row_ok && n0 + cb + 16 * j < N)
-                                    *reinterpret_cast<i32x2*>(drow + (cb + 16 * j + 4 * q) * 2) = pk[t0 + j];
                             }
-                        });
+                            if (row_ok) {
+#pragma unroll
+                                for (int b = 0; b < NQ / 4; ++b) {
+                                    if (!whole(first_of(4 * b))) continue;
+                                    uint8_t* const d = drow + (first_of(4 * b) + (q ? 0 : 16)) * 2;
+                                    *reinterpret_cast<i32x4*>(d) = w[b][0];
+                                    *reinterpret_cast<i32x4*>(d + 16) = w[b][1];
+                                }
+                            }
+                        } else {
+                            // per pair of 16-column blocks of a half: after swapping the odd and even lane groups a lane
+                            // holds eight columns in a row of block q % 2, from 8 (q / 2) on
+                            i32x4 w[NQ / 2];
+                            static_for<2>([&](auto hb_c) {
+                                constexpr int hb = decltype(hb_c)::value;
+                                static_for<SB::nb(hb) / 2>([&](auto j_c) {
+                                    constexpr int j = decltype(j_c)::value, t = (hb ? SB::NB0 : 0) + 2 * j;
+                                    const auto s0 = __builtin_amdgcn_permlane16_swap(pk[t][0], pk[t + 1][0], false, false);
+                                    const auto s1 = __builtin_amdgcn_permlane16_swap(pk[t][1], pk[t + 1][1], false, false);
+                                    w[(hb ? SB::NB0 / 2 : 0) + j] = i32x4{(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
+                                });
+                            });
+                            if (row_ok) {
+                                static_for<2>([&](auto hb_c) {
+                                    constexpr int hb = decltype(hb_c)::value;
+                                    const int cb = col_of(hb_c);
+                                    static_for<SB::nb(hb) / 2>([&](auto j_c) {
+                                        constexpr int j = decltype(j_c)::value;
+                                        const int first = cb + 32 * j + 16 * (q & 1);
+                                        if (whole(first)) {
+                                            i32x4* const d = reinterpret_cast<i32x4*>(drow + (first + 8 * (q >> 1)) * 2);
+                                            if (p.stream_d) __builtin_nontemporal_store(w[(hb ? SB::NB0 / 2 : 0) + j], d);
+                                            else *d = w[(hb ? SB::NB0 / 2 : 0) + j];
+                                        }
+                                    });
+                                    if constexpr (SB::nb(hb) % 2 != 0) {
+                                        constexpr int j = SB::nb(hb) - 1;
+                                        if (whole(cb + 16 * j))
+                                            *reinterpret_cast<i32x2*>(drow + (cb + 16 * j + 4 * q) * 2) = pk[(hb ? SB::NB0 : 0) + j];
+                                    }
+                                });
+                            }
+                        }
                     }
-                }
+                });
             });
-        });
+        };
+        if (p.has_bias || p.accumulate || cut < BN) store_rows(Int<0>{});
+        else store_rows(Int<1>{});
+        if (cut < BN) {
+            __syncthreads();
+            for (int e = tid; e < BM * (MR / 4); e += 256) {
+                const int m = m0 + e / (MR / 4), n = n0 + cut + e % (MR / 4) * 4;
+                bool row_ok, pad_row;
+                row_state(m, row_ok, pad_row);
+                if (!row_ok || n >= N) continue;
+                store_quartet<EPI>(p, *reinterpret_cast<const f32x4*>(strip + e * 4), tl.d_base, m, n, N, pad_row);
+            }
+        }
         return;
     }
     static_for<2>([&](auto ha_c) {

@@ -127,6 +127,52 @@ def test_quad_accumulate_bias(force, tile, dt, n):
     _check(d, (ref + bias.float()).to(dt))
 
 
+@pytest.mark.parametrize('kind', ['e4m3', 'e2m1', 'bf16'])
+@pytest.mark.parametrize('n', [4, 12, 36, 100, 164, 236, 241, 246, 270, 511])
+def test_quad_cut_rows(force, kind, n):
+    """Rows of aligned quartets that end inside a block of columns (and inside a quartet): each output mode gives the
+    columns of the call whose rows are whole, bit for bit, and what lies past the row stays as it was."""
+    m, k = 270, 384
+    ldd, full = -(-n // 8) * 8 + 8, -(-n // 256) * 256
+    a, b, a_deq, b_deq = _fp8(m, full, k, 27, 'e2m1' if kind == 'e2m1' else 'e4m3')
+    ref = og.gemm_nt(a_deq, b_deq, torch.float32)
+    scale = float(ref.abs().mean())
+    fn = deep_gemm.fp8_gemm_nt if kind == 'e4m3' else deep_gemm.fp8_fp4_gemm_nt
+    if kind == 'bf16':
+        fn, a, b = deep_gemm.bf16_gemm_nt, a_deq.bfloat16().cuda(), (b_deq / scale).bfloat16().cuda()
+        ref, scale = og.gemm_nt(a.float().cpu(), b.float().cpu(), torch.float32), 1.0
+    cut = (lambda x: x[:n].contiguous()) if kind == 'bf16' else (lambda x: tuple(t[:n].contiguous() for t in x))
+    bias = (torch.randn(1, full, generator=gen(28)) * scale).cuda()
+    old = (torch.randn(m, full, generator=gen(29)) * scale).cuda()
+    for tile in ['256x256', '256x128', '128x128'] + (['256x224', '256x160'] if kind != 'bf16' else []):
+        force(tile)
+        for dt in (torch.bfloat16, torch.float32):
+            for mode in ['plain', 'bias', 'accumulate'] + (['stochastic'] if dt == torch.bfloat16 and kind != 'bf16' else []):
+                print(f'quad cut rows {tile} {kind} n={n} {dt} {mode}', flush=True)
+                whole = old.to(dt).clone()
+                buf = torch.full((m, ldd), 7.0, dtype=dt, device='cuda')
+                d = buf[:, :n]
+                d.copy_(whole[:, :n])
+                keys_w, keys_c = {}, {}
+                if mode == 'bias':
+                    keys_w, keys_c = dict(c=bias.to(dt)), dict(c=bias[:, :n].to(dt).contiguous())
+                elif mode == 'accumulate':
+                    keys_w, keys_c = dict(c=whole), dict(c=d)
+                elif mode == 'stochastic':
+                    keys_w = keys_c = dict(epilogue=deep_gemm.epilogue.BF16StochasticRounding())
+                fn(a, b, whole, **keys_w)
+                fn(a, cut(b), d, **keys_c)
+                last = n // 4 * 4 if mode == 'stochastic' else n   # (columns past the row hash as zeros)
+                assert torch.equal(d[:, :last], whole[:, :last])
+                assert bool((buf[:, n:] == 7.0).all())
+                want = ref + (bias.to(dt).float().cpu() if mode == 'bias' else old.to(dt).float().cpu() if mode == 'accumulate' else 0)
+                if mode != 'stochastic':
+                    _check(d, want[:, :n].to(dt))
+                else:
+                    unit = d.float().cpu().abs() * 2.0 ** -7 + 1e-3 * scale
+                    assert bool(((d.float().cpu() - want[:, :n]).abs() <= unit).all())
+
+
 @pytest.mark.parametrize('tile,split', [('256x256', 2), ('256x256', 5), ('128x128', 3), ('128x128', 11)])
 @pytest.mark.parametrize('m,n,k', [(300, 260, 1408), (130, 127, 2000)])
 def test_quad_split(force, tile, split, m, n, k):
