@@ -761,6 +761,16 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
             }
             __syncthreads();
         }
+        // m_indices: which of the lane's rows are padding, read in one burst (read where each row block is stored,
+        // every read waited for the stores before it)
+        uint32_t idx_pad = 0;
+        if (gemm_type == kMGroupedIdx && !tl.anchored) {
+            static_for<SA::NB0 + SA::NB1>([&](auto b_c) {
+                constexpr int b = decltype(b_c)::value, ha = b >= SA::NB0;
+                const int m = row_of(Int<ha>{}, Int<(ha ? b - SA::NB0 : b)>{}, wm, r);
+                idx_pad |= (p.layout[min(m, tl.tile_end - 1)] != tl.group ? 1u : 0u) << b;
+            });
+        }
         constexpr int NQ = (SB::NB0 + SB::NB1) * (kBf16 ? 4 : 1);   // quartets of a row a lane holds
         auto first_of = [&](int t) -> int {   // first column of a quartet's block within the tile
             const int b = kBf16 ? t / 4 : t;
@@ -774,9 +784,11 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
             static_for<2>([&](auto ha_c) {
                 constexpr int ha = decltype(ha_c)::value;
                 static_for<SA::nb(ha)>([&](auto i_c) {
+                    constexpr int row_block = (ha ? SA::NB0 : 0) + decltype(i_c)::value;
                     const int m = row_of(ha_c, i_c, wm, r);
-                    bool row_ok, pad_row;
-                    row_state(m, row_ok, pad_row);
+                    const bool row_ok = m < tl.tile_end && !(gemm_type == kMasked && m >= tl.valid_end);
+                    const bool pad_row = (gemm_type == kMGroupedPsum || (gemm_type == kMGroupedIdx && tl.anchored)) ? m >= tl.valid_end
+                                                                                                                   : (idx_pad >> row_block & 1) != 0;
                     uint8_t* const drow = tl.d_base + ((int64_t)m * p.ldd + n0) * DE;
                     f32x4 v[NQ];
                     int col[NQ];   // a quartet's first column within the tile

@@ -173,6 +173,26 @@ def test_quad_cut_rows(force, kind, n):
                     assert bool(((d.float().cpu() - want[:, :n]).abs() <= unit).all())
 
 
+@pytest.mark.parametrize('tile', ['256x256', '256x160', '128x128'])
+@pytest.mark.parametrize('n', [200, 256])
+def test_quad_m_indices_padding(force, tile, n):
+    """Rows of an m_indices layout that lie past their group inside a tile are written as zeros, the others not."""
+    sizes, alignment, k = [1, 255, 256, 300, 130, 17], 256, 416
+    print(f'quad m_indices {tile} n={n}', flush=True)
+    force(tile)
+    total, ps = ol.psum_from_sizes(sizes, alignment)
+    layout = ol.m_indices_from_psum(ps, alignment, total)
+    g = gen(30)
+    a, sfa, a_deq = operand(total, k, 'e4m3', (1, 32), g)
+    b, sfb, b_deq = operand(n, k, 'e4m3', (1, 32), g, batch=len(sizes))
+    d = torch.full((total, n), float('nan'), dtype=torch.bfloat16, device='cuda')
+    deep_gemm.m_grouped_fp8_gemm_nt_contiguous((a.cuda(), sfa.cuda()), (b.cuda(), sfb.cuda()), d, layout.cuda(), use_psum_layout=False)
+    out, ref = d.cpu(), og.m_grouped_contiguous(a_deq, b_deq, layout, False, alignment)
+    live = layout >= 0
+    _check(out[live], ref[live])
+    assert torch.equal(out[~live], torch.zeros_like(out[~live]))
+
+
 @pytest.mark.parametrize('tile,split', [('256x256', 2), ('256x256', 5), ('128x128', 3), ('128x128', 11)])
 @pytest.mark.parametrize('m,n,k', [(300, 260, 1408), (130, 127, 2000)])
 def test_quad_split(force, tile, split, m, n, k):
