@@ -104,13 +104,12 @@ __device__ __forceinline__ i32x2 pack_quartet(f32x4 v, int n) {
     }
 }
 
-// Old D values (accumulate) at d: four consecutive columns, aligned for a vector load.
-template <int EPI>
-__device__ __forceinline__ f32x4 load_old4(const uint8_t* d) {
+// Old D values (accumulate) of four consecutive columns, as loaded.
+template <int EPI, typename T>
+__device__ __forceinline__ f32x4 old_values(T w) {
     if constexpr (EPI == kEpiF32) {
-        return *reinterpret_cast<const f32x4*>(d);
+        return w;
     } else {
-        const i32x2 w = *reinterpret_cast<const i32x2*>(d);
         return f32x4{bf16_to_f32((uint16_t)(w[0] & 0xffff)), bf16_to_f32((uint16_t)((uint32_t)w[0] >> 16)),
                      bf16_to_f32((uint16_t)(w[1] & 0xffff)), bf16_to_f32((uint16_t)((uint32_t)w[1] >> 16))};
     }
@@ -125,7 +124,10 @@ __device__ __forceinline__ void store_quartet(const KParams& p, f32x4 v, uint8_t
     uint8_t* const d = d_base + ((int64_t)m * p.ldd + n) * (kF32 ? 4 : 2);
     const bool vec = p.vec_store && n + 4 <= N;
     f32x4 old = {0.f, 0.f, 0.f, 0.f};
-    if (p.accumulate && vec) old = load_old4<EPI == kEpiF32 ? kEpiF32 : kEpiBf16>(d);
+    if (p.accumulate && vec) {
+        typedef typename Cond<kF32, f32x4, i32x2>::type old_t;
+        old = old_values<EPI>(*reinterpret_cast<const old_t*>(d));
+    }
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
         if (n + x >= N) {
@@ -776,11 +778,26 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
             const int b = kBf16 ? t / 4 : t;
             return b >= SB::NB0 ? col_of(Int<1>{}) + (b - SB::NB0) * MR : col_of(Int<0>{}) + b * MR;
         };
+        auto col_at = [&](int t) -> int { return first_of(t) + 4 * q + (kBf16 ? 8 * (t % 4) : 0); };   // its own
+        // Old D values (accumulate) of the lane's row in a row block.  Each block's are loaded ahead of the stores of
+        // the one before: a load is waited for together with every store that went out before it.  Rows and blocks
+        // that are not stored from registers read a place that is, so that no load is conditional.
         constexpr bool kMayAccumulate = EPI == kEpiF32 || EPI == kEpiBf16;
+        typedef typename Cond<kF32, f32x4, i32x2>::type old_t;
+        old_t old[NQ];
+        const bool add_old = kMayAccumulate && p.accumulate && row_cols >= MR;
+        auto load_old = [&](auto block_c) {
+            constexpr int b = decltype(block_c)::value, ha = b >= SA::NB0;
+            const int m = min(row_of(Int<ha>{}, Int<(ha ? b - SA::NB0 : b)>{}, wm, r), tl.tile_end - 1);
+            const uint8_t* const row = tl.d_base + ((int64_t)m * p.ldd + n0) * DE;
+#pragma unroll
+            for (int t = 0; t < NQ; ++t) old[t] = *reinterpret_cast<const old_t*>(row + (whole(first_of(t)) ? col_at(t) : 0) * DE);
+        };
         // PLAIN: no bias, no old values and no cut block.  The straight-line code of a tile's rows runs once per tile, so
         // that its size is time.
         auto store_rows = [&](auto plain_tag) {
             constexpr bool PLAIN = decltype(plain_tag)::value != 0;
+            if (!PLAIN && add_old) load_old(Int<0>{});
             static_for<2>([&](auto ha_c) {
                 constexpr int ha = decltype(ha_c)::value;
                 static_for<SA::nb(ha)>([&](auto i_c) {
@@ -817,16 +834,10 @@ __device__ __forceinline__ void quad_tile_body(const KParams& p, const TileLoc& 
 #pragma unroll
                             for (int t = 0; t < NQ; ++t) v[t] = v[t] + *reinterpret_cast<const f32x4*>(lds_bias + col[t]);
                         }
-                        if (p.accumulate) {
-                            // (the row's old values in one burst, then the sums)
-                            f32x4 old[NQ];
+                        if (add_old) {
 #pragma unroll
-                            for (int t = 0; t < NQ; ++t) {
-                                old[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                                if (row_ok && whole(first_of(t))) old[t] = load_old4<EPI>(drow + col[t] * DE);
-                            }
-#pragma unroll
-                            for (int t = 0; t < NQ; ++t) v[t] = v[t] + old[t];
+                            for (int t = 0; t < NQ; ++t) v[t] = v[t] + old_values<EPI>(old[t]);
+                            if constexpr (row_block + 1 < SA::NB0 + SA::NB1) load_old(Int<row_block + 1>{});
                         }
                     }
                     if (pad_row) {
