@@ -129,10 +129,10 @@ std::string source_of(const Spec& s) {
     if (quad_tile(s.kind, s.t.bm, s.t.bn)) {
         snprintf(buf, sizeof(buf),
                  "#include \"quad_kernel.hpp\"\n"
-                 "extern \"C\" __global__ __launch_bounds__(256, dg::quad_occupancy(%d, %d)) void dg_jit_kernel(const dg::KParams p) {\n"
+                 "extern \"C\" __global__ __launch_bounds__(256, (dg::quad_occupancy<%d, %d, %d, false, false>())) void dg_jit_kernel(const dg::KParams p) {\n"
                  "    dg::quad_body<%d, %d, %d, %d, %d, %d, %d, %d, %d>(p, blockIdx.x + p.vbase);\n"
                  "}\n",
-                 s.t.bm, s.t.bn, s.t.bm, s.t.bn, s.kind, s.epi, s.ct, s.cs, s.cm, s.cn, s.ck);
+                 s.t.bm, s.t.bn, s.kind, s.t.bm, s.t.bn, s.kind, s.epi, s.ct, s.cs, s.cm, s.cn, s.ck);
         return buf;
     }
     snprintf(buf, sizeof(buf),

@@ -991,12 +991,13 @@ __device__ __forceinline__ void quad_body(const KParams& p, const int vb) {
     }
 }
 
-// Workgroups per CU: two 128 x 128 tiles share a CU (68 KB of LDS each) and cover each other's prologue, epilogue
-// and LDS latency.
-constexpr int quad_occupancy(int bm, int bn) { return bm * bn <= 128 * 128 ? 2 : 1; }
+// Workgroups per CU: as many as the LDS holds.  Two 128 x 128 tiles of K-major operands (68 KB each) share a CU and cover
+// each other's prologue, epilogue and LDS latency; an MN-major side takes the LDS of 128 elements in each half.
+template <int BM, int BN, int KIND, bool AMN, bool BMN>
+constexpr int quad_occupancy() { return 2 * QuadTile<BM, BN, KIND, AMN, BMN>::LDS_BYTES <= 160 * 1024 ? 2 : 1; }
 
 template <int BM, int BN, int KIND, int EPI, bool AMN = false, bool BMN = false>
-__global__ __launch_bounds__(256, quad_occupancy(BM, BN)) void quad_kernel(const KParams p) {
+__global__ __launch_bounds__(256, (quad_occupancy<BM, BN, KIND, AMN, BMN>())) void quad_kernel(const KParams p) {
     quad_body<BM, BN, KIND, EPI, -1, 0, 0, 0, 0, AMN, BMN>(p, blockIdx.x + p.vbase);
 }
 
