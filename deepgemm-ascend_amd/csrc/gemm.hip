@@ -432,13 +432,27 @@ bool cus_capped(int cus) { return cus < device_cus(); }
 struct QuadRate {
     int bm, bn, occ;
     double light, share, fixed;
+    double mn_stage = 1.0;   // a stage's factor where an operand is MN-major
 };
 constexpr QuadRate kQuadFp8[] = {{256, 256, 1, 0.94, 0.0045, 7.5}, {256, 224, 1, 0.815, 0.0040, 8.2}, {256, 160, 1, 0.64, 0.0030, 7.5},
                                  {256, 128, 1, 0.54, 0.00245, 6.5}, {128, 128, 2, 0.353, 0.00172, 6.5}};
-constexpr QuadRate kQuadBf16[] = {{256, 256, 1, 0.87, 0.0058, 9.0}, {256, 128, 1, 0.49, 0.00334, 6.5}, {128, 128, 2, 0.32, 0.00217, 6.0}};
+constexpr QuadRate kQuadBf16[] = {{256, 256, 1, 0.87, 0.0058, 9.0}, {256, 128, 1, 0.49, 0.00334, 6.5}, {128, 128, 2, 0.32, 0.00217, 6.0},
+                                  {256, 224, 1, 1.05, 0.0054, 9.3, 1.12}, {256, 160, 1, 0.80, 0.0040, 8.4, 1.25}};
 // MN-major operands of a 128-row tile come in half lines and fill the LDS of a whole CU (bf16 tn 4096^3: 163 us
 // against 115 on 256x256 tiles)
 constexpr QuadRate kQuadMn128 = {128, 128, 1, 0.48, 0.0022, 7.0};
+
+// The last two bf16 tiles run the eight-wave kernel: two waves a SIMD cover more of a tile's fill and epilogue, while a
+// stage takes longer.  They win where 256x256 tiles leave CUs idle (nt 1000x9000x1024 23.8 us against 26.2, 3000x3000x512
+// 17.8 and 19.5) and, with MN-major operands, whose fill is longer, at short K: tn 2304x4000, 256x160 against 256x256,
+// K = 256 16.0 and 19.0, 512 21.2 and 22.7, 1024 30.5 and 30.2, 2048 50.9 and 46.6; tn 5440x9168, 256x224 against 256x256,
+// 67.5 and 76.6, 91.2 and 98.1, 138.7 and 135.1, 232.7 and 219.3.
+constexpr double kQuadMnFixedBf16 = 3.0;
+constexpr int kEightWaveMnStages = 8;   // (K of a tile, 64 each)
+// Under a CU cap a tile with a persistent kernel pays its fill and epilogue about half; the others go out in launches
+// of one tile per allowed CU, 3 us apart (bf16 4096x7168x2048 on 200 CUs: 256x224 120 us, 256x256 131; the e4m3 rates
+// choose the persistent tiles where they are the faster ones without it: 512x2112x2048 on 64 CUs 15.3, with it 20.9).
+constexpr double kLaunchGap = 3.0;
 
 double quad_time(const QuadRate& q, int64_t tiles, int stages, int cus) {
     const int64_t slots = (int64_t)cus * q.occ, full = tiles / slots, rest = tiles % slots;
@@ -462,17 +476,28 @@ bool quad_plan(const dg_gemm_args& a, int cus, bool allow_split, Plan& out) {
     const int num = bf16 ? (int)(sizeof(kQuadBf16) / sizeof(QuadRate)) : (int)(sizeof(kQuadFp8) / sizeof(QuadRate));
     double best = 1e300;
     for (int i = 0; i < num; ++i) {
-        const QuadRate q = mn && rates[i].bm == 128 ? kQuadMn128 : rates[i];
+        QuadRate q = mn && rates[i].bm == 128 ? kQuadMn128 : rates[i];
         if (!tile_allowed(a, q.bm, q.bn)) continue;
+        const bool quad = quad_tile(a.kind, q.bm, q.bn);
+        if (mn && !quad && ns > kEightWaveMnStages) continue;
         TileCfg tc = {};
         for (const TileCfg& c : kTiles)
             if (c.bm == q.bm && c.bn == q.bn) tc = c;
+        if (mn) {
+            q.light *= q.mn_stage;
+            q.share *= q.mn_stage;
+            if (bf16 && quad) q.fixed += kQuadMnFixedBf16;
+        }
+        const bool capped = bf16 && cus_capped(cus), walks = capped && !mn && a.gemm_type != kKGrouped && tile_persistable(tc);
         const int64_t tiles = plan_tiles(a, tc), slots = (int64_t)cus * q.occ;
         for (int sp = 1; sp <= 8 && sp <= ns; ++sp) {
-            if (sp > 1 && (!allow_split || tiles * sp > slots || tiles > kMaxSplitTiles || ns < 4 * sp)) break;
+            if (sp > 1 && (!allow_split || !quad || tiles * sp > slots || tiles > kMaxSplitTiles || ns < 4 * sp)) break;
             const int sps = ceil_div(ns, sp);
             if (ceil_div(ns, sps) != sp) continue;
-            double t = quad_time(q, tiles * sp, sps, cus);
+            QuadRate r = q;
+            if (sp == 1 && walks) r.fixed *= 0.5;
+            double t = quad_time(r, tiles * sp, sps, cus);
+            if (sp == 1 && capped && !walks) t += kLaunchGap * (ceil_div64(tiles, cus) - 1);
             if (sp > 1) t += 3.5 + 8.0 * sp * a.m * (double)a.n * groups / 7e6;
             if (t < best * (sp > 1 ? 0.97 : 1.0)) {
                 best = t;

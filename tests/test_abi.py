@@ -289,6 +289,27 @@ def test_large_mn_major_operands_are_copied(lib, monkeypatch, kind, m, n, k, for
     assert launches[-1] == (int(a_mn and not big[0]), int(b_mn and not big[1]), 0), launches
 
 
+@pytest.mark.parametrize('kind, gemm_type, m, n, k, groups, mn, cus, tile, threads', [
+    # bf16, MN-major operands: eight-wave tiles at short K, four-wave 256 x 256 from K = 1024
+    (3, 0, 2304, 4000, 512, 1, 3, 256, (256, 160), 512), (3, 0, 2304, 4000, 1024, 1, 3, 256, (256, 256), 256),
+    (3, 0, 5440, 9168, 512, 1, 3, 256, (256, 224), 512), (3, 0, 2112, 7168, 4096, 1, 3, 256, (256, 256), 256),
+    (3, 5, 1280, 1600, 2051, 8, 3, 256, (256, 160), 512),
+    # K-major: where 256 x 256 tiles leave CUs idle
+    (3, 0, 1000, 9000, 1024, 1, 0, 256, (256, 160), 512), (3, 0, 4096, 4096, 7168, 1, 0, 256, (256, 256), 256),
+    # under a CU cap: the tile with a persistent kernel
+    (3, 0, 4096, 7168, 2048, 1, 0, 200, (256, 224), 512)])
+def test_tile_choice(lib, kind, gemm_type, m, n, k, groups, mn, cus, tile, threads):
+    """Both sides of the lines between the four-wave tiles and the eight-wave kernel's."""
+    args = _plan_args(m, n, k, cus)
+    args.kind, args.gemm_type, args.num_groups, args.alpha = kind, gemm_type, groups, 1.0
+    args.a_mn_major, args.b_mn_major = mn & 1, mn >> 1
+    args.k = -(-k // 64) * 64
+    args.lda, args.ldb = m if mn & 1 else args.k, n if mn & 2 else args.k
+    info = _lib.LaunchInfo()
+    assert lib.dg_launch_plan(args, ctypes.byref(info)) == 0, lib.dg_last_error()
+    assert ((info.block_m, info.block_n), info.threads) == (tile, threads)
+
+
 def test_error_words_and_stream_workspace_without_device(lib):
     # no kernel has run: nothing pending; the workspace query rejects null outputs
     assert lib.dg_take_errors() == 0

@@ -82,11 +82,12 @@ def test_jit_fp8_fp4_and_bf16():
 
 
 @pytest.mark.parametrize('b_kind', ['e4m3', 'e2m1'])
-@pytest.mark.parametrize('m,n,k', [(512, 512, 128), (512, 1056, 256), (1024, 2112, 384), (256, 512, 640)])
-def test_jit_few_stages(b_kind, m, n, k):
+@pytest.mark.parametrize('m,n,k,tile', [(512, 512, 128, '256x256'), (512, 1056, 256, '256x224'), (1024, 2112, 384, '128x128'),
+                                        (256, 512, 640, '256x128')])
+def test_jit_few_stages(monkeypatch, b_kind, m, n, k, tile):
     """Four-wave bodies whose K is a compile-time constant of one to five stages: straight-line loops."""
-    print(f'jit few stages {b_kind} m={m} n={n} k={k}', flush=True)
-    assert deep_gemm.launch_plan(m, n, k)['block_m'] >= 128
+    print(f'jit few stages {b_kind} {tile} m={m} n={n} k={k}', flush=True)
+    monkeypatch.setenv('DG_FORCE_BLOCK', tile)
     g = gen(36)
     a, sfa, a_deq = operand(m, k, 'e4m3', (1, 32), g)
     b, sfb, b_deq = operand(n, k, b_kind, (1, 32), g)
