@@ -449,6 +449,19 @@ constexpr QuadRate kQuadMn128 = {128, 128, 1, 0.48, 0.0022, 7.0};
 // 67.5 and 76.6, 91.2 and 98.1, 138.7 and 135.1, 232.7 and 219.3.
 constexpr double kQuadMnFixedBf16 = 3.0;
 constexpr int kEightWaveMnStages = 8;   // (K of a tile, 64 each)
+// Small problems of short K take 64x128 tiles of the eight-wave kernel's menu (four waves, two workgroups a CU), whose
+// fill and epilogue are the shorter ones; by kind: e4m3, e4m3 x e2m1, bf16.  Measured, 64x128 against 128x128: e4m3
+// 136x2112 K = 256 5.0 and 5.8, 512 5.8 and 6.4, 1024 7.4 and 7.7, 1536 9.0 and 8.9, 512x4096 5.6 and 6.2, 6.5 and 6.9,
+// 8.2 and 8.3, 9.8 and 9.7, 300x7000 (more tiles than CUs) 7.2 and 7.2, 8.2 and 7.9, 10.9 and 9.2; e4m3 x e2m1 136x2112
+// K = 256 4.8 and 5.8, 1024 6.9 and 7.7; bf16 136x2112 K = 256 5.2 and 5.5, 512 6.6 and 6.5.  Past kSmallStages (K of
+// 1024, bf16 512) rows that end inside a block gain alone: 291x3796, e4m3 1056 8.6 and 9.5, 2048 11.4 and 11.7, bf16
+// 768 8.6 and 9.4, 1536 12.6 and 12.6.
+constexpr QuadRate kSmall[] = {{64, 128, 2, 0.49, 0.0013, 5.5}, {64, 128, 2, 0.39, 0.0013, 5.2}, {64, 128, 2, 0.40, 0.0012, 5.35}};
+constexpr int kSmallStages = 8;
+// The four-wave kernel's last tile of a row that ends inside a block of columns stores a strip through LDS (291x3796 at
+// K = 512, 64x128 against 128x128: e4m3 6.4 and 7.7, bf16 7.3 and 8.4), and rows of unaligned quartets go through it
+// whole (136x2111x512 7.7 and 13.6; with more tiles than CUs less is left of it, 1000x3001x1024 17.5 and 15.8).
+constexpr double kCutRow = 1.2, kUnalignedRows = 3.5;
 // Under a CU cap a tile with a persistent kernel pays its fill and epilogue about half; the others go out in launches
 // of one tile per allowed CU, 3 us apart (bf16 4096x7168x2048 on 200 CUs: 256x224 120 us, 256x256 131; the e4m3 rates
 // choose the persistent tiles where they are the faster ones without it: 512x2112x2048 on 64 CUs 15.3, with it 20.9).
@@ -474,9 +487,11 @@ bool quad_plan(const dg_gemm_args& a, int cus, bool allow_split, Plan& out) {
     const int ns = std::max(1, ceil_div(k_tile, bf16 ? 64 : 128));
     const QuadRate* const rates = bf16 ? kQuadBf16 : kQuadFp8;
     const int num = bf16 ? (int)(sizeof(kQuadBf16) / sizeof(QuadRate)) : (int)(sizeof(kQuadFp8) / sizeof(QuadRate));
+    const bool dense = a.gemm_type == kNormal || a.gemm_type == kBatched;
+    const bool small = dense && !mn && !cus_capped(cus) && ns <= kSmallStages, cut = a.n % (bf16 ? 32 : 16) != 0;
     double best = 1e300;
-    for (int i = 0; i < num; ++i) {
-        QuadRate q = mn && rates[i].bm == 128 ? kQuadMn128 : rates[i];
+    for (int i = small ? -1 : 0; i < num; ++i) {
+        QuadRate q = i < 0 ? kSmall[bf16 ? 2 : a.kind == kFP8FP4 ? 1 : 0] : mn && rates[i].bm == 128 ? kQuadMn128 : rates[i];
         if (!tile_allowed(a, q.bm, q.bn)) continue;
         const bool quad = quad_tile(a.kind, q.bm, q.bn);
         if (mn && !quad && ns > kEightWaveMnStages) continue;
@@ -498,6 +513,7 @@ bool quad_plan(const dg_gemm_args& a, int cus, bool allow_split, Plan& out) {
             if (sp == 1 && walks) r.fixed *= 0.5;
             double t = quad_time(r, tiles * sp, sps, cus);
             if (sp == 1 && capped && !walks) t += kLaunchGap * (ceil_div64(tiles, cus) - 1);
+            if (quad && cut) t += a.n % 4 == 0 ? kCutRow : kUnalignedRows;
             if (sp > 1) t += 3.5 + 8.0 * sp * a.m * (double)a.n * groups / 7e6;
             if (t < best * (sp > 1 ? 0.97 : 1.0)) {
                 best = t;
@@ -506,15 +522,6 @@ bool quad_plan(const dg_gemm_args& a, int cus, bool allow_split, Plan& out) {
         }
     }
     return best < 1e300;
-}
-
-// Rows of D that end inside a 32-column block send the four-wave kernel's last tile of each row through LDS, about
-// 7 us that a short contraction of one round does not hide (e4m3 291 x N x 544, packed scales: N = 3840 7.0 us,
-// N = 3796 14.0 and 6.7 on 64x128 tiles of gemm_kernel; 1000 x 3001 x 1024 18.4 there; bf16 291 x 3796 x 512 7.1).
-bool cut_rows_short(const dg_gemm_args& a, int cus) {
-    return (a.gemm_type == kNormal || a.gemm_type == kBatched) && !a.a_mn_major && !a.b_mn_major && a.n % 32 != 0 &&
-           a.k <= (a.kind == kBF16 ? 512 : 1024) &&
-           ceil_div64(a.m, 128) * ceil_div64(a.n, 128) * (a.gemm_type == kBatched ? a.num_groups : 1) <= cus;
 }
 
 Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
@@ -537,8 +544,7 @@ Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
             if (tc.bm == 384 && tc.bn == (fp4_b ? 128 : 192)) return {tc, 1, ceil_div(a.k, k_stage_elems(a.kind, tc)), 0, 0, 0};
     }
     Plan quad;
-    const bool cut_short = cut_rows_short(a, cus);
-    if (!cut_short && quad_plan(a, cus, allow_split, quad)) return quad;
+    if (quad_plan(a, cus, allow_split, quad)) return quad;
     allow_split = false;   // wide problems fill the CUs with tiles
     const int groups = (a.gemm_type == kBatched || a.gemm_type == kMasked || a.gemm_type == kKGrouped) ? a.num_groups : 1;
     // (K-grouped: each tile contracts one group's share of K)
@@ -555,7 +561,7 @@ Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
         // (anchored tiles only where the alignment rules out 256-row tiles, above: at alignment 256 they
         // measured behind, 526 vs 443 us for 256x224 at G=32 N=4096 K=7168, and FP8 x FP4 G=8 x 4096
         // rows N=7168 K=3072 took 2546 us on 384x192)
-        if (!tile_allowed(a, tc.bm, tc.bn) || tile_anchored(tc.bm) || (cut_short && quad_tile(a.kind, tc.bm, tc.bn))) continue;
+        if (!tile_allowed(a, tc.bm, tc.bn) || tile_anchored(tc.bm)) continue;
         const int ns = ceil_div(k_tile, k_stage_elems(a.kind, tc));
         const int64_t tiles = plan_tiles(a, tc);
         const int max_split = allow_split && tile_splittable(a.kind, tc) && tiles <= kMaxSplitTiles ? std::min(16, std::max(1, ns / 4)) : 1;

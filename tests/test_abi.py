@@ -297,7 +297,10 @@ def test_large_mn_major_operands_are_copied(lib, monkeypatch, kind, m, n, k, for
     # K-major: where 256 x 256 tiles leave CUs idle
     (3, 0, 1000, 9000, 1024, 1, 0, 256, (256, 160), 512), (3, 0, 4096, 4096, 7168, 1, 0, 256, (256, 256), 256),
     # under a CU cap: the tile with a persistent kernel
-    (3, 0, 4096, 7168, 2048, 1, 0, 200, (256, 224), 512)])
+    (3, 0, 4096, 7168, 2048, 1, 0, 200, (256, 224), 512),
+    # small problems of short K
+    (0, 0, 136, 2112, 256, 1, 0, 256, (64, 128), 256), (0, 0, 300, 7000, 512, 1, 0, 256, (128, 128), 256),
+    (1, 0, 136, 2112, 1024, 1, 0, 256, (64, 128), 256), (0, 0, 136, 2112, 2048, 1, 0, 256, (128, 128), 256)])
 def test_tile_choice(lib, kind, gemm_type, m, n, k, groups, mn, cus, tile, threads):
     """Both sides of the lines between the four-wave tiles and the eight-wave kernel's."""
     args = _plan_args(m, n, k, cus)

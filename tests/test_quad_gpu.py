@@ -17,7 +17,7 @@ from helpers import gen, operand, calc_diff
 
 pytestmark = pytest.mark.gpu
 THRESH = 1e-5
-TILES = ['256x256', '256x224', '256x160', '128x128']
+TILES = ['256x256', '256x224', '256x160', '256x128', '128x128']
 
 
 @pytest.fixture
@@ -74,7 +74,7 @@ def test_quad_fp4(force, tile, m, n, k):
     _check(d, og.gemm_nt(a_deq, b_deq))
 
 
-@pytest.mark.parametrize('tile', ['256x256', '256x224', '128x128'])
+@pytest.mark.parametrize('tile', TILES)
 @pytest.mark.parametrize('form', ['nn', 'tn', 'tt'])
 @pytest.mark.parametrize('m,n,k', [(256, 224, 128), (272, 240, 416), (144, 496, 1152)])
 def test_quad_mn_major(force, tile, form, m, n, k):
@@ -90,7 +90,7 @@ def test_quad_mn_major(force, tile, form, m, n, k):
     _check(d, og.gemm_nt(a_deq, b_deq, torch.float32))
 
 
-@pytest.mark.parametrize('tile', ['256x256', '128x128'])
+@pytest.mark.parametrize('tile', ['256x256', '256x128', '128x128'])
 @pytest.mark.parametrize('form', ['nt', 'nn', 'tn', 'tt'])
 @pytest.mark.parametrize('m,n,k', [(256, 256, 64), (264, 120, 200), (136, 392, 520)])
 def test_quad_bf16(force, tile, form, m, n, k):
@@ -207,6 +207,72 @@ def test_quad_split(force, tile, split, m, n, k):
         _check(d, og.gemm_nt(a_deq, b_deq, dt))
         out[dt] = d
     assert torch.equal(out[torch.bfloat16], out[torch.float32].bfloat16())
+
+
+@pytest.mark.parametrize('tile', TILES)
+@pytest.mark.parametrize('kind,form', [('e4m3', 'nt'), ('e4m3', 'tn'), ('e2m1', 'nt'), ('bf16', 'nt'), ('bf16', 'nn')])
+def test_quad_split_forms(force, tile, kind, form):
+    """Partials of every tile's layout (the uneven halves of 224 and 160 columns too), operand kind and major; plain,
+    accumulated and with a bias row."""
+    if kind == 'bf16' and tile in ('256x224', '256x160'):
+        pytest.skip('bf16 runs these tiles on the eight-wave kernel, without K splits')
+    m, n, k = 272, 240, 1168
+    g = gen(31)
+    a, sfa, a_deq = operand(m, k, 'e4m3', (1, 32), g)
+    b, sfb, b_deq = operand(n, k, 'e4m3' if kind == 'bf16' else kind, (1, 32), g)
+    scale = 1.0
+    if kind == 'bf16':
+        a_deq, b_deq = (x / x.abs().mean() for x in (a_deq, b_deq))
+        a, b = a_deq.bfloat16(), b_deq.bfloat16()
+        a_deq, b_deq = a.float(), b.float()
+    if form[0] == 't':
+        a, sfa = a.t().contiguous(), sfa.t().contiguous()
+    if form[1] == 'n':
+        b, sfb = b.t().contiguous(), sfb.t().contiguous()
+    ref = og.gemm_nt(a_deq, b_deq, torch.float32)
+    scale = float(ref.abs().mean())
+    x, y = (a.cuda(), b.cuda()) if kind == 'bf16' else ((a.cuda(), sfa.cuda()), (b.cuda(), sfb.cuda()))
+    fn = getattr(deep_gemm, {'e4m3': 'fp8_gemm_', 'e2m1': 'fp8_fp4_gemm_', 'bf16': 'bf16_gemm_'}[kind] + form)
+    bias = torch.randn(1, n, generator=gen(32)) * scale
+    old = torch.randn(m, n, generator=gen(33)) * scale
+    for split in (2, 5):
+        print(f'quad split {split} {tile} {kind} {form}', flush=True)
+        force(tile, split)
+        d = torch.full((m, n), float('nan'), device='cuda')
+        fn(x, y, d)
+        _check(d, ref)
+        fn(x, y, d, c=bias.cuda())
+        _check(d, ref + bias)
+        d = old.clone().cuda()
+        fn(x, y, d, c=d)
+        _check(d, ref + old)
+
+
+@pytest.mark.parametrize('tile', ['256x256', '256x160', '128x128'])
+def test_quad_split_batched(force, tile):
+    bsz, m, n, k = 3, 140, 264, 1056
+    print(f'quad split bmm {tile}', flush=True)
+    force(tile, 3)
+    g = gen(34)
+    a, sfa, a_deq = operand(m, k, 'e4m3', (1, 32), g, batch=bsz)
+    b, sfb, b_deq = operand(n, k, 'e4m3', (1, 32), g, batch=bsz)
+    d = torch.full((bsz, m, n), float('nan'), device='cuda')
+    deep_gemm.fp8_bmm((a.cuda(), sfa.cuda()), (b.cuda(), sfb.cuda()), d)
+    for i in range(bsz):
+        _check(d[i], og.gemm_nt(a_deq[i], b_deq[i], torch.float32))
+
+
+@pytest.mark.parametrize('b_kind', ['e4m3', 'e2m1'])
+@pytest.mark.parametrize('n', [2080, 2076])
+def test_quad_d_past_the_caches(b_kind, n):
+    """A D of more than 192 MiB at short K is stored past the caches; with rows that end at, and inside, a block."""
+    m, k = 49157, 160
+    print(f'quad stores past the caches {b_kind} n={n}', flush=True)
+    assert 2 * m * n >= 192 << 20
+    a, b, a_deq, b_deq = _fp8(m, n, k, 35, b_kind)
+    d = torch.full((m, n), float('nan'), dtype=torch.bfloat16, device='cuda')
+    (deep_gemm.fp8_gemm_nt if b_kind == 'e4m3' else deep_gemm.fp8_fp4_gemm_nt)(a, b, d)
+    _check(d, og.gemm_nt(a_deq, b_deq))
 
 
 @pytest.mark.parametrize('b_kind', ['e4m3', 'e2m1'])
