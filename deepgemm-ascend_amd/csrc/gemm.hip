@@ -545,7 +545,7 @@ Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
     }
     Plan quad;
     if (quad_plan(a, cus, allow_split, quad)) return quad;
-    allow_split = false;   // wide problems fill the CUs with tiles
+    // FP4 x FP4, which the four-wave kernel does not serve: waves of workgroups, unsplit (wide problems fill the CUs).
     const int groups = (a.gemm_type == kBatched || a.gemm_type == kMasked || a.gemm_type == kKGrouped) ? a.num_groups : 1;
     // (K-grouped: each tile contracts one group's share of K)
     const int k_tile = a.gemm_type == kKGrouped ? ceil_div(a.k, std::max(1, a.num_groups)) : a.k;
@@ -563,31 +563,15 @@ Plan select_plan(const dg_gemm_args& a, int cus, bool allow_split) {
         // rows N=7168 K=3072 took 2546 us on 384x192)
         if (!tile_allowed(a, tc.bm, tc.bn) || tile_anchored(tc.bm)) continue;
         const int ns = ceil_div(k_tile, k_stage_elems(a.kind, tc));
-        const int64_t tiles = plan_tiles(a, tc);
-        const int max_split = allow_split && tile_splittable(a.kind, tc) && tiles <= kMaxSplitTiles ? std::min(16, std::max(1, ns / 4)) : 1;
-        for (int sp = 1; sp <= max_split; ++sp) {
-            const int sps = ceil_div(ns, sp);
-            const int s_eff = ceil_div(ns, sps);
-            if (sp > 1 && s_eff != sp) continue;
-            // The splits of a tile run on one XCD (kXcds of them, cus / kXcds CUs each).
-            const int64_t rounds = sp == 1 ? ceil_div64(tiles, (int64_t)cus * tc.occ)
-                                           : ceil_div64(ceil_div64(tiles, kXcds) * sp, std::max(1, cus / kXcds));
-            if (sp > 1 && rounds > 1) break;
-            // Waves of workgroups x (their K stages at the tile's measured stage time + the
-            // fixed cost of a tile: pipeline fill and the epilogue's stores), plus the split
-            // reduction (measured ~10K cycles: partial stores, arrival count, partial reads).
-            // (co-resident workgroups share the CU's MFMAs but overlap each other's fixed costs)
-            double t = (double)rounds * ((double)tc.occ * sps * tc.km * tc.stage_cycles + 6000.0 + tc.bm * tc.bn / 8.0);
-            double bytes = hbm_bytes;
-            if (sp > 1) {
-                t += 10000.0 + 500.0 * sp;
-                bytes += 8.0 * a.m * a.n * groups * sp;
-            }
-            t = std::max(t, bytes / 3800.0);
-            if (t < best * 0.97) {
-                best = t;
-                pick = {tc, sp, sps, 0, 0, 0};
-            }
+        const int64_t rounds = ceil_div64(plan_tiles(a, tc), (int64_t)cus * tc.occ);
+        // Waves of workgroups x (their K stages at the tile's measured stage time + the
+        // fixed cost of a tile: pipeline fill and the epilogue's stores).
+        // (co-resident workgroups share the CU's MFMAs but overlap each other's fixed costs)
+        double t = (double)rounds * ((double)tc.occ * ns * tc.km * tc.stage_cycles + 6000.0 + tc.bm * tc.bn / 8.0);
+        t = std::max(t, hbm_bytes / 3800.0);
+        if (t < best * 0.97) {
+            best = t;
+            pick = {tc, 1, ns, 0, 0, 0};
         }
     }
     return pick;
