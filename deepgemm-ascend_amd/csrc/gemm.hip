@@ -5,9 +5,8 @@
 // bf16_gemm.hpp:16-78) and its select_gemm_config cost model
 // (csrc/jit_kernels/heuristics.hpp:592-755).  Kernels are compiled ahead of time for a
 // fixed menu of tile shapes; the heuristic scores each shape with a gfx950 model
-// (256 CUs, waves-of-tiles quantisation; the four-wave tiles by costs fitted to measurements,
-// quad_time, the others by cycles per K stage and a fixed per-tile cost) and memoises the choice
-// per problem signature.
+// (256 CUs, waves-of-tiles quantisation, costs fitted to measurements, quad_time; FP4 x FP4 by
+// cycles per K stage and a fixed per-tile cost) and memoises the choice per problem signature.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -477,7 +476,7 @@ double quad_time(const QuadRate& q, int64_t tiles, int stages, int cus) {
     return full * round(slots) + (rest ? round(rest) : 0.0);
 }
 
-// Best four-wave plan by that model.  K is split while the ranges still run at once; their fp32 partials are
+// Best tile plan by that model.  K is split while the ranges still run at once; their fp32 partials are
 // written and read back (7 TB/s, mostly from the caches) and summed by a second launch (3.5 us).
 bool quad_plan(const dg_gemm_args& a, int cus, bool allow_split, Plan& out) {
     if (a.kind == kFP4FP4) return false;

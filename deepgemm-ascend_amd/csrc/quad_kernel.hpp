@@ -18,8 +18,8 @@
 // SIMD's matrix pipe for 32 cycles, in which a wave can issue about six other instructions, so LDS reads and
 // loads are dealt out one at a time between MFMAs (slots), the K offset of a stage rides in the loads' vector
 // offset and the row steps in constant scalar offsets (two instructions per load).  Measured on MI355X (e4m3,
-// 8192^3, sustained): MFMA busy 77 % of the cycles against 69 % for the eight-wave kernel it replaced, 2.9
-// against 2.5 PFLOP/s.
+// 8192^3, the shortest of twenty passes in a row): MFMA busy 76 % of the cycles against 70 % for the eight-wave kernel
+// it replaced, 2.85 against 2.57 PFLOP/s.
 //
 // e4m3 / e2m1: v_mfma_scale_f32_16x16x128_f8f6f4.  With random e4m3 operands in registers it sustains 4.26
 // PFLOP/s against 3.95 for the 32x32x64 form (less power per FLOP); errors against fp64 are the same.

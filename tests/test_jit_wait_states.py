@@ -1,5 +1,5 @@
-"""Wait states of run-time compiled four-wave bodies (csrc/quad_kernel.hpp), read from the gfx950 assembly of the
-code objects built here.  Their matrix instructions are inline asm, for which the compiler inserts no wait states:
+"""Wait states of four-wave bodies (csrc/quad_kernel.hpp), run-time compiled and the ahead-of-time 384-row tiles, read
+from the gfx950 assembly of the code objects built here.  Their matrix instructions are inline asm, for which the compiler inserts no wait states:
 a VALU write of an operand has to lie two wait states ahead of the matrix instruction that reads it, and an
 accumulator may be touched 11 (16x16x128) or 19 (32x32x16) after the one that wrote it.  K of one, two and three
 stages is the form in which the loop becomes straight-line code that the compiler may move instructions along."""
@@ -13,7 +13,8 @@ import pytest
 from deep_gemm import _lib
 from test_jit import _args
 
-OBJDUMP = '/opt/rocm/llvm/bin/llvm-objdump'
+LLVM = '/opt/rocm/llvm/bin/'
+OBJDUMP = LLVM + 'llvm-objdump'
 OPERAND_WAIT, RESULT_WAIT = 2, {'16x16': 11, '32x32': 19}
 
 
@@ -78,13 +79,19 @@ def _writers_within(code, before, i, states, hit):
 def violations(listing):
     code, before = _parse(listing)
     out, count = [], 0
+    # (most instructions have neither a matrix instruction nor a branch target close behind them: nothing to follow)
+    close, last = [], -RESULT_WAIT['32x32'] - 1
+    for i, x in enumerate(code):
+        if x.mfma or before[i] != [i - 1]:
+            last = i
+        close.append(i - last <= RESULT_WAIT['32x32'])
     for i, x in enumerate(code):
         if x.mfma:
             count += 1
             operands = frozenset().union(*x.regs[1:])
             for w, gap in _writers_within(code, before, i, OPERAND_WAIT, lambda w: w.valu and w.writes & operands):
                 out.append(f'{w.op} at {w.address:x} is {gap} wait states ahead of the {x.op} at {x.address:x}')
-        elif x.touched:
+        elif x.touched and close[i]:
             for shape, wait in RESULT_WAIT.items():
                 for w, gap in _writers_within(code, before, i, wait, lambda w: w.mfma and shape in w.op and w.regs[0] & x.touched):
                     out.append(f'{x.op} at {x.address:x} is {gap} wait states behind the {w.op} at {w.address:x}')
@@ -135,3 +142,29 @@ def test_jit_wait_states(tmp_path, monkeypatch, kind, gemm_type, m, n, k, alignm
     assert 'ds_read' in listing and 'v_mfma' in listing
     found = violations(listing)
     assert not found, (len(found), found[:8])
+
+
+def test_ahead_of_time_wide_tiles(tmp_path):
+    """The 384-row tiles, whose loops hold the scales' shifts in place without an asm of their own."""
+    if not os.path.exists(OBJDUMP):
+        pytest.skip('no llvm-objdump')
+    fat = tmp_path / 'fatbin'
+    subprocess.run([LLVM + 'llvm-objcopy', f'--dump-section=.hip_fatbin={fat}', str(_lib.library_path()), '/dev/null'],
+                   check=True, timeout=60)
+    checked = 0
+    for i, part in enumerate(fat.read_bytes().split(b'__CLANG_OFFLOAD_BUNDLE__')[1:]):
+        if b'quad_kernelILi384' not in part:
+            continue
+        bundle, obj = tmp_path / f'bundle{i}', tmp_path / f'obj{i}'
+        bundle.write_bytes(b'__CLANG_OFFLOAD_BUNDLE__' + part)
+        subprocess.run([LLVM + 'clang-offload-bundler', '--unbundle', '--type=o', '--targets=hipv4-amdgcn-amd-amdhsa--gfx950',
+                        f'--input={bundle}', f'--output={obj}'], check=True, timeout=60)
+        listing = subprocess.run([OBJDUMP, '-d', '--mcpu=gfx950', str(obj)], capture_output=True, text=True, check=True,
+                                 timeout=120).stdout
+        functions = re.split(r'^[0-9a-f]{16} <(.*)>:\n', listing, flags=re.M)[1:]
+        for name, body in zip(functions[::2], functions[1::2]):
+            if 'quad_kernelILi384' in name:
+                found = violations(body)
+                assert not found, (name, len(found), found[:8])
+                checked += 1
+    assert checked >= 6
